@@ -9,6 +9,7 @@
 
 #include "apsm_device.h"
 #include "apsm_train2.h"
+#include "apsm_train_win.h"
 #include "apsm_detect_launch.h"
 
 namespace apsm {
@@ -51,6 +52,15 @@ __global__ void __launch_bounds__( kSeqThreads ) batch_seq2( const Seq2Desc* __r
     if ( (int)blockIdx.x >= s.a.U )
         return;
     seq2Body<TP, NEWPER, PMAX>( s.Z, s.Zn, s.Y, s.C, s.Fg, s.thF, s.P, s.Gact, s.EvF, s.a, blockIdx.x );
+}
+
+template <int TP>
+__global__ void __launch_bounds__( winThreads( TP ) ) batch_train_win( const Seq2Desc* __restrict__ d )
+{
+    const Seq2Desc& s = d[ blockIdx.y ];
+    if ( (int)blockIdx.x >= s.a.U )
+        return;
+    winBody<TP>( s.Z, s.Zn, s.Y, s.C, s.Fg, s.thF, s.P, s.Gact, s.EvF, s.a, blockIdx.x );
 }
 
 __global__ void batch_theta( const ThetaDesc* __restrict__ d )

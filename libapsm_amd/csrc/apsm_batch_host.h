@@ -86,45 +86,6 @@ void launchBatchDetectAny( hipStream_t s, int nmax, int umax, int threads, const
     }
 }
 
-template <int TP, int NEWPER, int PMAX>
-void launchBatchSeq2( hipStream_t s, const apsm::Seq2Desc* d, int n, int gridX, size_t lds )
-{
-    if ( lds > 64 * 1024 )
-        HIP_OR_THROW( hipFuncSetAttribute( (const void*)apsm::batch_seq2<TP, NEWPER, PMAX>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds ) );
-    hipLaunchKernelGGL( ( apsm::batch_seq2<TP, NEWPER, PMAX> ), dim3( gridX, n ), dim3( apsm::kSeqThreads ), lds, s, d );
-    HIP_OR_THROW( hipGetLastError() );
-}
-
-template <int NEWPER>
-void launchBatchSeq2Tp( hipStream_t s, int tp, const apsm::Seq2Desc* d, int n, int gridX, size_t lds )
-{
-    switch ( tp )
-    {
-    case 2: launchBatchSeq2<2, NEWPER, 24>( s, d, n, gridX, lds ); break;
-    case 4: launchBatchSeq2<4, NEWPER, 16>( s, d, n, gridX, lds ); break;
-    case 7: launchBatchSeq2<7, NEWPER, 12>( s, d, n, gridX, lds ); break;
-    case 10: launchBatchSeq2<10, NEWPER, 10>( s, d, n, gridX, lds ); break;
-    case 16: launchBatchSeq2<16, NEWPER, 8>( s, d, n, gridX, lds ); break;
-    default: launchBatchSeq2<27, NEWPER, 6>( s, d, n, gridX, lds ); break;
-    }
-}
-
-int pmaxOfTp( int tp ) { return apsm::seq2PmaxOfTp( tp ); }
-
-// One block of one instance's train as batched-launch descriptors.
-struct TrainBlk
-{
-    apsm::EntryMfmaDesc e;
-    int nmax;
-    apsm::GramDesc g;
-    apsm::EvDesc v;
-    apsm::Seq2Desc s;
-    bool hasEv;
-    int umax, tp, newPer;
-    size_t lds;
-};
-
 // Host-side descriptor storage: typed arrays appended into one byte buffer; launches refer to
 // offsets that become device pointers once the buffer is uploaded.
 struct DescArena
@@ -259,7 +220,7 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
     {
         apsm_handle* h = B->inst[ i ];
         const apsm_params& p = h->p;
-        const int N = h->N, L = h->L, U = h->U, w2 = h->w2, Wc = w2 / 2;
+        const int N = h->N, L = h->L, U = h->U, w2 = h->w2;
         const int64_t Ti = T[ i ];
         // fresh state: the stream buffer holds this call's pilots only
         h->varSet = true;
@@ -279,119 +240,17 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
 
         const float wG = p.gaussian_kernel_weight, wL = p.linear_kernel_weight;
         const float g2 = 0.5f / h->var * kLog2e;
-        const int64_t q = p.sample_step;
-        const int newPer = (int)( q / 2 );
-        const int64_t R2 = 2 * Ti;
-        const int64_t nStepsTotal = R2 / q;
+        const int64_t nStepsTotal = 2 * Ti / p.sample_step;
         const int64_t steps = blockedSteps( h );
         reserveBlockedScratch( h, steps );
-        const int tp = seq2Tp( Wc );
-        const int nParts = std::min( apsm::kSeqThreads / Wc, ( Wc + tp - 1 ) / tp );
-        if ( tp < 0 || nParts > apsm::kMaxParts || nParts * tp < Wc || nParts > pmaxOfTp( tp ) )
-            throw ApsmError { APSM_ERR_UNSUPPORTED, "window layout does not fit the blocked train path" };
         int64_t a0Next = 0;
         for ( int64_t k0 = 0; k0 < nStepsTotal; k0 += steps )
         {
-            const int64_t nb = std::min( steps, nStepsTotal - k0 );
-            const int64_t sPrev = k0 * q, sFirst = sPrev + q, sLast = sPrev + nb * q;
-            const int64_t a0 = sFirst - std::min<int64_t>( w2, sFirst );
-            const int64_t sNext = sLast + q;
-            a0Next = sNext - std::min<int64_t>( w2, sNext );
-            const int nNewC = (int)( nb * newPer );
-            const int nActC = (int)( ( sLast - a0 ) / 2 );
-            TrainBlk k {};
-            k.umax = umaxOf( U );
-            k.tp = tp;
-            k.newPer = newPer;
-            apsm::EntryArgs& ea = k.e.a;
-            ea.N = N;
-            ea.L = L;
-            ea.U = U;
-            ea.q = (int)q;
-            ea.rowBase = 0;
-            ea.newC0 = sPrev / 2;
-            ea.sFirst = sFirst;
-            ea.H = h->H;
-            ea.a0 = a0;
-            ea.ldYC = ld;
-            ea.nNewC = nNewC;
-            ea.wL = wL;
-            ea.wG = wG;
-            ea.g2 = g2;
-            k.nmax = nmaxOf( N );
-            k.e.Z = b.Z.ptr;
-            k.e.Zn = b.Zn.ptr;
-            k.e.C = b.C.ptr;
-            k.e.thF = h->thOld.ptr;
-            k.e.P = h->Pbuf.ptr;
-            k.e.part = h->Ppart.ptr;
-            apsm::entryChunks( ea, k.e.jBeg, k.e.nChunks );
-            apsm::GramArgs& ga = k.g.a;
-            ga.N = N;
-            ga.L = L;
-            ga.c0 = a0 / 2;
-            ga.nA = nActC;
-            ga.wL = wL;
-            ga.wG = wG;
-            ga.g2 = g2;
-            k.g.Z = b.Z.ptr;
-            k.g.Zn = b.Zn.ptr;
-            k.g.Gact = h->Gact.ptr;
-            const int64_t loLast = sLast > h->H ? sLast - h->H : 0, loPrev = sPrev > h->H ? sPrev - h->H : 0;
-            k.hasEv = loLast > loPrev;
-            apsm::EvArgs& ev = k.v.a;
-            ev.N = N;
-            ev.L = L;
-            ev.U = U;
-            ev.q = (int)q;
-            ev.w2 = w2;
-            ev.nSteps = (int)nb;
-            ev.rowBase = 0;
-            ev.sPrev = sPrev;
-            ev.sFirst = sFirst;
-            ev.H = h->H;
-            ev.ldYC = ld;
-            ev.wG = wG;
-            ev.g2 = g2;
-            k.v.Z = b.Z.ptr;
-            k.v.Zn = b.Zn.ptr;
-            k.v.C = b.C.ptr;
-            k.v.EvF = h->EvF.ptr;
-            apsm::Seq2Args& s2 = k.s.a;
-            s2.N = N;
-            s2.L = L;
-            s2.U = U;
-            s2.w2 = w2;
-            s2.Wc = Wc;
-            s2.q = (int)q;
-            s2.nSteps = (int)nb;
-            s2.hasEv = k.hasEv ? 1 : 0;
-            s2.nParts = nParts;
-            s2.ramp = a0 == 0 ? 1 : 0;
-            s2.a0modW = (int)( a0 % w2 );
-            s2.sFirstRel = (int)( sFirst - a0 );
-            s2.nNewC = nNewC;
-            s2.nActC = nActC;
-            s2.newRel0 = (int)( ( sPrev - a0 ) / 2 );
-            s2.nFr = (int)( ( a0Next - a0 ) / 2 );
-            s2.ldYC = ld;
-            s2.wL = wL;
-            s2.wG = wG;
-            s2.eB = p.eB;
-            k.s.Z = b.Z.ptr + ( a0 / 2 ) * L;
-            k.s.Zn = b.Zn.ptr + a0 / 2;
-            k.s.Y = b.Y.ptr + a0;
-            k.s.C = b.C.ptr + a0;
-            k.s.Fg = h->F.ptr;
-            k.s.thF = h->thOld.ptr;
-            k.s.P = h->Pbuf.ptr;
-            k.s.Gact = h->Gact.ptr;
-            k.s.EvF = h->EvF.ptr;
-            k.lds = apsm::seq2LdsBytes( newPer, w2, tp );
-            blocks[ i ].push_back( k );
+            blocks[ i ].emplace_back();
+            a0Next = planBlock( h, b, 0, 0, k0, std::min( steps, nStepsTotal - k0 ), wL, wG, g2, blocks[ i ].back() );
         }
         // stream bookkeeping after the train (same schedule as the kernels)
-        const int64_t used = nStepsTotal * q;
+        const int64_t used = nStepsTotal * p.sample_step;
         h->used = (uint64_t)used;
         h->a0Next = a0Next;
         h->cur = 0;
@@ -528,10 +387,7 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
                                  const int lane = (int)( k % ( nside + 1 ) );
                                  hipStream_t st = lane == 0 ? B->stream : B->side[ lane - 1 ];
                                  const apsm::Seq2Desc* d = (const apsm::Seq2Desc*)( base + sl[ k ].off );
-                                 if ( sl[ k ].newPer == 1 )
-                                     launchBatchSeq2Tp<1>( st, sl[ k ].tp, d, sl[ k ].cnt, sl[ k ].gx, sl[ k ].lds );
-                                 else
-                                     launchBatchSeq2Tp<2>( st, sl[ k ].tp, d, sl[ k ].cnt, sl[ k ].gx, sl[ k ].lds );
+                                 launchSequencer( st, sl[ k ].newPer, sl[ k ].tp, nullptr, d, sl[ k ].cnt, sl[ k ].gx, sl[ k ].lds );
                              }
                              for ( int k = 0; k < nside; k++ )
                              {

@@ -7,6 +7,7 @@
 #include "apsm_capi.h"
 #include "apsm_device.h"
 #include "apsm_train2.h"
+#include "apsm_train_win.h"
 #include "apsm_train_nc.h"
 #include "apsm_batch.h"
 #include "apsm_detect_launch.h"
@@ -409,37 +410,75 @@ bool blockedEligible( const apsm_params& p )
 
 constexpr int64_t kBlockRowsMax = 1024; // real rows entering per block (the active-sample limit binds first)
 
-template <int TP, int NEWPER, int PMAX>
-void launchSeq2( apsm_handle* h, const float* Z, const float* Zn, const float* Y, float* C, const float* Gact, const float* EvF,
-                 const apsm::Seq2Args& s2, size_t lds )
+// Sequencer launchers. One descriptor (single handle) goes as kernel arguments; n > 1 or a device
+// descriptor array is the batched kernel, gridX user workgroups per descriptor.
+template <typename K>
+void allowLds( K kernel, size_t lds )
 {
-    if ( s2.nParts > PMAX || PMAX * s2.Wc > apsm::kRedF )
-        throw ApsmError { APSM_ERR_UNSUPPORTED, "window layout does not fit the blocked train path" };
     if ( lds > 64 * 1024 )
-        HIP_OR_THROW( hipFuncSetAttribute( (const void*)apsm::apsm_train_seq2<TP, NEWPER, PMAX>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds ) );
-    hipLaunchKernelGGL( ( apsm::apsm_train_seq2<TP, NEWPER, PMAX> ), dim3( h->U ), dim3( apsm::kSeqThreads ), lds, h->stream, Z, Zn,
-                        Y, C, h->F.ptr, h->thOld.ptr, h->Pbuf.ptr, Gact, EvF, s2 );
+        HIP_OR_THROW( hipFuncSetAttribute( (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds ) );
+}
+
+template <int TP>
+void launchWinTp( hipStream_t s, const apsm::Seq2Desc* one, const apsm::Seq2Desc* d, int n, int gridX, size_t lds )
+{
+    if ( one )
+    {
+        allowLds( apsm::apsm_train_win<TP>, lds );
+        hipLaunchKernelGGL( ( apsm::apsm_train_win<TP> ), dim3( gridX ), dim3( apsm::winThreads( TP ) ), lds, s, one->Z, one->Zn, one->Y,
+                            one->C, one->Fg, one->thF, one->P, one->Gact, one->EvF, one->a );
+    }
+    else
+    {
+        allowLds( apsm::batch_train_win<TP>, lds );
+        hipLaunchKernelGGL( ( apsm::batch_train_win<TP> ), dim3( gridX, n ), dim3( apsm::winThreads( TP ) ), lds, s, d );
+    }
     HIP_OR_THROW( hipGetLastError() );
 }
 
-// Instantiations: (register triples per thread, upper bound of the t-slot part count).
-template <int NEWPER>
-void launchSeq2Tp( apsm_handle* h, int tp, const float* Z, const float* Zn, const float* Y, float* C, const float* Gact, const float* EvF,
-                   const apsm::Seq2Args& s2, size_t lds )
+template <int TP, int PMAX>
+void launchSeq2Tp( hipStream_t s, const apsm::Seq2Desc* one, const apsm::Seq2Desc* d, int n, int gridX, size_t lds )
 {
+    if ( one )
+    {
+        allowLds( apsm::apsm_train_seq2<TP, 2, PMAX>, lds );
+        hipLaunchKernelGGL( ( apsm::apsm_train_seq2<TP, 2, PMAX> ), dim3( gridX ), dim3( apsm::kSeqThreads ), lds, s, one->Z, one->Zn, one->Y,
+                            one->C, one->Fg, one->thF, one->P, one->Gact, one->EvF, one->a );
+    }
+    else
+    {
+        allowLds( apsm::batch_seq2<TP, 2, PMAX>, lds );
+        hipLaunchKernelGGL( ( apsm::batch_seq2<TP, 2, PMAX> ), dim3( gridX, n ), dim3( apsm::kSeqThreads ), lds, s, d );
+    }
+    HIP_OR_THROW( hipGetLastError() );
+}
+
+// newPer 1 (sampleStep 2): the window sequencer; newPer 2 (sampleStep 4): two samples enter per
+// step, which the window sequencer's early takeover does not cover.
+void launchSequencer( hipStream_t s, int newPer, int tp, const apsm::Seq2Desc* one, const apsm::Seq2Desc* d, int n, int gridX, size_t lds )
+{
+    if ( newPer == 1 )
+        switch ( tp )
+        {
+        case 5: launchWinTp<5>( s, one, d, n, gridX, lds ); return;
+        case 10: launchWinTp<10>( s, one, d, n, gridX, lds ); return;
+        case 16: launchWinTp<16>( s, one, d, n, gridX, lds ); return;
+        case 20: launchWinTp<20>( s, one, d, n, gridX, lds ); return;
+        case 28: launchWinTp<28>( s, one, d, n, gridX, lds ); return;
+        default: launchWinTp<40>( s, one, d, n, gridX, lds ); return;
+        }
     switch ( tp )
     {
-    case 2: launchSeq2<2, NEWPER, 24>( h, Z, Zn, Y, C, Gact, EvF, s2, lds ); break;
-    case 4: launchSeq2<4, NEWPER, 16>( h, Z, Zn, Y, C, Gact, EvF, s2, lds ); break;
-    case 7: launchSeq2<7, NEWPER, 12>( h, Z, Zn, Y, C, Gact, EvF, s2, lds ); break;
-    case 10: launchSeq2<10, NEWPER, 10>( h, Z, Zn, Y, C, Gact, EvF, s2, lds ); break;
-    case 16: launchSeq2<16, NEWPER, 8>( h, Z, Zn, Y, C, Gact, EvF, s2, lds ); break;
-    default: launchSeq2<27, NEWPER, 6>( h, Z, Zn, Y, C, Gact, EvF, s2, lds ); break;
+    case 2: launchSeq2Tp<2, 24>( s, one, d, n, gridX, lds ); return;
+    case 4: launchSeq2Tp<4, 16>( s, one, d, n, gridX, lds ); return;
+    case 7: launchSeq2Tp<7, 12>( s, one, d, n, gridX, lds ); return;
+    case 10: launchSeq2Tp<10, 10>( s, one, d, n, gridX, lds ); return;
+    case 16: launchSeq2Tp<16, 8>( s, one, d, n, gridX, lds ); return;
+    default: launchSeq2Tp<27, 6>( s, one, d, n, gridX, lds ); return;
     }
 }
 
-// Gram register triples per thread for a window of Wc complex slots (see apsm_train_seq2).
+// apsm_train_seq2: Gram register triples per thread for a window of Wc complex slots.
 int seq2Tp( int Wc )
 {
     const int parts = apsm::kSeqThreads / Wc;
@@ -451,7 +490,9 @@ int seq2Tp( int Wc )
 }
 
 // Projection steps per block of the blocked path: entering rows <= H - W + q (no active row
-// leaves the dictionary inside a block), active samples <= kActMax.
+// leaves the dictionary inside a block), active samples <= kActMax, and for the window sequencer
+// a block Gram buffer no larger than the triangle of kActMax samples (324 steps at windowSize 160,
+// 463 at 40).
 int64_t blockedSteps( const apsm_handle* h )
 {
     const int64_t q = h->p.sample_step;
@@ -461,6 +502,9 @@ int64_t blockedSteps( const apsm_handle* h )
         steps--;
     if ( ( w2 + steps * q ) / 2 > apsm::kActMax )
         throw ApsmError { APSM_ERR_UNSUPPORTED, "window too large for the blocked train path" };
+    if ( q == 2 )
+        while ( steps > 1 && apsm::winGactFloats( w2 / 2, (int)steps ) > apsm::gramRow<int64_t>( apsm::kActMax ) )
+            steps--;
     return steps;
 }
 
@@ -471,149 +515,203 @@ void reserveBlockedScratch( apsm_handle* h, int64_t steps )
     const int newPer = (int)( q / 2 );
     h->Pbuf.ensure( (size_t)h->U * steps * newPer * 2 );
     h->Ppart.ensure( (size_t)h->U * ( h->Hc / apsm::kEntryChunk + 2 ) * steps * newPer * 2 );
-    h->Gact.ensure( (size_t)apsm::gramRow<int64_t>( ( h->w2 + steps * q ) / 2 ) );
-    h->EvF.ensure( (size_t)h->U * steps * h->w2 );
+    if ( newPer == 1 )
+    {
+        h->Gact.ensure( (size_t)apsm::winGactFloats( h->w2 / 2, (int)steps ) );
+        h->EvF.ensure( (size_t)h->U * steps * apsm::winEvStride( h->w2 ) + 256 ); // whole 256-float copies
+    }
+    else
+    {
+        h->Gact.ensure( (size_t)apsm::gramRow<int64_t>( ( h->w2 + steps * q ) / 2 ) );
+        h->EvF.ensure( (size_t)h->U * steps * h->w2 );
+    }
+}
+
+// One block of a train call as launch descriptors.
+struct TrainBlk
+{
+    apsm::EntryMfmaDesc e;
+    int nmax;
+    apsm::GramDesc g;
+    apsm::EvDesc v;
+    apsm::Seq2Desc s;
+    bool hasEv;
+    int umax, tp, newPer;
+    size_t lds;
+};
+
+// The descriptors of the block of n steps from step k0 of a call that continues a stream of
+// usedOld real rows; b holds the call's stream from absolute real row rowBase on. Returns the frozen
+// boundary after the block.
+int64_t planBlock( const apsm_handle* h, const StreamBuf& b, int64_t usedOld, int64_t rowBase, int64_t k0, int64_t n, float wL, float wG,
+                   float g2, TrainBlk& k )
+{
+    const int N = h->N, L = h->L, U = h->U, w2 = h->w2, Wc = w2 / 2;
+    const int64_t q = h->p.sample_step, ld = 2 * b.capK;
+    const int64_t sPrev = usedOld + k0 * q, sFirst = sPrev + q, sLast = sPrev + n * q;
+    const int64_t a0 = sFirst - std::min<int64_t>( w2, sFirst );
+    const int64_t sNext = sLast + q;
+    const int64_t a0Next = sNext - std::min<int64_t>( w2, sNext );
+    k = TrainBlk {};
+    k.newPer = (int)( q / 2 );
+    k.umax = umaxOf( std::min( U, 16 ) );
+    k.nmax = nmaxOf( N );
+    const bool win = k.newPer == 1;
+    k.tp = win ? apsm::winTp( Wc ) : seq2Tp( Wc );
+    int nParts = 0;
+    if ( !win && k.tp > 0 )
+        nParts = std::min( apsm::kSeqThreads / Wc, ( Wc + k.tp - 1 ) / k.tp );
+    if ( k.tp < 0
+         || ( !win && ( nParts > apsm::kMaxParts || nParts * k.tp < Wc || nParts > apsm::seq2PmaxOfTp( k.tp ) || apsm::seq2PmaxOfTp( k.tp ) * Wc > apsm::kRedF ) ) )
+        throw ApsmError { APSM_ERR_UNSUPPORTED, "window layout does not fit the blocked train path" };
+
+    apsm::EntryArgs& ea = k.e.a;
+    ea.N = N;
+    ea.L = L;
+    ea.U = U;
+    ea.q = (int)q;
+    ea.rowBase = rowBase;
+    ea.newC0 = ( sPrev - rowBase ) / 2;
+    ea.sFirst = sFirst;
+    ea.H = h->H;
+    ea.a0 = a0;
+    ea.ldYC = ld;
+    ea.nNewC = (int)( n * k.newPer );
+    ea.wL = wL;
+    ea.wG = wG;
+    ea.g2 = g2;
+    k.e.Z = b.Z.ptr;
+    k.e.Zn = b.Zn.ptr;
+    k.e.C = b.C.ptr;
+    k.e.thF = h->thOld.ptr;
+    k.e.P = h->Pbuf.ptr;
+    k.e.part = h->Ppart.ptr;
+    apsm::entryChunks( ea, k.e.jBeg, k.e.nChunks );
+
+    apsm::GramArgs& ga = k.g.a;
+    ga.N = N;
+    ga.L = L;
+    ga.c0 = ( a0 - rowBase ) / 2;
+    ga.nA = ( sLast - a0 ) / 2;
+    ga.wL = wL;
+    ga.wG = wG;
+    ga.g2 = g2;
+    if ( win )
+    {
+        ga.Wc = Wc;
+        ga.newRel0 = (int)( ( sPrev - a0 ) / 2 );
+        ga.cMod = (int)( a0 / 2 % Wc );
+        ga.tp = k.tp;
+    }
+    k.g.Z = b.Z.ptr;
+    k.g.Zn = b.Zn.ptr;
+    k.g.Gact = h->Gact.ptr;
+
+    const int64_t loLast = sLast > h->H ? sLast - h->H : 0, loPrev = sPrev > h->H ? sPrev - h->H : 0;
+    k.hasEv = loLast > loPrev;
+    apsm::EvArgs& ev = k.v.a;
+    ev.N = N;
+    ev.L = L;
+    ev.U = U;
+    ev.q = (int)q;
+    ev.w2 = w2;
+    ev.nSteps = (int)n;
+    ev.stride = win ? apsm::winEvStride( w2 ) : w2;
+    ev.bySlot = win ? 1 : 0;
+    ev.rowBase = rowBase;
+    ev.sPrev = sPrev;
+    ev.sFirst = sFirst;
+    ev.H = h->H;
+    ev.ldYC = ld;
+    ev.wG = wG;
+    ev.g2 = g2;
+    k.v.Z = b.Z.ptr;
+    k.v.Zn = b.Zn.ptr;
+    k.v.C = b.C.ptr;
+    k.v.EvF = h->EvF.ptr;
+
+    apsm::Seq2Args& s2 = k.s.a;
+    s2.N = N;
+    s2.L = L;
+    s2.U = U;
+    s2.w2 = w2;
+    s2.Wc = Wc;
+    s2.q = (int)q;
+    s2.nSteps = (int)n;
+    s2.hasEv = k.hasEv ? 1 : 0;
+    s2.nParts = nParts;
+    s2.ramp = a0 == 0 ? 1 : 0;
+    s2.a0modW = (int)( a0 % w2 );
+    s2.sFirstRel = (int)( sFirst - a0 );
+    s2.nNewC = ea.nNewC;
+    s2.nActC = (int)ga.nA;
+    s2.newRel0 = (int)( ( sPrev - a0 ) / 2 );
+    s2.nFr = (int)( ( a0Next - a0 ) / 2 );
+    s2.ldYC = ld;
+    s2.wL = wL;
+    s2.wG = wG;
+    s2.eB = h->p.eB;
+    const int64_t aR = a0 - rowBase; // local real row of the first active row
+    k.s.Z = b.Z.ptr + ( aR / 2 ) * L;
+    k.s.Zn = b.Zn.ptr + aR / 2;
+    k.s.Y = b.Y.ptr + aR;
+    k.s.C = b.C.ptr + aR;
+    k.s.Fg = h->F.ptr;
+    k.s.thF = h->thOld.ptr;
+    k.s.P = h->Pbuf.ptr;
+    k.s.Gact = h->Gact.ptr;
+    k.s.EvF = h->EvF.ptr;
+    k.lds = win ? apsm::winLdsBytes( k.tp ) : apsm::seq2LdsBytes( k.newPer, w2, k.tp );
+    return a0Next;
 }
 
 // Runs the projection steps of one call in blocks (see apsm_train2.h).
-void trainBlocked( apsm_handle* h, const StreamBuf& b, int64_t ld, int64_t usedOld, int64_t R2, int64_t rowBase, float wL, float wG,
-                   float g2 )
+void trainBlocked( apsm_handle* h, const StreamBuf& b, int64_t usedOld, int64_t R2, int64_t rowBase, float wL, float wG, float g2 )
 {
-    const int64_t q = h->p.sample_step;
-    const int w2 = h->w2, Wc = w2 / 2, U = h->U;
-    const int newPer = (int)( q / 2 );
-    const int64_t nStepsTotal = R2 / q;
+    const int64_t nStepsTotal = R2 / h->p.sample_step;
     const int64_t steps = blockedSteps( h );
     reserveBlockedScratch( h, steps );
-
-    const int tp = seq2Tp( Wc );
-    if ( tp < 0 )
-        throw ApsmError { APSM_ERR_UNSUPPORTED, "window too large for the blocked train path" };
-    const int nParts = std::min( apsm::kSeqThreads / Wc, ( Wc + tp - 1 ) / tp );
-    if ( nParts > apsm::kMaxParts || nParts * tp < Wc )
-        throw ApsmError { APSM_ERR_UNSUPPORTED, "window layout does not fit the blocked train path" };
-
-    const int nmax = nmaxOf( h->N );
+    const int U = h->U;
     for ( int64_t k0 = 0; k0 < nStepsTotal; k0 += steps )
     {
-        const int64_t n = std::min( steps, nStepsTotal - k0 );
-        const int64_t sPrev = usedOld + k0 * q, sFirst = sPrev + q, sLast = sPrev + n * q;
-        const int64_t a0 = sFirst - std::min<int64_t>( w2, sFirst );
-        const int64_t sNext = sLast + q;
-        const int64_t a0Next = sNext - std::min<int64_t>( w2, sNext );
-        const int nNewC = (int)( n * newPer );
-        const int nActC = (int)( ( sLast - a0 ) / 2 );
-
-        apsm::EntryArgs ea {};
-        ea.N = h->N;
-        ea.L = h->L;
-        ea.U = U;
-        ea.q = (int)q;
-        ea.rowBase = rowBase;
-        ea.newC0 = ( sPrev - rowBase ) / 2;
-        ea.sFirst = sFirst;
-        ea.H = h->H;
-        ea.a0 = a0;
-        ea.ldYC = ld;
-        ea.nNewC = nNewC;
-        ea.wL = wL;
-        ea.wG = wG;
-        ea.g2 = g2;
-        int64_t jBeg = 0;
-        int nChunks = 0;
-        apsm::entryChunks( ea, jBeg, nChunks );
-
-        apsm::GramArgs ga {};
-        ga.N = h->N;
-        ga.L = h->L;
-        ga.c0 = ( a0 - rowBase ) / 2;
-        ga.nA = nActC;
-        ga.wL = wL;
-        ga.wG = wG;
-        ga.g2 = g2;
-        const int64_t loLast = sLast > h->H ? sLast - h->H : 0, loPrev = sPrev > h->H ? sPrev - h->H : 0;
-        const int hasEv = loLast > loPrev ? 1 : 0;
-        apsm::EvArgs ev {};
-        ev.N = h->N;
-        ev.L = h->L;
-        ev.U = U;
-        ev.q = (int)q;
-        ev.w2 = w2;
-        ev.nSteps = (int)n;
-        ev.rowBase = rowBase;
-        ev.sPrev = sPrev;
-        ev.sFirst = sFirst;
-        ev.H = h->H;
-        ev.ldYC = ld;
-        ev.wG = wG;
-        ev.g2 = g2;
+        TrainBlk k;
+        const int64_t a0Next = planBlock( h, b, usedOld, rowBase, k0, std::min( steps, nStepsTotal - k0 ), wL, wG, g2, k );
+        const int nNewC = k.e.a.nNewC, nChunks = k.e.nChunks;
 
         // one launch for the entry share of the first 16 users, the Gram and the eviction
         // shares; further user groups get entry launches of their own; then the combines
         const int evPre = h->prof ? profRecord( h ) : -1;
         for ( int u0 = 0; u0 < U; u0 += 16 )
         {
-            apsm::EntryArgs eu = ea;
+            apsm::EntryArgs eu = k.e.a;
             eu.U = std::min( 16, U - u0 );
-            const float* Cg = b.C.ptr + (size_t)u0 * ld;
-            float* partG = h->Ppart.ptr + (size_t)u0 * nChunks * nNewC * 2;
+            const float* Cg = k.e.C + (size_t)u0 * eu.ldYC;
+            float* partG = k.e.part + (size_t)u0 * nChunks * nNewC * 2;
             if ( u0 == 0 )
             {
                 apsm::PreDesc pd {};
-                pd.e = apsm::EntryMfmaDesc { b.Z.ptr, b.Zn.ptr, Cg, h->thOld.ptr, h->Pbuf.ptr, partG, eu, jBeg, nChunks };
-                pd.g = apsm::GramDesc { b.Z.ptr, b.Zn.ptr, h->Gact.ptr, ga };
-                pd.v = apsm::EvDesc { b.Z.ptr, b.Zn.ptr, b.C.ptr, h->EvF.ptr, ev };
-                pd.hasEv = hasEv;
+                pd.e = k.e;
+                pd.e.a = eu;
+                pd.g = k.g;
+                pd.v = k.v;
+                pd.hasEv = k.hasEv ? 1 : 0;
                 apsm::preShape( pd );
-                HIP_OR_THROW( apsm::launchBlockPre( nmax, umaxOf( eu.U ), h->stream, pd ) );
+                HIP_OR_THROW( apsm::launchBlockPre( k.nmax, umaxOf( eu.U ), h->stream, pd ) );
             }
             else
-                HIP_OR_THROW( apsm::launchEntryMfma( nmax, umaxOf( eu.U ), h->stream, b.Z.ptr, b.Zn.ptr, Cg, partG, eu, jBeg, nChunks, 0,
+                HIP_OR_THROW( apsm::launchEntryMfma( k.nmax, umaxOf( eu.U ), h->stream, k.e.Z, k.e.Zn, Cg, partG, eu, k.e.jBeg, nChunks, 0,
                                                      nChunks * apsm::entryTiles( nNewC ) ) );
         }
         for ( int u0 = 0; u0 < U; u0 += 16 )
         {
-            apsm::EntryArgs eu = ea;
+            apsm::EntryArgs eu = k.e.a;
             eu.U = std::min( 16, U - u0 );
-            const float* thg = h->thOld.ptr + (size_t)u0 * h->L;
-            float* Pg = h->Pbuf.ptr + (size_t)u0 * nNewC * 2;
-            float* partG = h->Ppart.ptr + (size_t)u0 * nChunks * nNewC * 2;
-            HIP_OR_THROW( apsm::launchEntryCombine( h->stream, b.Z.ptr, thg, partG, Pg, eu, nChunks ) );
+            HIP_OR_THROW( apsm::launchEntryCombine( h->stream, k.e.Z, k.e.thF + (size_t)u0 * h->L, k.e.part + (size_t)u0 * nChunks * nNewC * 2,
+                                                    k.e.P + (size_t)u0 * nNewC * 2, eu, nChunks ) );
         }
-
-        apsm::Seq2Args s2 {};
-        s2.N = h->N;
-        s2.L = h->L;
-        s2.U = U;
-        s2.w2 = w2;
-        s2.Wc = Wc;
-        s2.q = (int)q;
-        s2.nSteps = (int)n;
-        s2.hasEv = hasEv;
-        s2.nParts = nParts;
-        s2.ramp = a0 == 0 ? 1 : 0;
-        s2.a0modW = (int)( a0 % w2 );
-        s2.sFirstRel = (int)( sFirst - a0 );
-        s2.nNewC = nNewC;
-        s2.nActC = nActC;
-        s2.newRel0 = (int)( ( sPrev - a0 ) / 2 );
-        s2.nFr = (int)( ( a0Next - a0 ) / 2 );
-        s2.ldYC = ld;
-        s2.wL = wL;
-        s2.wG = wG;
-        s2.eB = h->p.eB;
-        const size_t lds = apsm::seq2LdsBytes( newPer, w2, tp );
         const int evSeq = h->prof ? profRecord( h ) : -1;
         profMark( h, APSM_PROFILE_BLOCK_PRE, evPre, evSeq );
-        const int64_t aR = a0 - rowBase; // local real row of the first active row
-        const float* Za = b.Z.ptr + ( aR / 2 ) * h->L;
-        const float* Zna = b.Zn.ptr + aR / 2;
-        const float* Ya = b.Y.ptr + aR;
-        float* Ca = b.C.ptr + aR;
-        if ( newPer == 1 )
-            launchSeq2Tp<1>( h, tp, Za, Zna, Ya, Ca, h->Gact.ptr, h->EvF.ptr, s2, lds );
-        else
-            launchSeq2Tp<2>( h, tp, Za, Zna, Ya, Ca, h->Gact.ptr, h->EvF.ptr, s2, lds );
+        launchSequencer( h->stream, k.newPer, k.tp, &k.s, nullptr, 1, U, k.lds );
         if ( h->prof )
             profMark( h, APSM_PROFILE_SEQUENCER, evSeq, profRecord( h ) );
         h->a0Next = a0Next;
@@ -779,7 +877,7 @@ void trainDev( apsm_handle* h, const float* d_rx, const float* d_tx, int64_t T, 
             + apsm::kSeqWaves * apsm::kWave );
     HIP_OR_THROW( hipEventRecord( h->ev0, h->stream ) );
     if ( h->blocked )
-        trainBlocked( h, nb, ld, (int64_t)h->used, 2 * T, a.rowBase, wL, wG, a.g2 );
+        trainBlocked( h, nb, (int64_t)h->used, 2 * T, a.rowBase, wL, wG, a.g2 );
     else if ( p.norm_constraint > 0.f )
     {
         apsm::NcArgs nca { h->GramG.ptr, h->FG.ptr, h->Qn.ptr, p.norm_constraint };

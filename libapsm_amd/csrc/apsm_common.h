@@ -12,6 +12,7 @@ constexpr int kWave = 64;
 constexpr int kSeqThreads = 1024; // train sequencer workgroup
 constexpr int kSeqWaves = kSeqThreads / kWave;
 constexpr int kNewMax = 4; // complex samples entering per chunk inside one step
+constexpr int kActMax = 512; // active complex samples of a train block (host guarantees)
 constexpr int kDetTile = 64; // dictionary entries per LDS tile in detect
 constexpr int kDetThreads = 256;
 
@@ -60,14 +61,17 @@ __device__ __forceinline__ void pairDots( const float* __restrict__ x, const flo
 struct EvArgs
 {
     int N, L, U, q, w2, nSteps;
+    int stride; // floats per (user, step)
+    int bySlot; // place of a window row: 0 its position in the window, 1 its slot (absolute row % w2)
     int64_t rowBase, sPrev, sFirst, H, ldYC;
     float wG, g2;
 };
 
 // EvF[u][k][2*pc + part]: Gaussian share of the rows leaving the dictionary at step k, for
-// the window row at position 2*pc + part (row s_k - W_k + 2*pc + part) if it entered before
-// step k; zero otherwise. One thread per (step, complex window position); the kernel values
-// of the (at most kNewMax) leaving samples are computed once and contracted for every user.
+// the window row at position 2*pc + part (row s_k - W_k + 2*pc + part), or with bySlot for the
+// window row in real slot 2*pc + part, if it entered before step k; zero otherwise. One thread per
+// (step, complex window position or slot); the kernel values of the (at most kNewMax) leaving
+// samples are computed once and contracted for every user.
 __device__ __forceinline__ void evictCorrBody( const float* __restrict__ Z, const float* __restrict__ Zn, const float* __restrict__ C,
                                                float* __restrict__ EvF, const EvArgs& a, const int64_t idx )
 {
@@ -79,8 +83,17 @@ __device__ __forceinline__ void evictCorrBody( const float* __restrict__ Z, cons
     const int64_t sp = kk == 0 ? a.sPrev : s - a.q;
     const int64_t W = s < a.w2 ? s : a.w2;
     const int64_t lo = s > a.H ? s - a.H : 0, loP = sp > a.H ? sp - a.H : 0;
-    const int64_t r = s - W + 2 * pc; // absolute real row (a-row of the complex sample)
-    const bool live = ( 2 * pc < W ) && ( r < sp ) && ( lo > loP );
+    int64_t r = s - W + 2 * pc; // absolute real row (a-row of the complex sample)
+    bool live = 2 * pc < W;
+    if ( a.bySlot )
+    {
+        const int64_t cl = s / 2 - 1; // the newest window sample; slot pc holds cl - ((cl - pc) mod Wc)
+        int dt = (int)( cl % Wc ) - pc;
+        dt += dt < 0 ? Wc : 0;
+        r = 2 * ( cl - dt );
+        live = r >= 0;
+    }
+    live = live && r < sp && lo > loP;
     const int64_t e0 = ( loP - a.rowBase ) / 2;
     const int ne = live ? (int)( ( lo - loP ) / 2 ) : 0; // <= kNewMax
     float K0[ kNewMax ], K1[ kNewMax ], K2[ kNewMax ];
@@ -115,7 +128,7 @@ __device__ __forceinline__ void evictCorrBody( const float* __restrict__ Z, cons
                 dFb += ca * K2[ i ] + cb * K0[ i ];
             }
         }
-        float* o = EvF + ( (int64_t)u * a.nSteps + kk ) * a.w2;
+        float* o = EvF + ( (int64_t)u * a.nSteps + kk ) * a.stride;
         o[ 2 * pc ] = a.wG * dFa;
         o[ 2 * pc + 1 ] = a.wG * dFb;
     }

@@ -81,9 +81,13 @@ struct EntryMfmaDesc
 // to c0), kappa = wL x.z + wG K in the three real forms A = kappa(a_i,a_j) = kappa(b_i,b_j),
 // B = kappa(a_i,b_j), C = kappa(b_i,a_j); 32 x 32 sample blocks of the lower triangle on the
 // matrix cores, four per workgroup.
+// With Wc > 0 the buffer has the window sequencer's layout instead (apsm_train_win.h): Wc the
+// window's complex samples, newRel0 the first entering sample (relative to c0), cMod the slot of
+// sample 0, tp its t-slots per lane.
 struct GramArgs
 {
     int N, L;
+    int Wc, newRel0, cMod, tp;
     int64_t c0; // local complex index of the first active sample
     int64_t nA; // active complex samples
     float wL, wG, g2;

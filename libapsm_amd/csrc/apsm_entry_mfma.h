@@ -218,7 +218,12 @@ __device__ __forceinline__ void blockPreBody( const PreDesc& d, int b )
     {
         const int64_t blk = (int64_t)b * ( kMfmaThreads / 64 ) + ( threadIdx.x >> 6 );
         if ( blk < gramBlocks( d.g.a.nA ) )
-            gramBlockMfma<NMAX>( d.g.Z, d.g.Zn, d.g.Gact, d.g.a, blk );
+        {
+            if ( d.g.a.Wc )
+                gramWinMfma<NMAX>( d.g.Z, d.g.Zn, d.g.Gact, d.g.a, blk );
+            else
+                gramBlockMfma<NMAX>( d.g.Z, d.g.Zn, d.g.Gact, d.g.a, blk );
+        }
         return;
     }
     b -= d.gramWg;

@@ -95,7 +95,7 @@ apsm::DetDesc detectDescOf( apsm_handle* h, const float* d_rx, int64_t M, float*
 void planTrainCall( apsm_handle* h, const float* d_rx, const float* d_tx, int64_t T, CallPlan& cp )
 {
     const apsm_params& p = h->p;
-    const int N = h->N, L = h->L, U = h->U, w2 = h->w2, Wc = w2 / 2;
+    const int N = h->N, L = h->L, U = h->U, w2 = h->w2;
     ARG_CHECK( T > 0, "train needs at least one pilot" );
     if ( !h->varSet )
     {
@@ -129,115 +129,14 @@ void planTrainCall( apsm_handle* h, const float* d_rx, const float* d_tx, int64_
     cp.stage = apsm::StageDesc { d_rx, d_tx, nb.Z.ptr + nOld * L, nb.Zn.ptr + nOld, nb.Y.ptr + 2 * nOld, nb.C.ptr + 2 * nOld, T, ld, N, U };
 
     const int64_t q = p.sample_step;
-    const int newPer = (int)( q / 2 );
     const int64_t usedOld = (int64_t)h->used, R2 = 2 * T, rowBase = 2 * ( usedC - nOld );
     const int64_t nStepsTotal = R2 / q;
     const int64_t steps = blockedSteps( h );
-    const int tp = seq2Tp( Wc );
-    const int nParts = std::min( apsm::kSeqThreads / Wc, ( Wc + tp - 1 ) / tp );
-    if ( tp < 0 || nParts > apsm::kMaxParts || nParts * tp < Wc || nParts > pmaxOfTp( tp ) )
-        throw ApsmError { APSM_ERR_UNSUPPORTED, "window layout does not fit the blocked train path" };
     int64_t a0Next = h->a0Next;
     for ( int64_t k0 = 0; k0 < nStepsTotal; k0 += steps )
     {
-        const int64_t n = std::min( steps, nStepsTotal - k0 );
-        const int64_t sPrev = usedOld + k0 * q, sFirst = sPrev + q, sLast = sPrev + n * q;
-        const int64_t a0 = sFirst - std::min<int64_t>( w2, sFirst );
-        const int64_t sNext = sLast + q;
-        a0Next = sNext - std::min<int64_t>( w2, sNext );
-        const int nNewC = (int)( n * newPer );
-        const int nActC = (int)( ( sLast - a0 ) / 2 );
-        TrainBlk k {};
-        k.umax = umaxOf( U );
-        k.tp = tp;
-        k.newPer = newPer;
-        apsm::EntryArgs& ea = k.e.a;
-        ea.N = N;
-        ea.L = L;
-        ea.U = U;
-        ea.q = (int)q;
-        ea.rowBase = rowBase;
-        ea.newC0 = ( sPrev - rowBase ) / 2;
-        ea.sFirst = sFirst;
-        ea.H = h->H;
-        ea.a0 = a0;
-        ea.ldYC = ld;
-        ea.nNewC = nNewC;
-        ea.wL = wL;
-        ea.wG = wG;
-        ea.g2 = g2;
-        k.nmax = nmaxOf( N );
-        k.e.Z = nb.Z.ptr;
-        k.e.Zn = nb.Zn.ptr;
-        k.e.C = nb.C.ptr;
-        k.e.thF = h->thOld.ptr;
-        k.e.P = h->Pbuf.ptr;
-        k.e.part = h->Ppart.ptr;
-        apsm::entryChunks( ea, k.e.jBeg, k.e.nChunks );
-        apsm::GramArgs& ga = k.g.a;
-        ga.N = N;
-        ga.L = L;
-        ga.c0 = ( a0 - rowBase ) / 2;
-        ga.nA = nActC;
-        ga.wL = wL;
-        ga.wG = wG;
-        ga.g2 = g2;
-        k.g.Z = nb.Z.ptr;
-        k.g.Zn = nb.Zn.ptr;
-        k.g.Gact = h->Gact.ptr;
-        const int64_t loLast = sLast > h->H ? sLast - h->H : 0, loPrev = sPrev > h->H ? sPrev - h->H : 0;
-        k.hasEv = loLast > loPrev;
-        apsm::EvArgs& ev = k.v.a;
-        ev.N = N;
-        ev.L = L;
-        ev.U = U;
-        ev.q = (int)q;
-        ev.w2 = w2;
-        ev.nSteps = (int)n;
-        ev.rowBase = rowBase;
-        ev.sPrev = sPrev;
-        ev.sFirst = sFirst;
-        ev.H = h->H;
-        ev.ldYC = ld;
-        ev.wG = wG;
-        ev.g2 = g2;
-        k.v.Z = nb.Z.ptr;
-        k.v.Zn = nb.Zn.ptr;
-        k.v.C = nb.C.ptr;
-        k.v.EvF = h->EvF.ptr;
-        apsm::Seq2Args& s2 = k.s.a;
-        s2.N = N;
-        s2.L = L;
-        s2.U = U;
-        s2.w2 = w2;
-        s2.Wc = Wc;
-        s2.q = (int)q;
-        s2.nSteps = (int)n;
-        s2.hasEv = k.hasEv ? 1 : 0;
-        s2.nParts = nParts;
-        s2.ramp = a0 == 0 ? 1 : 0;
-        s2.a0modW = (int)( a0 % w2 );
-        s2.sFirstRel = (int)( sFirst - a0 );
-        s2.nNewC = nNewC;
-        s2.nActC = nActC;
-        s2.newRel0 = (int)( ( sPrev - a0 ) / 2 );
-        s2.nFr = (int)( ( a0Next - a0 ) / 2 );
-        s2.ldYC = ld;
-        s2.wL = wL;
-        s2.wG = wG;
-        s2.eB = p.eB;
-        const int64_t aR = a0 - rowBase;
-        k.s.Z = nb.Z.ptr + ( aR / 2 ) * L;
-        k.s.Zn = nb.Zn.ptr + aR / 2;
-        k.s.Y = nb.Y.ptr + aR;
-        k.s.C = nb.C.ptr + aR;
-        k.s.Fg = h->F.ptr;
-        k.s.thF = h->thOld.ptr;
-        k.s.P = h->Pbuf.ptr;
-        k.s.Gact = h->Gact.ptr;
-        k.s.EvF = h->EvF.ptr;
-        k.lds = apsm::seq2LdsBytes( newPer, w2, tp );
-        cp.blocks.push_back( k );
+        cp.blocks.emplace_back();
+        a0Next = planBlock( h, nb, usedOld, rowBase, k0, std::min( steps, nStepsTotal - k0 ), wL, wG, g2, cp.blocks.back() );
     }
     // bookkeeping, as trainDev
     const int64_t first = ( p.start_with_full_window && h->used == 0 ) ? w2 : q;
@@ -712,10 +611,7 @@ bool serverLaunchTrainRound( apsm_server* S )
             const int lane = (int)( k % ( nside + 1 ) );
             hipStream_t ss = lane == 0 ? st : S->side[ lane - 1 ];
             const apsm::Seq2Desc* d = (const apsm::Seq2Desc*)( base + sl[ k ].off );
-            if ( sl[ k ].newPer == 1 )
-                launchBatchSeq2Tp<1>( ss, sl[ k ].tp, d, sl[ k ].cnt, sl[ k ].gx, sl[ k ].lds );
-            else
-                launchBatchSeq2Tp<2>( ss, sl[ k ].tp, d, sl[ k ].cnt, sl[ k ].gx, sl[ k ].lds );
+            launchSequencer( ss, sl[ k ].newPer, sl[ k ].tp, nullptr, d, sl[ k ].cnt, sl[ k ].gx, sl[ k ].lds );
         }
         for ( int k = 0; k < nside; k++ )
         {

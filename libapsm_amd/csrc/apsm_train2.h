@@ -25,7 +25,6 @@
 
 namespace apsm {
 
-constexpr int kActMax = 512; // active complex samples per block (host guarantees)
 constexpr int kMaxParts = 32; // t-slot parts of the register Gram (1024 / Wc for Wc >= 32)
 constexpr int kRedF = 2048; // per-part f partial slots (>= PMAX * Wc of every instantiation)
 // Thread roles in the sequencer's entering phase: [0, w2) reduce f (w2 <= 320), [kColBase,

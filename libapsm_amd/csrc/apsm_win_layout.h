@@ -1,0 +1,78 @@
+// Shapes of the window sequencer (apsm_train_win.h) and the layout of what its block precompute
+// writes for it. No kernels here: the Gram's translation unit includes it too.
+#pragma once
+
+#include "apsm_common.h"
+
+namespace apsm {
+
+constexpr int kWinTpCount = 6;
+constexpr int kWinTps[ kWinTpCount ] = { 5, 10, 16, 20, 28, 40 }; // t-slots per lane: windowSize <= 4 TP
+
+// t-slots per lane for a window of Wc complex samples (-1: none fits).
+__host__ __device__ inline int winTp( int Wc )
+{
+    for ( int k = 0; k < kWinTpCount; k++ )
+        if ( Wc <= 4 * kWinTps[ k ] )
+            return kWinTps[ k ];
+    return -1;
+}
+
+// Image of one sample's Gram column in slot order: 4 parts (16-lane rows) of three planes (A, C, B)
+// of TPQ floats; parts padded to 16 bytes.
+__host__ __device__ constexpr int winTpq( int tp ) { return ( tp + 1 ) & ~1; }
+__host__ __device__ constexpr int winPart( int tp ) { return ( 3 * winTpq( tp ) + 3 ) & ~3; }
+__host__ __device__ constexpr int winImg( int tp ) { return 4 * winPart( tp ); }
+__host__ __device__ constexpr int winProductWaves( int tp ) { return ( 4 * tp + 15 ) / 16; }
+// Helper waves: three while the workgroup then has at most 8 waves (256 registers per wave),
+// else two (12 waves at TP = 40: 168 registers, 120 of them the Gram).
+__host__ __device__ constexpr int winHelperWaves( int tp ) { return tp <= 20 ? 3 : 2; }
+__host__ __device__ constexpr int winThreads( int tp ) { return 64 * ( winProductWaves( tp ) + winHelperWaves( tp ) ); }
+// Package buffers: a package is issued BUFS - 2 steps before its first use, which has to cover the
+// memory latency; the short steps of the small windows need more of them.
+__host__ __device__ constexpr int winBufs( int tp ) { return tp <= 20 ? 6 : 4; }
+
+// Block Gram buffer: Wc images of the window's samples at the block start (both orders of every
+// pair), then one package row per entering sample e: its image over the window one step before it
+// enters, 4 floats (kappa with itself: A, C, B, 0), and the kappa with the active samples that have
+// left the window by then, three planes (A, kappa(a_e,b_j), kappa(b_e,a_j)) of ceil4(older) floats.
+__host__ __device__ inline int winOlder( int e, int newRel0, int Wc )
+{
+    const int m = newRel0 + e - Wc;
+    return m > 0 ? m : 0;
+}
+// sum of ceil4(o) over o < m
+__host__ __device__ inline int winOlderSum( int m )
+{
+    if ( m < 2 )
+        return 0;
+    const int full = ( m - 1 ) >> 2, rem = ( m - 1 ) & 3;
+    return 8 * full * ( full + 1 ) + 4 * rem * ( full + 1 );
+}
+__host__ __device__ inline int winRow( int e, int newRel0, int Wc, int tp )
+{
+    return Wc * winImg( tp ) + e * ( winImg( tp ) + 4 ) + 3 * winOlderSum( winOlder( e, newRel0, Wc ) );
+}
+// Floats of a block of `steps` steps (largest: a full window before the block), plus the last
+// package copy's overrun (copies are whole 256-float chunks).
+inline int64_t winGactFloats( int Wc, int steps )
+{
+    return (int64_t)winRow( steps, Wc - 1, Wc, winTp( Wc ) ) + 256;
+}
+// Row stride of the eviction shares [U][steps][stride], in slot order.
+__host__ __device__ inline int winEvStride( int w2 ) { return ( w2 + 3 ) & ~3; }
+
+// Floats of the Gram part of a package buffer: image, self, older planes (at most kActMax samples).
+__host__ __device__ constexpr int winPkGram( int tp ) { return ( winImg( tp ) + 4 + 3 * kActMax + 255 ) & ~255; }
+__host__ __device__ constexpr int winPkCap( int tp ) { return winPkGram( tp ) + ( ( 8 * tp + 255 ) & ~255 ); }
+// Floats of one beta buffer: every slot a lane reads (3 TP + 16 ceil(TP / 16)) or writes.
+__host__ __device__ constexpr int winBetaFloats( int tp )
+{
+    return 2 * ( 3 * tp + 16 * ( ( tp + 15 ) / 16 ) > 16 * winProductWaves( tp ) ? 3 * tp + 16 * ( ( tp + 15 ) / 16 ) : 16 * winProductWaves( tp ) );
+}
+inline size_t winLdsBytes( int tp )
+{
+    return sizeof( float ) * ( (size_t)winBufs( tp ) * winPkCap( tp ) + 2 * winBetaFloats( tp ) + 2 * 32 * winProductWaves( tp ) + 2 * kActMax + 5 * kActMax + 8 );
+}
+
+} // namespace apsm
