@@ -10,8 +10,6 @@
 // the lanes of rows 0 and 2 and the b-part in those of rows 1 and 3. f, c, y and the projection weight
 // of a slot stay in its lanes' registers from the sample's entry to its departure. The only thing
 // that crosses waves is beta, through a double-buffered LDS array: projection k, barrier, product k.
-// A wave reads its beta pairs once per lane (ceil(TP / 16) 8-byte LDS reads) and broadcasts each
-// inside the 16-lane row by DPP (row_newbcast) in the multiply-adds themselves.
 //
 // A sample's f needs its share of every earlier coefficient: H_k = P_k + sum_j c_j kappa(j, k). To keep
 // that off the chain, a sample takes over its u-slot one step EARLY: after projection k - 1 the slot's
@@ -31,102 +29,150 @@
 #include "apsm_train2.h"
 #include "apsm_win_layout.h"
 
+#include <type_traits>
+
 namespace apsm {
 
-// s_waitcnt vmcnt(min(n, 31)) for a wave-uniform n
-__device__ __forceinline__ void waitVmUpTo31( int n )
-{
-    switch ( n )
-    {
-    case 16: waitVm<16>(); break;
-    case 17: waitVm<17>(); break;
-    case 18: waitVm<18>(); break;
-    case 19: waitVm<19>(); break;
-    case 20: waitVm<20>(); break;
-    case 21: waitVm<21>(); break;
-    case 22: waitVm<22>(); break;
-    case 23: waitVm<23>(); break;
-    case 24: waitVm<24>(); break;
-    case 25: waitVm<25>(); break;
-    case 26: waitVm<26>(); break;
-    case 27: waitVm<27>(); break;
-    case 28: waitVm<28>(); break;
-    case 29: waitVm<29>(); break;
-    case 30: waitVm<30>(); break;
-    default:
-        if ( n > 30 )
-            waitVm<31>();
-        else
-            waitVmN( n );
-        break;
-    }
-}
+typedef float wf32x4 __attribute__( ( ext_vector_type( 4 ) ) );
 
-// One register plane of the window Gram: TP floats, read at constant indices, written at a
-// wave-uniform one (VGPR index mode works on up to 32 registers, so TP = 40 is 32 + 8).
+// The window Gram of a lane: planes A, C, B of TP floats, read at constant indices, written at a
+// wave-uniform one. The compiler writes a vector of 9 to 32 registers in VGPR index mode (a shorter one
+// by a select per register, a longer one through memory), so three short planes share one vector
+// and at TP = 40 the last 8 registers of each plane are scalars behind a switch.
 template <int TP>
-struct WinPlane
+struct WinRegs
 {
-    static constexpr int LO = TP <= 32 ? TP : 32, HI = TP <= 32 ? 2 : TP - 32;
-    typedef float VLo __attribute__( ( ext_vector_type( LO ) ) );
-    typedef float VHi __attribute__( ( ext_vector_type( HI ) ) );
-    VLo lo;
-    VHi hi;
-    __device__ __forceinline__ float get( int j ) const { return j < LO ? lo[ j ] : hi[ j - LO ]; }
-    __device__ __forceinline__ void put( int j, float v ) // constant j
+    static constexpr bool ONE = 3 * TP <= 32;
+    static constexpr int LO = ONE ? 3 * TP : TP <= 32 ? TP : 32, TAIL = TP > 32 ? TP - 32 : 0;
+    typedef float V __attribute__( ( ext_vector_type( LO ) ) );
+    V a, c, b; // (ONE: all three planes in a)
+    float ta[ TAIL ? TAIL : 1 ], tc[ TAIL ? TAIL : 1 ], tb[ TAIL ? TAIL : 1 ];
+    __device__ __forceinline__ float get( int plane, int j ) const
     {
+        if ( ONE )
+            return a[ plane * TP + j ];
         if ( j < LO )
-            lo[ j ] = v;
+            return plane == 0 ? a[ j ] : plane == 1 ? c[ j ] : b[ j ];
+        return plane == 0 ? ta[ j - LO ] : plane == 1 ? tc[ j - LO ] : tb[ j - LO ];
+    }
+    __device__ __forceinline__ void put( int plane, int j, float v )
+    {
+        if ( ONE )
+            a[ plane * TP + j ] = v;
+        else if ( j < LO )
+            ( plane == 0 ? a[ j ] = v : plane == 1 ? c[ j ] = v : b[ j ] = v );
         else
-            hi[ j - LO ] = v;
+            ( plane == 0 ? ta[ j - LO ] : plane == 1 ? tc[ j - LO ] : tb[ j - LO ] ) = v;
+    }
+    template <int I>
+    __device__ __forceinline__ void insertTail( int j, float xa, float xc, float xb )
+    {
+        if constexpr ( I < TAIL )
+        {
+            if ( j == LO + I )
+            {
+                ta[ I ] = xa;
+                tc[ I ] = xc;
+                tb[ I ] = xb;
+                asm volatile( "" );
+            }
+            else
+                insertTail<I + 1>( j, xa, xc, xb );
+        }
+    }
+    // Slot j (uniform over the wave) of the lanes that take it. The readfirstlane keeps the lane mask a
+    // branch: as selects, the writes would copy whole planes.
+    __device__ __forceinline__ void insert( int j, bool take, float xa, float xc, float xb )
+    {
+        if ( take )
+        {
+            const int js = __builtin_amdgcn_readfirstlane( j );
+            if ( TAIL == 0 || js < LO )
+            {
+                a[ js ] = xa;
+                if constexpr ( ONE )
+                {
+                    a[ TP + js ] = xc;
+                    a[ 2 * TP + js ] = xb;
+                }
+                else
+                {
+                    c[ js ] = xc;
+                    b[ js ] = xb;
+                }
+            }
+            else
+                insertTail<0>( js, xa, xc, xb );
+        }
     }
 };
 
-// Four t-slots I .. I + 3 of the product: acc += kappa * beta with the beta pair of t-slot I + m taken
-// from lane I + m of the 16-lane row. The leading s_nop gives a preceding vector write of the
-// beta registers (a copy the compiler may place) its two wait states before the DPP reads.
-template <int I>
-__device__ __forceinline__ void winFma4( float& a0, float& b0, float& a1, float& b1, const float bx, const float by, const float A0, const float A1,
-                                         const float A2, const float A3, const float C0, const float C1, const float C2, const float C3,
-                                         const float B0, const float B1, const float B2, const float B3 )
+// The product over this lane's t-slots: fa += A beta_a + C beta_b, fb += B beta_a + A beta_b, the beta pairs
+// (q: two t-slots per 16 bytes) read from LDS, one address per 16-lane row, CH pairs of t-slots ahead
+// of their multiply-adds. Plain register operands on purpose: two waves of a SIMD then issue a
+// multiply-add in 2.2 to 3.1 cycles each (measured), against 4.3 with a DPP or scalar operand, and
+// an FP32 matrix instruction shares the vector ALU's multipliers (4 x 4 x 1: 8.2 cycles for two).
+template <int TP, typename F>
+__device__ __forceinline__ void winProduct( const WinRegs<TP>& g, const float* sBr, float& fa, float& fb, F&& readAhead )
 {
-#define APSM_WF( acc, bt, g, i ) "v_fmac_f32_dpp " acc ", " bt ", " g " row_newbcast:" i " row_mask:0xf bank_mask:0xf\n\t"
-    asm( "s_nop 1\n\t" APSM_WF( "%0", "%4", "%6", "%18" ) APSM_WF( "%1", "%5", "%6", "%18" ) APSM_WF( "%2", "%5", "%10", "%18" )
-             APSM_WF( "%3", "%4", "%14", "%18" ) APSM_WF( "%0", "%4", "%7", "%19" ) APSM_WF( "%1", "%5", "%7", "%19" )
-                 APSM_WF( "%2", "%5", "%11", "%19" ) APSM_WF( "%3", "%4", "%15", "%19" ) APSM_WF( "%0", "%4", "%8", "%20" )
-                     APSM_WF( "%1", "%5", "%8", "%20" ) APSM_WF( "%2", "%5", "%12", "%20" ) APSM_WF( "%3", "%4", "%16", "%20" )
-                         APSM_WF( "%0", "%4", "%9", "%21" ) APSM_WF( "%1", "%5", "%9", "%21" ) APSM_WF( "%2", "%5", "%13", "%21" )
-                             APSM_WF( "%3", "%4", "%17", "%21" )
-         : "+v"( a0 ), "+v"( b0 ), "+v"( a1 ), "+v"( b1 )
-         : "v"( bx ), "v"( by ), "v"( A0 ), "v"( A1 ), "v"( A2 ), "v"( A3 ), "v"( C0 ), "v"( C1 ), "v"( C2 ), "v"( C3 ), "v"( B0 ), "v"( B1 ),
-           "v"( B2 ), "v"( B3 ), "n"( I ), "n"( I + 1 ), "n"( I + 2 ), "n"( I + 3 ) );
-}
-template <int I>
-__device__ __forceinline__ void winFma1( float& a0, float& b0, float& a1, float& b1, const float bx, const float by, const float A, const float C, const float B )
-{
-    asm( "s_nop 1\n\t" APSM_WF( "%0", "%4", "%6", "%9" ) APSM_WF( "%1", "%5", "%6", "%9" ) APSM_WF( "%2", "%5", "%7", "%9" )
-             APSM_WF( "%3", "%4", "%8", "%9" )
-         : "+v"( a0 ), "+v"( b0 ), "+v"( a1 ), "+v"( b1 )
-         : "v"( bx ), "v"( by ), "v"( A ), "v"( C ), "v"( B ), "n"( I ) );
-#undef APSM_WF
+    constexpr int Q = ( TP + 1 ) / 2, CH = 2, NCH = ( Q + CH - 1 ) / CH;
+    const float4* q4 = reinterpret_cast<const float4*>( sBr );
+    float4 q[ 2 ][ CH ];
+#pragma unroll
+    for ( int m = 0; m < CH; m++ )
+        q[ 0 ][ m ] = q4[ m < Q ? m : 0 ];
+    readAhead();
+    asm volatile( "" ::: "memory" ); // the next step's reads go out here, before the product
+    float a0 = 0.f, a1 = 0.f, b0 = 0.f, b1 = 0.f;
+#pragma unroll
+    for ( int ch = 0; ch < NCH; ch++ )
+    {
+#pragma unroll
+        for ( int m = 0; m < CH; m++ )
+            if ( ( ch + 1 ) * CH + m < Q )
+                q[ ( ch + 1 ) & 1 ][ m ] = q4[ ( ch + 1 ) * CH + m ];
+#pragma unroll
+        for ( int m = 0; m < CH; m++ )
+        {
+            const int j = 2 * ( ch * CH + m );
+            const float4 x = q[ ch & 1 ][ m ];
+            if ( j < TP )
+            {
+                a0 = fmaf( x.x, g.get( 0, j ), a0 );
+                b0 = fmaf( x.x, g.get( 2, j ), b0 );
+                a1 = fmaf( x.y, g.get( 1, j ), a1 );
+                b1 = fmaf( x.y, g.get( 0, j ), b1 );
+            }
+            if ( j + 1 < TP )
+            {
+                a0 = fmaf( x.z, g.get( 0, j + 1 ), a0 );
+                b0 = fmaf( x.z, g.get( 2, j + 1 ), b0 );
+                a1 = fmaf( x.w, g.get( 1, j + 1 ), a1 );
+                b1 = fmaf( x.w, g.get( 0, j + 1 ), b1 );
+            }
+        }
+        // bound the reads in flight (registers): the next ones stay behind this chunk's multiply-adds
+        asm volatile( "" : "+v"( a0 ), "+v"( a1 ), "+v"( b0 ), "+v"( b1 )::"memory" );
+    }
+    fa = a0 + a1;
+    fb = b0 + b1;
 }
 
-// The product over t-slots J .. TP - 1 of this lane's part; beta pairs of t-slot j in bt[j / 16].
-template <int TP, int J>
-__device__ __forceinline__ void winProduct( float& a0, float& b0, float& a1, float& b1, const float2* bt, const WinPlane<TP>& gA,
-                                            const WinPlane<TP>& gC, const WinPlane<TP>& gB )
+// Sums of two values over the wave: lanes 0..31 get a's, lanes 32..63 b's.
+__device__ __forceinline__ float waveSumPair( float a, float b )
 {
-    if constexpr ( J + 4 <= TP && J % 16 <= 12 )
-    {
-        winFma4<J % 16>( a0, b0, a1, b1, bt[ J / 16 ].x, bt[ J / 16 ].y, gA.get( J ), gA.get( J + 1 ), gA.get( J + 2 ), gA.get( J + 3 ), gC.get( J ),
-                         gC.get( J + 1 ), gC.get( J + 2 ), gC.get( J + 3 ), gB.get( J ), gB.get( J + 1 ), gB.get( J + 2 ), gB.get( J + 3 ) );
-        winProduct<TP, J + 4>( a0, b0, a1, b1, bt, gA, gC, gB );
-    }
-    else if constexpr ( J < TP )
-    {
-        winFma1<J % 16>( a0, b0, a1, b1, bt[ J / 16 ].x, bt[ J / 16 ].y, gA.get( J ), gC.get( J ), gB.get( J ) );
-        winProduct<TP, J + 1>( a0, b0, a1, b1, bt, gA, gC, gB );
-    }
+    const auto s1 = __builtin_amdgcn_permlane32_swap( __float_as_uint( a ), __float_as_uint( b ), false, false );
+    float v = __uint_as_float( s1[ 0 ] ) + __uint_as_float( s1[ 1 ] );
+    const auto s2 = __builtin_amdgcn_permlane16_swap( __float_as_uint( v ), __float_as_uint( v ), false, false );
+    v = __uint_as_float( s2[ 0 ] ) + __uint_as_float( s2[ 1 ] );
+    int x = __float_as_int( v );
+    v += __int_as_float( __builtin_amdgcn_update_dpp( 0, x, 0x128, 0xF, 0xF, false ) );
+    x = __float_as_int( v );
+    v += __int_as_float( __builtin_amdgcn_update_dpp( 0, x, 0x124, 0xF, 0xF, false ) );
+    x = __float_as_int( v );
+    v += __int_as_float( __builtin_amdgcn_update_dpp( 0, x, 0x4E, 0xF, 0xF, false ) );
+    x = __float_as_int( v );
+    return v + __int_as_float( __builtin_amdgcn_update_dpp( 0, x, 0xB1, 0xF, 0xF, false ) );
 }
 
 // Row indices are relative to the block's first active row a0; Z, Zn point at the first active
@@ -138,9 +184,10 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
                                          const float* __restrict__ EvF, const Seq2Args& a, const int u )
 {
     constexpr int TPQ = winTpq( TP ), PART = winPart( TP ), IMG = winImg( TP ), NP = winProductWaves( TP ), NH = winHelperWaves( TP );
-    constexpr int THREADS = winThreads( TP ), BUFS = winBufs( TP ), MB = ( TP + 15 ) / 16, VS = 16 * NP;
-    constexpr int PKG = winPkGram( TP ), PKCAP = winPkCap( TP ), SB = winBetaFloats( TP );
+    constexpr int THREADS = winThreads( TP ), BUFS = kWinBufs, VS = 16 * NP, RING = winRing( TP );
+    constexpr int PKG = winPkGram( TP ), PKCAP = winPkCap( TP ), NC = PKCAP / 256, SB = winBetaFloats( TP ), RUN = winBetaRun( TP );
     static_assert( VS >= 4 * TP, "a u-slot lane for every slot" );
+    static_assert( NC * ( BUFS - 3 ) <= 63, "copies in flight beyond the wait counter" );
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane( tid / 64 );
     const int Wc = a.Wc, w2 = a.w2, K = a.nSteps, newRel0 = a.newRel0, nAct = a.nActC;
@@ -148,63 +195,67 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
     const int evStride = winEvStride( w2 );
 
     extern __shared__ float sm[];
-    float* sPk = sm; // [BUFS][PKCAP]: Gram part, eviction shares
+    float* sPk = sm; // [BUFS][PKCAP]: image and self entries, eviction shares
     float* sB = sPk + BUFS * PKCAP; // [2][SB]
     float* sCw = sB + 2 * SB; // [2][2 VS]: coefficients of the window after a projection, by slot
     float* sC = sCw + 4 * VS; // [2 kActMax]: coefficients of the active rows that have left the window
-    float* sY = sC + 2 * kActMax; // [2 K]: targets, projection weights and frozen shares of the entering samples
-    float* sInv = sY + 2 * kActMax; // [K]
-    float* sP = sInv + kActMax; // [2 K]
-    float* sH = sP + 2 * kActMax; // [2][4]: entering shares (window + P: a, b; left rows: a, b)
+    // [kActMax + 2][4]: per step the next sample's targets (a, b) and projection weight
+    // 1 / (wL|x|^2 + wG), and 1 / W of the step itself
+    float* sStep = sC + 2 * kActMax;
+    float* sP = sStep + 4 * ( kActMax + 2 ); // [2 K]: frozen shares of the entering samples
+    float* sH = sP + 2 * ( kActMax + 2 ); // [2][NH][2]: entering shares (window rows and P, left rows)
 
     const float* Yu = Y + u * a.ldYC;
     float* Cu = C + u * a.ldYC;
     const float* Pu = P + (int64_t)u * K * 2;
     const float* EvU = EvF + (int64_t)u * K * evStride;
 
-    // ---- packages (one wave) ----
+    // package m into buffer slot (one wave; NC copies whatever m is, so that counting waits are
+    // constants: past the last step the last package again, without eviction shares stale memory
+    // that nothing reads)
     const uint32_t pkLds = __builtin_amdgcn_readfirstlane( (uint32_t)(uintptr_t)( __attribute__( ( address_space( 3 ) ) ) float* )( sPk ) );
-    const int nE = a.hasEv ? ( evStride + 255 ) / 256 : 0;
-    auto pkCopies = [ & ]( int m ) { return ( IMG + 4 + 3 * ( ( winOlder( m, newRel0, Wc ) + 3 ) & ~3 ) + 255 ) / 256 + nE; };
-    auto pkIssue = [ & ]( int m ) {
-        const uint32_t dst = pkLds + (uint32_t)( ( m % BUFS ) * PKCAP ) * 4u;
-        const float* src = Gact + winRow( m, newRel0, Wc, TP );
-        const int nG = pkCopies( m ) - nE;
-#pragma unroll 1
-        for ( int d = 0; d < nG; d++ )
+    auto pkIssue = [ & ]( int m, int slot ) {
+        const int mm = m < K ? m : K - 1;
+        const uint32_t dst = pkLds + (uint32_t)( slot * PKCAP ) * 4u;
+        const float* src = Gact + winRow( mm, newRel0, Wc, TP );
+        const float* ev = EvU + (int64_t)mm * evStride;
+#pragma unroll
+        for ( int d = 0; d < PKG / 256; d++ )
             dmaDwordx4( src + d * 256, 16u * (uint32_t)lane, __builtin_amdgcn_readfirstlane( dst + (uint32_t)d * 1024u ) );
-        const float* ev = EvU + (int64_t)m * evStride;
-#pragma unroll 1
-        for ( int d = 0; d < nE; d++ )
+#pragma unroll
+        for ( int d = 0; d < ( PKCAP - PKG ) / 256; d++ )
             dmaDwordx4( ev + d * 256, 16u * (uint32_t)lane, __builtin_amdgcn_readfirstlane( dst + (uint32_t)( PKG + d * 256 ) * 4u ) );
     };
     if ( wave == NP )
-        for ( int m = 0; m < BUFS && m < K; m++ )
-            pkIssue( m );
+        for ( int m = 0; m < BUFS; m++ )
+            pkIssue( m, m );
 
     for ( int i = tid; i < 2 * SB; i += THREADS )
         sB[ i ] = 0.f;
     for ( int i = tid; i < 2 * kActMax; i += THREADS )
         sC[ i ] = 0.f;
     for ( int i = tid; i < 2 * K; i += THREADS )
-    {
-        sY[ i ] = Yu[ 2 * newRel0 + i ];
         sP[ i ] = Pu[ i ];
+    for ( int i = tid; i <= K; i += THREADS ) // record i: step i - 1's next sample is sample i
+    {
+        const int rel = newRel0 + ( i < K ? i : K - 1 );
+        const int W = a.sFirstRel + 2 * i;
+        sStep[ 4 * i ] = Yu[ 2 * rel ];
+        sStep[ 4 * i + 1 ] = Yu[ 2 * rel + 1 ];
+        sStep[ 4 * i + 2 ] = 1.f / ( a.wL * Zn[ rel ] + a.wG );
+        sStep[ 4 * i + 3 ] = 1.f / (float)( a.ramp && W < w2 ? W : w2 );
     }
-    for ( int i = tid; i < K; i += THREADS )
-        sInv[ i ] = 1.f / ( a.wL * Zn[ newRel0 + i ] + a.wG );
 
     const int kLast = newRel0 - 1; // newest sample before the block
     const int pLast = ( cMod + kLast + Wc ) % Wc;
-    int p = pLast + 1 < Wc ? pLast + 1 : 0; // slot of the sample entering at step k
-    const float invWfull = 1.f / (float)w2;
 
     if ( wave < NP )
     {
         // ================= product waves =================
         const int r = lane >> 4, pt = r & 1, v = wave * 16 + ( lane & 15 );
         const bool vOk = v < Wc;
-        WinPlane<TP> gA, gC, gB;
+        int p = pLast + 1 < Wc ? pLast + 1 : 0; // slot of the sample entering at step k
+        WinRegs<TP> g;
         float f, c, y, inv;
         {
             int dv = pLast - v;
@@ -216,18 +267,31 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             y = ex ? Yu[ 2 * rv + pt ] : 0.f;
             inv = ex ? 1.f / ( a.wL * Zn[ rv ] + a.wG ) : 0.f;
             const float* g0 = Gact + (int64_t)( ex ? v : 0 ) * IMG + r * PART;
+            constexpr int VL = TP % 4 == 0 ? 4 : TP % 2 == 0 ? 2 : 1; // floats per load
+            typedef float VecL __attribute__( ( ext_vector_type( VL ) ) );
 #pragma unroll
-            for ( int j = 0; j < TP; j++ )
+            for ( int j = 0; j < TP; j += VL )
             {
-                const int t = r * TP + j;
-                int dt = pLast - t;
-                dt += dt < 0 ? Wc : 0;
-                const bool ok = ex && t < Wc && kLast - dt >= 0;
-                const float xa = g0[ j ], xc = g0[ TPQ + j ], xb = g0[ 2 * TPQ + j ];
-                gA.put( j, ok ? xa : 0.f );
-                gC.put( j, ok ? xc : 0.f );
-                gB.put( j, ok ? xb : 0.f );
-                if ( ( j & 7 ) == 7 )
+                bool ok[ VL ];
+#pragma unroll
+                for ( int m = 0; m < VL; m++ )
+                {
+                    const int t = r * TP + j + m;
+                    int dt = pLast - t;
+                    dt += dt < 0 ? Wc : 0;
+                    ok[ m ] = ex && t < Wc && kLast - dt >= 0;
+                }
+#pragma unroll
+                for ( int pl = 0; pl < 3; pl++ )
+                {
+                    const VecL x = *reinterpret_cast<const VecL*>( g0 + pl * TPQ + j );
+#pragma unroll
+                    for ( int m = 0; m < VL; m++ )
+                    {
+                        g.put( pl, j + m, ok[ m ] ? x[ m ] : 0.f );
+                    }
+                }
+                if ( j % 8 >= 8 - VL )
                     __builtin_amdgcn_sched_barrier( 0 );
             }
             if ( lane < 32 )
@@ -236,150 +300,125 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
                 sCw[ 2 * v + pt ] = 0.f;
             }
         }
-        const int imgV = ( v / TP ) * PART + v % TP; // this u-slot's place in an image
+        const int imgV = vOk ? ( v / TP ) * PART + v % TP : 0; // this u-slot's place in an image
+        // where this lane's beta goes, and where it reads the ones of its row's t-slots
+        float* sBw = sB + 2 * ( v < 4 * TP ? ( v / TP ) * RUN + v % TP : 4 * RUN ) + pt;
+        const float* sBr = sB + 2 * r * RUN;
+        float* sCv = sCw + 2 * v + pt;
+        const int evAt = PKG + ( vOk ? 2 * v + pt : 0 );
         __syncthreads(); // packages 0 .. BUFS - 1 and the LDS arrays are in place
         __syncthreads(); // entering shares of steps 0 and 1
         auto loadColumn = [ & ]( const float* pk ) {
             const float* q = pk + r * PART;
-            if constexpr ( TP % 4 == 0 )
+#pragma unroll
+            for ( int pl = 0; pl < 3; pl++ )
             {
-                const float4* q4 = reinterpret_cast<const float4*>( q );
-#pragma unroll
-                for ( int j = 0; j < TP / 4; j++ )
+                if constexpr ( TP % 4 == 0 )
                 {
-                    const float4 xa = q4[ j ], xc = q4[ TPQ / 4 + j ], xb = q4[ TPQ / 2 + j ];
-                    const float va[ 4 ] = { xa.x, xa.y, xa.z, xa.w }, vc[ 4 ] = { xc.x, xc.y, xc.z, xc.w }, vb[ 4 ] = { xb.x, xb.y, xb.z, xb.w };
 #pragma unroll
-                    for ( int m = 0; m < 4; m++ )
+                    for ( int j = 0; j < TP / 4; j++ )
                     {
-                        gA.put( 4 * j + m, va[ m ] );
-                        gC.put( 4 * j + m, vc[ m ] );
-                        gB.put( 4 * j + m, vb[ m ] );
+                        const float4 x = reinterpret_cast<const float4*>( q + pl * TPQ )[ j ];
+                        g.put( pl, 4 * j, x.x );
+                        g.put( pl, 4 * j + 1, x.y );
+                        g.put( pl, 4 * j + 2, x.z );
+                        g.put( pl, 4 * j + 3, x.w );
                     }
-                }
-            }
-            else
-            {
-#pragma unroll
-                for ( int j = 0; j < TP; j++ )
-                {
-                    gA.put( j, q[ j ] );
-                    gC.put( j, q[ TPQ + j ] );
-                    gB.put( j, q[ 2 * TPQ + j ] );
-                }
-            }
-        };
-        // step 0's sample takes its u-slot over (later ones do so one step early)
-        if ( v == p )
-        {
-            f = 0.f;
-            c = 0.f;
-            y = sY[ pt ];
-            inv = sInv[ 0 ];
-            loadColumn( sPk );
-        }
-        float x = 0.f; // this row's product of the previous step
-        float evv = a.hasEv ? sPk[ PKG + ( vOk ? 2 * v + pt : 0 ) ] : 0.f;
-        float h = v == p ? sH[ pt ] + sH[ 2 + pt ] : 0.f;
-        float rA, rC, rB; // kappa(entering, v): what t-slot p gets
-        {
-            const bool self = v == p;
-            const int o = self ? IMG : ( vOk ? imgV : 0 ), st = self ? 1 : TPQ;
-            rA = sPk[ o ];
-            rC = sPk[ o + ( self ? 1 : 2 * TPQ ) ];
-            rB = sPk[ o + ( self ? 2 : st ) ];
-        }
-        float yn = K > 1 ? sY[ 2 + pt ] : 0.f, invn = K > 1 ? sInv[ 1 ] : 0.f;
-        int rp = p / TP, jp = p - rp * TP; // 16-lane row and register of t-slot p
-
-#pragma unroll 1
-        for ( int k = 0; k < K; k++ )
-        {
-            const bool more = k + 1 < K;
-            const int pn = p + 1 < Wc ? p + 1 : 0;
-            // ---- projection ----
-            if ( a.hasEv )
-                f -= evv;
-            f += x + h;
-            const float res = y - f;
-            const float bb = res - __builtin_amdgcn_fmed3f( res, -a.eB, a.eB );
-            float invW = invWfull;
-            if ( a.ramp )
-            {
-                const int W = a.sFirstRel + 2 * k;
-                invW = 1.f / (float)( W < w2 ? W : w2 );
-            }
-            const float beta = bb * invW * inv;
-            c += beta;
-            const bool leave = more && v == pn;
-            if ( lane < 32 )
-            {
-                sB[ ( k & 1 ) * SB + 2 * v + pt ] = beta;
-                sCw[ ( k & 1 ) * 2 * VS + 2 * v + pt ] = leave ? 0.f : c;
-                const int relOld = newRel0 + k + 1 - Wc; // sample leaving slot pn
-                if ( leave && relOld >= 0 )
-                    sC[ 2 * relOld + pt ] = c;
-            }
-            // ---- t-slot p: the sample that enters now ----
-            if ( r == rp && vOk )
-            {
-                // the active lanes share r, so jp is uniform: one indexed register write per plane
-                const int js = __builtin_amdgcn_readfirstlane( jp );
-                if ( TP <= 32 || js < 32 )
-                {
-                    gA.lo[ js ] = rA;
-                    gC.lo[ js ] = rC;
-                    gB.lo[ js ] = rB;
                 }
                 else
                 {
-                    gA.hi[ js - 32 ] = rA;
-                    gC.hi[ js - 32 ] = rC;
-                    gB.hi[ js - 32 ] = rB;
+#pragma unroll
+                    for ( int j = 0; j < TP; j++ )
+                        g.put( pl, j, q[ pl * TPQ + j ] );
                 }
             }
-            // ---- u-slot pn: the sample of the next step ----
-            const float* pkn = sPk + ( ( k + 1 ) % BUFS ) * PKCAP;
+        };
+        // The entering sample in its u-slot: its kappa with itself (what row insertion needs instead
+        // of the image, which there holds the leaving sample)
+        float selfA = 0.f, selfC = 0.f;
+        bool isP = v == p;
+        auto takeOver = [ & ]( const float* pk, float ny, float ninv ) {
+            f = 0.f;
+            c = 0.f;
+            y = ny;
+            inv = ninv;
+            selfA = pk[ IMG ];
+            selfC = pk[ IMG + 1 ]; // kappa(b,a) = kappa(a,b)
+            loadColumn( pk );
+        };
+        // step 0's sample takes its u-slot over (later ones do so one step early)
+        if ( isP )
+            takeOver( sPk, sStep[ pt ], sStep[ 2 ] );
+        // read one step ahead: eviction share, kappa(entering, v) for t-slot p, the entering shares,
+        // the weight 1 / W, and target and weight of the sample after it
+        float evv, rA, rC, rB, h[ NH ], yn, invn, iw;
+        const float* sRec = sStep; // record of the step read ahead
+        auto readAhead = [ & ]( const float* pk, int par ) {
+            evv = pk[ evAt ];
+            const float* q = pk + imgV;
+            rA = q[ 0 ];
+            rC = q[ 2 * TPQ ];
+            rB = q[ TPQ ];
+#pragma unroll
+            for ( int i = 0; i < NH; i++ )
+                h[ i ] = sH[ ( par * NH + i ) * 2 + pt ];
+            iw = sRec[ 3 ];
+            yn = sRec[ 4 + pt ];
+            invn = sRec[ 6 ];
+            sRec += 4;
+        };
+        readAhead( sPk, 0 );
+        float x = 0.f; // this row's product of the previous step
+        int rp = p / TP, jp = p - rp * TP; // 16-lane row and register of t-slot p
+        const int rSel = vOk ? r : -1;
+        int slot = 0; // k % BUFS
+        int relOld = newRel0 + 1 - Wc; // sample that leaves after step k's projection
+
+        auto step = [ & ]( auto half ) { // k & 1
+            const int pn = p + 1 < Wc ? p + 1 : 0;
+            slot = ( slot + 1 ) & ( BUFS - 1 );
+            const float* pkn = sPk + slot * PKCAP;
+            // ---- projection ----
+            float hs = h[ 0 ] + h[ 1 ];
+            if constexpr ( NH > 2 )
+                hs += h[ 2 ];
+            f -= a.hasEv ? evv : 0.f;
+            f += isP ? hs : 0.f;
+            f += x;
+            const float res = y - f;
+            const float bb = res - __builtin_amdgcn_fmed3f( res, -a.eB, a.eB );
+            const float beta = bb * ( iw * inv );
+            c += beta;
+            // (the two upper rows of a wave write what the two lower ones write)
+            sBw[ half * SB ] = beta;
+            sCv[ half * 2 * VS ] = c;
+            const bool leave = v == pn;
             if ( leave )
             {
-                f = 0.f;
-                c = 0.f;
-                y = yn;
-                inv = invn;
-                loadColumn( pkn );
+                sCv[ half * 2 * VS ] = 0.f;
+                if ( relOld >= 0 )
+                    sC[ 2 * relOld + pt ] = c;
             }
-            ldsBarrier();
+            relOld++;
+            // ---- t-slot p: the sample that enters now ----
+            g.insert( jp, rSel == rp, isP ? selfA : rA, isP ? selfC : rC, isP ? selfC : rB );
+            asm volatile( "s_waitcnt lgkmcnt(0)" ::: "memory" );
+            // ---- u-slot pn: the sample of the next step (the reads need not end before the barrier;
+            //      after the last step it takes a stale package, whose slot nothing reads) ----
+            if ( leave )
+                takeOver( pkn, yn, invn );
+            isP = leave;
+            asm volatile( "s_barrier" ::: "memory" );
             // ---- product, with the next step's reads in flight ----
-            float2 bt[ MB ];
-            const float2* sB2 = reinterpret_cast<const float2*>( sB + ( k & 1 ) * SB ) + r * TP + ( lane & 15 );
-#pragma unroll
-            for ( int m = 0; m < MB; m++ )
-                bt[ m ] = sB2[ 16 * m ];
-            h = 0.f;
-            if ( more )
-            {
-                if ( a.hasEv )
-                    evv = pkn[ PKG + ( vOk ? 2 * v + pt : 0 ) ];
-                const bool self = v == pn;
-                const int o = self ? IMG : ( vOk ? imgV : 0 );
-                rA = pkn[ o ];
-                rC = pkn[ o + ( self ? 1 : 2 * TPQ ) ];
-                rB = pkn[ o + ( self ? 2 : TPQ ) ];
-                if ( self )
-                    h = sH[ ( ( k + 1 ) & 1 ) * 4 + pt ] + sH[ ( ( k + 1 ) & 1 ) * 4 + 2 + pt ];
-                if ( k + 2 < K )
-                {
-                    yn = sY[ 2 * ( k + 2 ) + pt ];
-                    invn = sInv[ k + 2 ];
-                }
-            }
-            float a0 = 0.f, b0 = 0.f, a1 = 0.f, b1 = 0.f;
-            winProduct<TP, 0>( a0, b0, a1, b1, bt, gA, gC, gB );
+            float fa, fb;
+            winProduct<TP>( g, sBr + half * SB, fa, fb, [ & ] { readAhead( pkn, half ^ 1 ); } );
             // rows 0 and 2 of the wave take the a-part, rows 1 and 3 the b-part
-            const auto s1 = __builtin_amdgcn_permlane16_swap( __float_as_uint( a0 + a1 ), __float_as_uint( b0 + b1 ), false, false );
+            const auto s1 = __builtin_amdgcn_permlane16_swap( __float_as_uint( fa ), __float_as_uint( fb ), false, false );
             const float xh = __uint_as_float( s1[ 0 ] ) + __uint_as_float( s1[ 1 ] );
             const auto s2 = __builtin_amdgcn_permlane32_swap( __float_as_uint( xh ), __float_as_uint( xh ), false, false );
             x = __uint_as_float( s2[ 0 ] ) + __uint_as_float( s2[ 1 ] );
+            // (the reads ahead are not moved behind the product)
+            asm volatile( "" : "+v"( evv ), "+v"( rA ), "+v"( rC ), "+v"( rB ), "+v"( h[ 0 ] ), "+v"( h[ 1 ] ), "+v"( yn ), "+v"( invn ), "+v"( iw ) );
             p = pn;
             jp++;
             if ( jp == TP || p == 0 )
@@ -387,7 +426,19 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
                 jp = 0;
                 rp = p == 0 ? 0 : rp + 1;
             }
-        }
+        };
+        if constexpr ( TP == 40 ) // (unrolled by two, the loop does not fit the registers)
+#pragma unroll 1
+            for ( int k = 0; k < K; k++ )
+                step( k & 1 );
+        else
+#pragma unroll 1
+            for ( int k = 0; k < K; k += 2 )
+            {
+                step( std::integral_constant<int, 0> {} );
+                if ( k + 1 < K )
+                    step( std::integral_constant<int, 1> {} );
+            }
         f += x;
         if ( lane < 32 && vOk )
         {
@@ -395,97 +446,135 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             const int kEnd = newRel0 + K - 1;
             int dv = ( p > 0 ? p - 1 : Wc - 1 ) - v;
             dv += dv < 0 ? Wc : 0;
-            if ( kEnd - dv >= 0 )
+            if ( kEnd - dv >= 0 && !isP ) // (slot p has been taken over; its sample's c is in sC already)
                 sC[ 2 * ( kEnd - dv ) + pt ] = c;
         }
     }
     else
     {
         // ================= helper waves =================
-        const int role = wave - NP; // 0: packages (and left rows with two helpers), 1: window rows, 2: left rows
-        // share of the window rows and P in H_m, coefficients as after projection m - 2 (buffer cw)
+        // Interval k (after barrier k): the packages' wave issues package k + BUFS into the buffer step k
+        // released; the entering share H_{k+2} is summed.
+        // window rows and P in H_m, coefficients as after projection m - 2 (buffer cw)
+        int tOff[ ( 4 * TP + 63 ) / 64 ];
+#pragma unroll
+        for ( int i = 0; i < ( 4 * TP + 63 ) / 64; i++ )
+        {
+            const int t = i * 64 + lane < 4 * TP ? i * 64 + lane : 4 * TP - 1;
+            tOff[ i ] = ( t / TP ) * PART + t % TP;
+        }
         auto windowShare = [ & ]( int m, int cw ) {
-            const float* pk = sPk + ( m % BUFS ) * PKCAP;
+            const float* pk = sPk + ( m & ( BUFS - 1 ) ) * PKCAP;
             const float2* cs = reinterpret_cast<const float2*>( sCw + cw * 2 * VS );
             float ea = 0.f, eb = 0.f;
 #pragma unroll
             for ( int i = 0; i < ( 4 * TP + 63 ) / 64; i++ )
             {
-                const int t = i * 64 + lane;
-                if ( t < Wc )
-                {
-                    const float* g = pk + ( t / TP ) * PART + t % TP;
-                    const float2 cc = cs[ t ];
-                    const float A = g[ 0 ];
-                    ea += cc.x * A + cc.y * g[ TPQ ];
-                    eb += cc.x * g[ 2 * TPQ ] + cc.y * A;
-                }
+                const bool ok = i * 64 + lane < 4 * TP;
+                const float* q = pk + tOff[ i ];
+                const float2 cc = cs[ ok ? i * 64 + lane : 0 ];
+                const float A = q[ 0 ], Cq = q[ TPQ ], Bq = q[ 2 * TPQ ];
+                const float sa = cc.x * A + cc.y * Cq, sb = cc.x * Bq + cc.y * A;
+                ea += ok ? sa : 0.f;
+                eb += ok ? sb : 0.f;
             }
-            const float va = waveSum( ea ), vb = waveSum( eb );
-            if ( lane < 2 )
-                sH[ ( m & 1 ) * 4 + lane ] = ( lane == 0 ? va : vb ) + sP[ 2 * m + lane ];
+            const float pv = sP[ 2 * m + ( lane >> 5 ) ];
+            const float s = waveSumPair( ea, eb );
+            if ( ( lane & 31 ) == 0 )
+                sH[ ( m & 1 ) * NH * 2 + ( lane >> 5 ) ] = s + pv;
         };
-        // share of the active rows that have left the window by step m - 1
-        auto leftShare = [ & ]( int m ) {
-            const int older = winOlder( m, newRel0, Wc ), o4 = ( older + 3 ) & ~3;
-            const float* pk = sPk + ( m % BUFS ) * PKCAP + IMG + 4;
+        // the active rows that have left the window by step m - 1 (LEFT * 256 of them from `base` on);
+        // their kappa planes come from memory through a ring of register sets
+        constexpr int LEFT = kActMax / 256 / ( NH - 1 );
+        struct Left
+        {
+            wf32x4 A[ LEFT ], B[ LEFT ], C[ LEFT ];
+        };
+        auto leftLoad = [ & ]( int m, int base, Left& q ) {
+            const int mm = m < K ? m : K - 1;
+            const int o4 = ( winOlder( mm, newRel0, Wc ) + 3 ) & ~3;
+            const float* src = Gact + winRow( mm, newRel0, Wc, TP ) + IMG + 4;
+#pragma unroll
+            for ( int i = 0; i < LEFT; i++ )
+            {
+                const int jj = base + i * 256 + 4 * lane;
+                const int j = jj < o4 ? jj : 0; // (row 0: never past the buffer)
+                q.A[ i ] = *reinterpret_cast<const wf32x4*>( src + j );
+                q.B[ i ] = *reinterpret_cast<const wf32x4*>( src + o4 + j );
+                q.C[ i ] = *reinterpret_cast<const wf32x4*>( src + 2 * o4 + j );
+            }
+        };
+        auto leftShare = [ & ]( int m, int base, int src, const Left& q ) {
+            const int older = winOlder( m, newRel0, Wc );
             float ea = 0.f, eb = 0.f;
 #pragma unroll
-            for ( int i = 0; i < kActMax / 256; i++ )
+            for ( int i = 0; i < LEFT; i++ )
             {
-                const int j = i * 256 + 4 * lane;
-                if ( j < older )
+                const int j = base + i * 256 + 4 * lane;
+                const float4 c0 = *reinterpret_cast<const float4*>( sC + 2 * j ), c1 = *reinterpret_cast<const float4*>( sC + 2 * j + 4 );
+                const wf32x4 A = q.A[ i ], B = q.B[ i ], Cq = q.C[ i ];
+                float sa = c0.x * A[ 0 ] + c0.y * B[ 0 ] + c0.z * A[ 1 ] + c0.w * B[ 1 ];
+                float sb = c0.x * Cq[ 0 ] + c0.y * A[ 0 ] + c0.z * Cq[ 1 ] + c0.w * A[ 1 ];
+                sa += c1.x * A[ 2 ] + c1.y * B[ 2 ] + c1.z * A[ 3 ] + c1.w * B[ 3 ];
+                sb += c1.x * Cq[ 2 ] + c1.y * A[ 2 ] + c1.z * Cq[ 3 ] + c1.w * A[ 3 ];
+                ea += j < older ? sa : 0.f;
+                eb += j < older ? sb : 0.f;
+            }
+            const float s = waveSumPair( ea, eb );
+            if ( ( lane & 31 ) == 0 )
+                sH[ ( ( m & 1 ) * NH + src ) * 2 + ( lane >> 5 ) ] = s;
+        };
+        const int role = wave - NP; // 0: packages and window rows, others: left rows
+        if ( role > 0 )
+        {
+            const int base = ( role - 1 ) * 256;
+            Left ring[ RING ]; // set m % RING: step m
+            Left first;
+            leftLoad( 0, base, first );
+            leftLoad( 1, base, ring[ 1 % RING ] );
+#pragma unroll
+            for ( int m = 2; m < RING + 1; m++ )
+                leftLoad( m, base, m == RING ? ring[ 0 ] : ring[ m ] );
+            __syncthreads();
+            leftShare( 0, base, role, first );
+            if ( K > 1 )
+                leftShare( 1, base, role, ring[ 1 ] );
+            leftLoad( RING + 1, base, ring[ 1 ] );
+            __syncthreads();
+#pragma unroll 1
+            for ( int k0 = 0; k0 < K; k0 += RING )
+            {
+#pragma unroll
+                for ( int d = 0; d < RING; d++ )
                 {
-                    const float4 A = *reinterpret_cast<const float4*>( pk + j ), Bv = *reinterpret_cast<const float4*>( pk + o4 + j ),
-                                 Cv = *reinterpret_cast<const float4*>( pk + 2 * o4 + j );
-                    const float4 c0 = *reinterpret_cast<const float4*>( sC + 2 * j ), c1 = *reinterpret_cast<const float4*>( sC + 2 * j + 4 );
-                    ea += c0.x * A.x + c0.y * Bv.x + c0.z * A.y + c0.w * Bv.y;
-                    eb += c0.x * Cv.x + c0.y * A.x + c0.z * Cv.y + c0.w * A.y;
-                    ea += c1.x * A.z + c1.y * Bv.z + c1.z * A.w + c1.w * Bv.w;
-                    eb += c1.x * Cv.z + c1.y * A.z + c1.z * Cv.w + c1.w * A.w;
+                    const int k = k0 + d;
+                    if ( k >= K )
+                        break;
+                    ldsBarrier();
+                    if ( k + 2 < K )
+                        leftShare( k + 2, base, role, ring[ ( d + 2 ) % RING ] );
+                    leftLoad( k + 2 + RING, base, ring[ ( d + 2 ) % RING ] );
                 }
             }
-            const float va = waveSum( ea ), vb = waveSum( eb );
-            if ( lane < 2 )
-                sH[ ( m & 1 ) * 4 + 2 + lane ] = lane == 0 ? va : vb;
-        };
-        if ( role == 0 )
-            waitVm<0>();
-        __syncthreads();
-        for ( int m = 0; m < 2 && m < K; m++ )
-        {
-            if ( role == 1 )
-                windowShare( m, 1 );
-            if ( role == NH - 1 && ( NH == 3 || role != 1 ) )
-                leftShare( m );
-            if ( NH == 2 && role == 0 )
-                leftShare( m );
         }
-        __syncthreads();
-#pragma unroll 1
-        for ( int k = 0; k < K; k++ )
+        else
         {
-            ldsBarrier();
-            // interval k: package k + BUFS goes into the buffer that step k released; H_{k+2}
-            if ( role == 0 && k + BUFS < K )
-                pkIssue( k + BUFS );
-            if ( k + 2 < K )
+            waitVm<0>();
+            __syncthreads();
+            for ( int m = 0; m < 2 && m < K; m++ )
+                windowShare( m, 1 );
+            __syncthreads();
+#pragma unroll 1
+            for ( int k = 0; k < K; k++ )
             {
-                if ( role == 1 )
+                ldsBarrier();
+                pkIssue( k + BUFS, k & ( BUFS - 1 ) );
+                if ( k + 2 < K )
                     windowShare( k + 2, k & 1 );
-                if ( role == ( NH == 3 ? 2 : 0 ) )
-                    leftShare( k + 2 );
+                // package k + 3 is first read after the next barrier; the younger ones stay in flight
+                waitVm<NC*( BUFS - 3 )>();
             }
-            // package k + 3 is first read after the next barrier; the younger ones stay in flight
-            if ( role == 0 && k + 3 < K )
-            {
-                int young = 0;
-#pragma unroll
-                for ( int m = 4; m <= BUFS; m++ )
-                    if ( k + m < K )
-                        young += pkCopies( k + m );
-                waitVmUpTo31( young );
-            }
+            waitVm<0>(); // the buffers are reused below
         }
     }
     __syncthreads();

@@ -24,13 +24,17 @@ __host__ __device__ constexpr int winTpq( int tp ) { return ( tp + 1 ) & ~1; }
 __host__ __device__ constexpr int winPart( int tp ) { return ( 3 * winTpq( tp ) + 3 ) & ~3; }
 __host__ __device__ constexpr int winImg( int tp ) { return 4 * winPart( tp ); }
 __host__ __device__ constexpr int winProductWaves( int tp ) { return ( 4 * tp + 15 ) / 16; }
-// Helper waves: three while the workgroup then has at most 8 waves (256 registers per wave),
-// else two (12 waves at TP = 40: 168 registers, 120 of them the Gram).
-__host__ __device__ constexpr int winHelperWaves( int tp ) { return tp <= 20 ? 3 : 2; }
+// Helper waves: the packages with the window rows' share, and the left rows' share, 256 active samples
+// per wave while the workgroup then has at most 8 waves (12 waves at TP = 40: 168 registers per
+// wave, 120 of them the Gram).
+__host__ __device__ constexpr int winLeftWaves( int tp ) { return tp <= 20 ? kActMax / 256 : 1; }
+__host__ __device__ constexpr int winHelperWaves( int tp ) { return 1 + winLeftWaves( tp ); }
 __host__ __device__ constexpr int winThreads( int tp ) { return 64 * ( winProductWaves( tp ) + winHelperWaves( tp ) ); }
 // Package buffers: a package is issued BUFS - 2 steps before its first use, which has to cover the
-// memory latency; the short steps of the small windows need more of them.
-__host__ __device__ constexpr int winBufs( int tp ) { return tp <= 20 ? 6 : 4; }
+// memory latency (about 1.2 us, four steps of the small windows).
+constexpr int kWinBufs = 8;
+// Left rows' kappa: register sets in flight of the helper that reads them (one per step).
+__host__ __device__ constexpr int winRing( int tp ) { return tp <= 20 ? 4 : 2; }
 
 // Block Gram buffer: Wc images of the window's samples at the block start (both orders of every
 // pair), then one package row per entering sample e: its image over the window one step before it
@@ -62,17 +66,17 @@ inline int64_t winGactFloats( int Wc, int steps )
 // Row stride of the eviction shares [U][steps][stride], in slot order.
 __host__ __device__ inline int winEvStride( int w2 ) { return ( w2 + 3 ) & ~3; }
 
-// Floats of the Gram part of a package buffer: image, self, older planes (at most kActMax samples).
-__host__ __device__ constexpr int winPkGram( int tp ) { return ( winImg( tp ) + 4 + 3 * kActMax + 255 ) & ~255; }
+// Package buffer in LDS: the image with the self entries, then the eviction shares, both in whole
+// 256-float copies (the left rows' planes are not copied: their helper reads them from memory).
+__host__ __device__ constexpr int winPkGram( int tp ) { return ( winImg( tp ) + 4 + 255 ) & ~255; }
 __host__ __device__ constexpr int winPkCap( int tp ) { return winPkGram( tp ) + ( ( 8 * tp + 255 ) & ~255 ); }
-// Floats of one beta buffer: every slot a lane reads (3 TP + 16 ceil(TP / 16)) or writes.
-__host__ __device__ constexpr int winBetaFloats( int tp )
-{
-    return 2 * ( 3 * tp + 16 * ( ( tp + 15 ) / 16 ) > 16 * winProductWaves( tp ) ? 3 * tp + 16 * ( ( tp + 15 ) / 16 ) : 16 * winProductWaves( tp ) );
-}
+// Beta pairs by t-slot, each 16-lane row's run padded to 16 bytes and so that the four rows' reads
+// fall into different LDS banks; one more pair takes the writes of lanes without a t-slot.
+__host__ __device__ constexpr int winBetaRun( int tp ) { return ( ( tp + 1 ) & ~1 ) + ( ( ( tp + 1 ) & ~1 ) % 16 == 0 ? 2 : 0 ); }
+__host__ __device__ constexpr int winBetaFloats( int tp ) { return 8 * winBetaRun( tp ) + 4; }
 inline size_t winLdsBytes( int tp )
 {
-    return sizeof( float ) * ( (size_t)winBufs( tp ) * winPkCap( tp ) + 2 * winBetaFloats( tp ) + 2 * 32 * winProductWaves( tp ) + 2 * kActMax + 5 * kActMax + 8 );
+    return sizeof( float ) * ( (size_t)kWinBufs * winPkCap( tp ) + 2 * winBetaFloats( tp ) + 2 * 32 * winProductWaves( tp ) + 2 * kActMax + 6 * ( kActMax + 2 ) + 4 * ( 1 + winLeftWaves( tp ) ) );
 }
 
 } // namespace apsm
