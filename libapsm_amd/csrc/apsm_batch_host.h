@@ -530,7 +530,7 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
         const int grid = std::max( 1, std::min( nItems, B->cus * bb ) );
         const apsm::WorkItem* it = (const apsm::WorkItem*)( base + db.itemOff[ bc ] );
         detLaunches.push_back( [ = ]( hipStream_t st ) { launch( st, threads, shape, it, nItems, grid ); } );
-        B->tuning.push_back( { nmax, umax, threads, bb, nItems, kernel, kernel < 0 ? apsm::kDetTile : apsm::mfmaShapeEntries( shape, nmax ),
+        B->tuning.push_back( { nmax, umax, threads, bb, nItems, kernel, kernel < 0 ? apsm::kDetTile : apsm::mfmaShapeEntries( shape, nmax, kernel ),
                                kernel < 0 ? threads : apsm::mfmaShapeSamples( shape ) } );
     }
     // the buckets run side by side (their tails overlap instead of draining the GPU in turn)

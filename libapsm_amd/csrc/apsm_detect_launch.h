@@ -20,7 +20,7 @@ constexpr int kMfmaSamples = 128; // samples per workgroup tile
 
 // Tile shapes of the persistent batched matrix-core detect, chosen by the batch autotuner:
 // waves per workgroup (32 samples each) and dictionary entries per LDS tile (0: the single
-// handle's choice, 64, or 32 at 64 antennas). Shape 0 is the single-handle shape; the others
+// handle's choice, mfmaTileOf). Shape 0 is the single-handle shape; the others
 // are built for one-user FP32 instances up to 32 antennas (mfmaShapeBuilt).
 struct MfmaShape
 {
@@ -33,7 +33,10 @@ inline bool mfmaShapeBuilt( int shape, int prec, int nmax, int umax )
     return shape == 0 || ( shape > 0 && shape < kMfmaShapes && prec == PREC_F32 && nmax <= 32 && umax == 1 );
 }
 inline int mfmaShapeSamples( int shape ) { return 32 * kMfmaShape[ shape ].waves; }
-inline int mfmaShapeEntries( int shape, int nmax ) { return kMfmaShape[ shape ].entries ? kMfmaShape[ shape ].entries : ( nmax >= 64 ? 32 : 64 ); }
+// Dictionary entries per LDS tile of the single-handle shape: two 32-entry blocks, one where
+// rows of 64 antennas, or three-part rows of 32, would leave room for one workgroup only.
+__host__ __device__ constexpr int mfmaTileOf( int nmax, int prec ) { return nmax >= 64 || ( prec == PREC_F32 && nmax >= 32 ) ? 32 : 64; }
+inline int mfmaShapeEntries( int shape, int nmax, int prec ) { return kMfmaShape[ shape ].entries ? kMfmaShape[ shape ].entries : mfmaTileOf( nmax, prec ); }
 
 struct EntryArgs
 {

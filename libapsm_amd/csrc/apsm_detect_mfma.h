@@ -1,21 +1,44 @@
 // Detect with the cross terms on the matrix cores.
 //
 // For data samples x (columns) and dictionary entries z (rows) the two real cross terms are
-// the GEMMs  P^T = Zp X^T  and  S^T = Zs X^T  with K = 2*NMAX (zero padded):
-//   Zp row = [Re z | Im z],  Zs row = [Im z | -Re z],  X row = [Re x | Im x],
+// the GEMMs  P^T = Zp X^T  and  S^T = Zp Xs^T  with K = 2*NMAX (zero padded):
+//   Zp row = [Re z | Im z],  X row = [Re x | Im x],  Xs row = [-Im x | Re x],
 // so p = a_x.a_z and s = a_x.b_z. One wave computes a 32 entries x 32 samples block of each
-// with v_mfma_f32_32x32x2_f32 (PREC_F32) or v_mfma_f32_32x32x16_{bf16,f16} (inputs rounded
-// to 16 bits, FP32 accumulation). In the result layout lane l holds sample l % 32 and the 16
-// entries 8*(v/4) + 4*(l/32) + v%4 (v = 0..15), so the rest of the pair work stays in the
-// lane: squared distances from the FP32 norms |x|^2 + |z|^2 (the norm correction is FP32 for
-// every precision), three exponentials, and the contraction with every user's coefficients.
-// The two lane halves hold disjoint entries of the same sample and are added at the end.
+// with v_mfma_f32_32x32x16_{bf16,f16}, FP32 accumulation. In the result layout lane l holds
+// sample l % 32 and the 16 entries 8*(v/4) + 4*(l/32) + v%4 (v = 0..15), so the rest of the pair
+// work stays in the lane: squared distances from the FP32 norms |x|^2 + |z|^2 (the norm
+// correction is FP32 for every precision), three exponentials, and the contraction with every
+// user's coefficients. The two lane halves hold disjoint entries of the same sample and are added
+// at the end.
 //
-// Workgroup: 4 waves x 32 samples; the dictionary streams through LDS in tiles of 64 entries
-// (32 at 64 antennas).
+// PREC_BF16 and PREC_F16 round the inputs to 16 bits. PREC_F32 cuts every input into three bf16
+// parts, v = h + m + l (8 bits each: all 24 of an FP32 mantissa), and sums the six products above
+// 2^-24, hl, mm, lh, hm, mh, hh, smallest first: exact products, FP32 accumulation, so the error is
+// that of an FP32 dot product (the dropped ml, lm, ll are below 2^-25 of |x||z|). Six bf16 products
+// of 16 components take 192 cycles against 512 for v_mfma_f32_32x32x2_f32, and unlike those (which
+// share the vector ALU's multipliers) they run beside the vector ALU's exponentials.
+//
+// Workgroup: WAVES waves x 32 samples; the dictionary streams through LDS in tiles of ETILE entries.
+// The vector ALU's share per block of 32 x 32 pairs is 16 x (3 exponentials of 8.2 cycles, which take
+// the clamp at 1 for free, 4 + 4 U multiply-adds and adds of about 4 between them): 900 cycles for one
+// user, against 12 matrix instructions of 32 cycles up to 8 antennas, 24 at 16, 48 at 32. The next
+// block's products run between this one's exponentials, so what bounds a block is the power limit: with both units busy
+// the clock falls from 2.1 GHz to 1.6 to 1.75. Detect calls before (FP32 products on
+// v_mfma_f32_32x32x2_f32, one block's products and exponentials after each other) and now:
+//   8 antennas, 685 centres, 3840 samples              60 -> 33 us
+//   16 antennas, 10 users, 4096 centres, 500k samples  5.69 -> 3.75 ms
+//   32 antennas, 3690 centres, 49999 samples           678 -> 280 us
+//   64 antennas, 12 users, 16384 centres, 400k samples, bf16  16.1 -> 12.9 ms
+// or per block of 32 x 32 and SIMD, in cycles as if at 2.4 GHz: 1460 (8 antennas), 2070 (16), 3340 (32), 6880 (64).
+// Measured and not kept: two column blocks per wave sharing the coefficient reads (10 % faster at 4 users,
+// slower elsewhere, 64 antennas spilled); 8 waves per workgroup (within 2 %); staging loads without
+// the bounds branches (20 % slower); all products before all exponentials (as fast up to 16
+// antennas, 64 antennas bf16 8540 against 5810).
 #pragma once
 
 #include "apsm_detect_launch.h"
+
+#include <utility>
 
 namespace apsm {
 
@@ -41,270 +64,443 @@ struct MfmaIn<PREC_F16>
     static __device__ __forceinline__ mf32x16 mma( V a, V b, mf32x16 c ) { return __builtin_amdgcn_mfma_f32_32x32x16_f16( a, b, c, 0, 0, 0 ); }
 };
 
-// WAVES: waves per workgroup (32 samples each); ETILE: dictionary entries per LDS tile (0: 64,
-// or 32 at 64 antennas).
+template <>
+struct MfmaIn<PREC_F32> : MfmaIn<PREC_BF16> // three bf16 parts
+{
+};
+
+typedef float mf32x2 __attribute__( ( ext_vector_type( 2 ) ) );
+
+// Two values as packed 16-bit inputs of the matrix cores: NS = 1 rounds, NS = 3 gives h, m, l.
+template <int PREC, int NS>
+__device__ __forceinline__ void mfmaParts( float v0, float v1, uint32_t ( &out )[ NS ] )
+{
+    typedef typename MfmaIn<PREC>::T T2 __attribute__( ( ext_vector_type( 2 ) ) );
+    mf32x2 v = { v0, v1 };
+#pragma unroll
+    for ( int i = 0; i < NS; i++ )
+    {
+        const T2 q = __builtin_convertvector( v, T2 );
+        out[ i ] = __builtin_bit_cast( uint32_t, q );
+        if ( i + 1 < NS )
+            v -= __builtin_convertvector( q, mf32x2 );
+    }
+}
+
+// f( 0 ) ... f( N - 1 ) with the index as a constant expression
+template <class F, int... I>
+__device__ __forceinline__ void unrollSeq( F& f, std::integer_sequence<int, I...> )
+{
+    ( f( std::integral_constant<int, I> {} ), ... );
+}
+template <int N, class F>
+__device__ __forceinline__ void unrollFor( F f )
+{
+    unrollSeq( f, std::make_integer_sequence<int, N> {} );
+}
+
+// WAVES: waves per workgroup (32 samples each); ETILE: dictionary entries per LDS tile (0:
+// mfmaTileOf).
 template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0>
 __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
                                                 const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
                                                 const float* __restrict__ theta, int64_t G, int U, float wL, float wG, float g2,
                                                 float* __restrict__ est, int N, const int64_t tile )
 {
-    constexpr int K = 2 * NMAX;
-    constexpr int kMfmaTile = ETILE ? ETILE : ( NMAX >= 64 ? 32 : 64 ); // dictionary entries per LDS tile
-    constexpr int kMfmaThreads = 64 * WAVES; // (shadows the single-handle shape)
-    constexpr int kMfmaSamples = 32 * WAVES;
-    static_assert( kMfmaTile <= kMfmaThreads && kMfmaTile % 32 == 0, "one entry norm per thread, 32-entry MFMA blocks" );
-    // 16-bit inputs: K padded to a multiple of 16 (one MFMA step), rows padded by 8 elements
-    // (16 bytes) against LDS bank conflicts of the 16-byte reads
-    constexpr int K16 = K < 16 ? 16 : K;
-    constexpr int RowH = K16 + 8;
-    // Only Zp = [Re z | Im z] is staged; Zs = [Im z | -Re z] is the same row shifted by NMAX
-    // with the sign of its second half flipped. Two tile buffers: the next tile's loads are in
-    // flight (in registers) while the current tile is used, so a tile costs one barrier.
-    constexpr int kTileF = PREC == PREC_F32 ? K * kMfmaTile : 0; // f32: [K][tile] (transposed)
-    constexpr int kTileH = PREC == PREC_F32 ? 0 : kMfmaTile * RowH; // 16-bit: [tile][RowH]
-    constexpr int KL = PREC == PREC_F32 ? K : K16; // staged components per entry
-    constexpr int kLoads = ( KL * kMfmaTile + kMfmaThreads - 1 ) / kMfmaThreads; // per thread and tile
-    constexpr int kCLoads = ( UMAX * kMfmaTile + kMfmaThreads - 1 ) / kMfmaThreads;
-    __shared__ float sZf[ 2 ][ kTileF > 0 ? kTileF : 1 ];
-    __shared__ __attribute__( ( aligned( 16 ) ) ) uint16_t sZh[ 2 ][ kTileH > 0 ? kTileH : 1 ];
-    __shared__ float sZn[ 2 ][ kMfmaTile ];
-    __shared__ float2 sC[ 2 ][ UMAX * kMfmaTile ];
+    constexpr int K = 2 * NMAX, K16 = K < 16 ? 16 : K, T = K16 / 16; // components, padded; steps of 16
+    constexpr int NS = PREC == PREC_F32 ? 3 : 1;
+    constexpr int kTile = ETILE ? ETILE : mfmaTileOf( NMAX, PREC );
+    constexpr int kThreads = 64 * WAVES, kSamples = 32 * WAVES;
+    constexpr int RowH = K16 + 8; // rows padded by 16 bytes against LDS bank conflicts of the 16-byte reads
+    constexpr int kAllQuads = K16 / 4 * kTile, kQuads = ( kAllQuads + kThreads - 1 ) / kThreads; // groups of four components staged per thread
+    constexpr int kCLoads = ( UMAX * kTile + kThreads - 1 ) / kThreads;
+    static_assert( kTile <= kThreads && kTile % 32 == 0, "staging shape" );
+    typedef typename MfmaIn<PREC>::V V;
+    typedef uint32_t u32x4 __attribute__( ( ext_vector_type( 4 ) ) );
+    // two tile buffers: the next tile's loads are in flight (in registers) while the current tile
+    // is used, so a tile costs one barrier
+    __shared__ __attribute__( ( aligned( 16 ) ) ) uint16_t sZ[ 2 ][ NS ][ kTile * RowH ];
+    __shared__ __attribute__( ( aligned( 16 ) ) ) float sZn[ 3 ][ kTile ];
+    __shared__ __attribute__( ( aligned( 16 ) ) ) float2 sC[ 3 ][ kTile * UMAX ]; // [entry][user]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, h = lane >> 5;
-    const int64_t m = tile * kMfmaSamples + wave * 32 + col; // this lane's sample
+    const int64_t m = tile * kSamples + wave * 32 + col; // this lane's sample
     const bool valid = m < M;
     const int L = 2 * N;
 
-    // This lane's half of the sample in B-operand order: component k of X row = [Re x | Im x]
-    // with k = 2t + h (FP32 steps of 2) or k = 16t + 8h + i (16-bit steps of 16). The norm is
-    // summed in FP32 over both halves; the linear term reloads x at the end.
-    constexpr int NB = PREC == PREC_F32 ? K / 2 : K16 / 2;
-    typedef typename MfmaIn<PREC == PREC_F32 ? PREC_BF16 : PREC>::V VH; // 16-bit B operand (unused for FP32)
-    typedef typename MfmaIn<PREC == PREC_F32 ? PREC_BF16 : PREC>::T TH;
-    float xb[ PREC == PREC_F32 ? NB : 1 ];
-    VH xv[ PREC == PREC_F32 ? 1 : NB / 8 ]; // 16-bit inputs are packed right away (half the registers)
-    float xn = 0.f;
-#pragma unroll
-    for ( int j = 0; j < NB; j++ )
+    // This lane's half of the sample as B operands: step t holds components 16t + 8h + i of X and Xs.
+    // A component pair (re, im) of an antenna is one 8-byte load; with NMAX a multiple of 16 the Re
+    // half of X is the second half of Xs, and only the negated Im half is kept besides X. At 64
+    // antennas in three parts not even that fits the registers: the products with Im x go to an
+    // accumulator of their own and are subtracted.
+    constexpr bool HALVES = NMAX % 16 == 0, SUBTRACT = NMAX >= 64 && NS == 3;
+    constexpr int TX = SUBTRACT ? 1 : HALVES ? T / 2 : T; // steps of Xs with registers of their own
+    V xp[ T ][ NS ], xs[ TX ][ NS ];
+    float xq; // -g2 |x|^2
     {
-        const int k = PREC == PREC_F32 ? 2 * j + h : 16 * ( j / 8 ) + 8 * h + ( j % 8 );
-        const int ant = k < NMAX ? k : k - NMAX;
-        float v = 0.f;
-        if ( valid && k < K && ant < N )
-            v = rx[ ( (int64_t)ant * M + m ) * 2 + ( k < NMAX ? 0 : 1 ) ];
-        if constexpr ( PREC == PREC_F32 )
-            xb[ j ] = v;
+        float xn = 0.f;
+        const float2* r2 = reinterpret_cast<const float2*>( rx );
+        if constexpr ( HALVES )
+        {
+#pragma unroll
+            for ( int t = 0; t < T / 2; t++ )
+            {
+                u32x4 re[ NS ], im[ NS ];
+#pragma unroll
+                for ( int i = 0; i < 8; i += 2 )
+                {
+                    float2 v[ 2 ];
+#pragma unroll
+                    for ( int e = 0; e < 2; e++ )
+                    {
+                        const int ant = 16 * t + 8 * h + i + e;
+                        v[ e ] = valid && ant < N ? r2[ (int64_t)ant * M + m ] : make_float2( 0.f, 0.f );
+                        xn += v[ e ].x * v[ e ].x + v[ e ].y * v[ e ].y;
+                    }
+                    uint32_t pr[ NS ], pi[ NS ];
+                    mfmaParts<PREC, NS>( v[ 0 ].x, v[ 1 ].x, pr );
+                    mfmaParts<PREC, NS>( v[ 0 ].y, v[ 1 ].y, pi );
+#pragma unroll
+                    for ( int q = 0; q < NS; q++ )
+                    {
+                        re[ q ][ i / 2 ] = pr[ q ];
+                        im[ q ][ i / 2 ] = pi[ q ];
+                    }
+                }
+#pragma unroll
+                for ( int q = 0; q < NS; q++ )
+                {
+                    xp[ t ][ q ] = __builtin_bit_cast( V, re[ q ] );
+                    xp[ t + T / 2 ][ q ] = __builtin_bit_cast( V, im[ q ] );
+                    if constexpr ( !SUBTRACT )
+                        xs[ t ][ q ] = __builtin_bit_cast( V, im[ q ] ^ 0x80008000u );
+                }
+            }
+            xn += __shfl_xor( xn, 32 );
+        }
         else
-            xv[ j / 8 ][ j % 8 ] = (TH)v;
-        xn += v * v;
+        {
+            // NMAX 8: half h = 0 holds Re x, h = 1 Im x; NMAX 4: half 0 holds both, half 1 is padding
+            u32x4 p4[ NS ], s4[ NS ];
+#pragma unroll
+            for ( int i = 0; i < 8; i += 2 )
+            {
+                float vp[ 2 ], vs[ 2 ];
+#pragma unroll
+                for ( int e = 0; e < 2; e++ )
+                {
+                    const int ant = ( i + e ) % NMAX;
+                    const float2 v = valid && ant < N ? r2[ (int64_t)ant * M + m ] : make_float2( 0.f, 0.f );
+                    if ( NMAX == 8 || i < 4 )
+                        xn += v.x * v.x + v.y * v.y;
+                    const bool lo = NMAX == 8 ? h == 0 : i < 4; // component of Re x
+                    const float keep = NMAX == 8 || h == 0 ? 1.f : 0.f;
+                    vp[ e ] = keep * ( lo ? v.x : v.y );
+                    vs[ e ] = keep * ( lo ? -v.y : v.x );
+                }
+                uint32_t pp[ NS ], ps[ NS ];
+                mfmaParts<PREC, NS>( vp[ 0 ], vp[ 1 ], pp );
+                mfmaParts<PREC, NS>( vs[ 0 ], vs[ 1 ], ps );
+#pragma unroll
+                for ( int q = 0; q < NS; q++ )
+                {
+                    p4[ q ][ i / 2 ] = pp[ q ];
+                    s4[ q ][ i / 2 ] = ps[ q ];
+                }
+            }
+#pragma unroll
+            for ( int q = 0; q < NS; q++ )
+            {
+                xp[ 0 ][ q ] = __builtin_bit_cast( V, p4[ q ] );
+                xs[ 0 ][ q ] = __builtin_bit_cast( V, s4[ q ] );
+            }
+        }
+        xq = -g2 * xn;
     }
-    xn += __shfl_xor( xn, 32 );
-    // exponent arguments with the scale folded in: -g2 * (|x|^2 + |z|^2 - 2p) = q + k2 * p
-    const float xq = -g2 * xn, k2 = 2.f * g2;
+    // exponent arguments with the scale folded in: -g2 * (|x|^2 + |z|^2 - 2p) = q + k2 * p; the
+    // constants in vector registers (a scalar operand halves the multiply-add's rate)
+    float k2 = 2.f * g2, k2n = -2.f * g2;
+    asm( "" : "+v"( k2 ), "+v"( k2n ) );
 
     float fa[ UMAX ], fb[ UMAX ];
 #pragma unroll
     for ( int u = 0; u < UMAX; u++ )
         fa[ u ] = fb[ u ] = 0.f;
 
-    // tile loads into registers: element r of this thread is component k, entry e with
-    // r * kMfmaThreads + tid = (f32) k * tile + e, (16-bit) e * K16 + k (zeros past the
-    // dictionary end, past N and, 16-bit, past K)
-    float zreg[ kLoads ];
+    // tile loads into registers (zeros past the dictionary end, past N and past K): components k to k + 3
+    // of entry e, r * kThreads + tid = e * K16/4 + k/4. With N == NMAX rows have no gaps: one 16-byte load.
+    float4 zreg[ kQuads ];
     float zn;
     float2 creg[ kCLoads ];
-    auto loadTile = [ & ]( int64_t j0, int nt ) {
-#pragma unroll
-        for ( int r = 0; r < kLoads; r++ )
+    const bool whole = N == NMAX && K == K16 && ( reinterpret_cast<uintptr_t>( Z ) & 15 ) == 0;
+    auto loadTile = [ & ]( int tt ) {
+        const int64_t j0 = (int64_t)tt * kTile;
+        const int nt = ( G - j0 ) < kTile ? (int)( G - j0 ) : kTile;
+        if ( whole )
         {
-            const int i = r * kMfmaThreads + tid;
-            const int k = PREC == PREC_F32 ? i / kMfmaTile : i % K16;
-            const int e = PREC == PREC_F32 ? i % kMfmaTile : i / K16;
-            const int n = k < NMAX ? k : k - NMAX;
-            float v = 0.f;
-            if ( i < KL * kMfmaTile && e < nt && k < K && n < N )
-                v = Z[ ( j0 + e ) * L + ( k < NMAX ? n : N + n ) ];
-            zreg[ r ] = v;
+            const float4* Zt = reinterpret_cast<const float4*>( Z + j0 * L );
+#pragma unroll
+            for ( int r = 0; r < kQuads; r++ )
+            {
+                const int i = r * kThreads + tid;
+                zreg[ r ] = i / ( K16 / 4 ) < nt ? Zt[ i ] : make_float4( 0.f, 0.f, 0.f, 0.f );
+            }
+        }
+        else
+        {
+#pragma unroll
+            for ( int r = 0; r < kQuads; r++ )
+            {
+                const int i = r * kThreads + tid;
+                const int k = 4 * ( i % ( K16 / 4 ) ), e = i / ( K16 / 4 );
+                const int n = k < NMAX ? k : k - NMAX;
+                const float* z = Z + ( j0 + e ) * L + ( k < NMAX ? n : N + n );
+                const int have = e < nt && k < K ? N - n : 0;
+                zreg[ r ].x = have > 0 ? z[ 0 ] : 0.f;
+                zreg[ r ].y = have > 1 ? z[ 1 ] : 0.f;
+                zreg[ r ].z = have > 2 ? z[ 2 ] : 0.f;
+                zreg[ r ].w = have > 3 ? z[ 3 ] : 0.f;
+            }
         }
         zn = tid < nt ? -g2 * Zn[ j0 + tid ] : 0.f;
 #pragma unroll
         for ( int r = 0; r < kCLoads; r++ )
         {
-            const int i = r * kMfmaThreads + tid;
-            const int u = i / kMfmaTile, e = i % kMfmaTile;
-            creg[ r ] = ( i < UMAX * kMfmaTile && u < U && e < nt )
+            const int i = r * kThreads + tid;
+            const int u = i / kTile, e = i % kTile;
+            creg[ r ] = ( i < UMAX * kTile && u < U && e < nt )
                 ? make_float2( C[ u * ldC + 2 * ( j0 + e ) ], C[ u * ldC + 2 * ( j0 + e ) + 1 ] )
                 : make_float2( 0.f, 0.f );
         }
     };
-    auto storeTile = [ & ]( int buf ) {
+    auto storeTile = [ & ]( int tt ) {
+        const int buf = tt & 1, slot = tt % 3;
 #pragma unroll
-        for ( int r = 0; r < kLoads; r++ )
+        for ( int r = 0; r < kQuads; r++ )
         {
-            const int i = r * kMfmaThreads + tid;
-            if ( i < KL * kMfmaTile )
-            {
-                if constexpr ( PREC == PREC_F32 )
-                    sZf[ buf ][ i ] = zreg[ r ];
-                else
-                {
-                    typedef typename MfmaIn<PREC>::T T;
-                    sZh[ buf ][ ( i / K16 ) * RowH + i % K16 ] = __builtin_bit_cast( uint16_t, (T)zreg[ r ] );
-                }
-            }
+            const int i = r * kThreads + tid;
+            const int k = 4 * ( i % ( K16 / 4 ) ), e = i / ( K16 / 4 );
+            if ( kAllQuads % kThreads != 0 && i >= kAllQuads )
+                break;
+            uint32_t lo[ NS ], hi[ NS ];
+            mfmaParts<PREC, NS>( zreg[ r ].x, zreg[ r ].y, lo );
+            mfmaParts<PREC, NS>( zreg[ r ].z, zreg[ r ].w, hi );
+#pragma unroll
+            for ( int q = 0; q < NS; q++ )
+                *reinterpret_cast<uint2*>( &sZ[ buf ][ q ][ e * RowH + k ] ) = make_uint2( lo[ q ], hi[ q ] );
         }
-        if ( tid < kMfmaTile )
-            sZn[ buf ][ tid ] = zn;
+        if ( tid < kTile )
+            sZn[ slot ][ tid ] = zn;
 #pragma unroll
         for ( int r = 0; r < kCLoads; r++ )
         {
-            const int i = r * kMfmaThreads + tid;
-            if ( i < UMAX * kMfmaTile )
-                sC[ buf ][ i ] = creg[ r ];
+            const int i = r * kThreads + tid;
+            if ( i < UMAX * kTile )
+                sC[ slot ][ ( i % kTile ) * UMAX + i / kTile ] = creg[ r ];
         }
     };
 
-    const int nTiles = (int)( ( G + kMfmaTile - 1 ) / kMfmaTile );
+    // Products of one block, in order: group (lvl, t) is step t of the products of order 2^-16, 2^-8, 1
+    // (lvl 0, 1, 2; 16-bit modes have the last only), each for P and S.
+    constexpr int kLvls = NS == 3 ? 3 : 1, kGroups = kLvls * T;
+    constexpr int kProducts = ( NS == 3 ? 12 : 2 ) * T;
+    // The next block's products run under this one's exponentials, into a second set of accumulators
+    // (one set, and one after the other, where two do not fit the registers).
+    constexpr bool PIPE = !SUBTRACT;
+    mf32x16 accP[ PIPE ? 2 : 1 ], accS[ PIPE ? 2 : 1 ], accM;
+    V az[ 2 ][ NS ];
+    auto readGroup = [ & ]( int buf, int cb, auto gC ) {
+        constexpr int g = gC, lvl = g / T, t = g % T;
+#pragma unroll
+        for ( int q = 0; q < kLvls - lvl; q++ )
+            az[ g & 1 ][ q ] = *reinterpret_cast<const V*>( &sZ[ buf ][ q ][ ( cb + col ) * RowH + 16 * t + 8 * h ] );
+    };
+    auto product = [ & ]( int buf, int cb, auto dC, auto kC ) {
+        constexpr int d = dC, k = kC;
+        constexpr int lvl = NS != 3 || k < 6 * T ? 0 : k < 10 * T ? 1 : 2;
+        constexpr int per = NS == 3 ? 6 - 2 * lvl : 2, r = k - ( lvl == 0 ? 0 : lvl == 1 ? 6 * T : 10 * T );
+        constexpr int t = r / per, o = r % per / 2, g = lvl * T + t;
+        constexpr int pz = o, px = kLvls - 1 - lvl - o; // parts of z and x: their orders add up to the level's
+        constexpr int TH = T / 2 > 0 ? T / 2 : 1;
+        if constexpr ( r % per == 0 && g + 1 < kGroups )
+            readGroup( buf, cb, std::integral_constant<int, ( g + 1 < kGroups ? g + 1 : 0 )> {} );
+        const V a = az[ g & 1 ][ pz ];
+        const mf32x16 zero {};
+        if constexpr ( k % 2 == 0 )
+            accP[ d ] = MfmaIn<PREC>::mma( a, xp[ t ][ px ], k == 0 ? zero : accP[ d ] );
+        else if constexpr ( HALVES && t >= TH )
+            accS[ d ] = MfmaIn<PREC>::mma( a, xp[ t - TH ][ px ], SUBTRACT && lvl == 0 && t == TH && o == 0 ? zero : accS[ d ] );
+        else if constexpr ( SUBTRACT )
+            accM = MfmaIn<PREC>::mma( a, xp[ t + TH ][ px ], k == 1 ? zero : accM );
+        else
+            accS[ d ] = MfmaIn<PREC>::mma( a, xs[ t % TX ][ px ], k == 1 ? zero : accS[ d ] );
+        if constexpr ( SUBTRACT && k == kProducts - 1 )
+            accS[ d ] -= accM;
+    };
+    // Distances, exponentials and every user's contraction of the block in accumulators S (entries cb of
+    // coefficient slot `slot`), between them the products of the next block (entries cbn of buffer
+    // bufn) into the other set. The fences keep the two streams interleaved entry by entry.
+    constexpr int PF = UMAX <= 2 ? 4 : 1; // entries whose coefficients are read ahead together
+    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC ) {
+        constexpr int d = dC;
+        float2 co[ 2 ][ PF * UMAX ];
+        float4 zq[ 2 ];
+        auto entryOf = [ & ]( int i ) { return cb + 8 * ( i / 4 ) + 4 * h + i % 4; }; // the lane's entry i within the tile
+        auto readCo = [ & ]( auto iC ) {
+            constexpr int i = iC;
+            const float2* cc = &sC[ slot ][ entryOf( i ) * UMAX ];
+#pragma unroll
+            for ( int u = 0; u < PF * UMAX; u++ )
+                co[ i / PF & 1 ][ u ] = cc[ u ];
+        };
+        if constexpr ( PIPE )
+            readGroup( bufn, cbn, std::integral_constant<int, 0> {} );
+        zq[ 0 ] = *reinterpret_cast<const float4*>( &sZn[ slot ][ entryOf( 0 ) ] );
+        readCo( std::integral_constant<int, 0> {} );
+        unrollFor<16>( [ & ]( auto iC ) {
+            constexpr int i = iC;
+            if constexpr ( i % PF == 0 && i + PF < 16 )
+                readCo( std::integral_constant<int, ( i + PF ) % 16> {} );
+            if constexpr ( i % 4 == 0 && i + 4 < 16 )
+                zq[ ( i / 4 + 1 ) & 1 ] = *reinterpret_cast<const float4*>( &sZn[ slot ][ entryOf( i + 4 ) ] );
+            constexpr int k0 = i * kProducts / 16, k1 = ( i + 1 ) * kProducts / 16;
+            if constexpr ( PIPE )
+                unrollFor<k1 - k0>( [ & ]( auto kC ) { product( bufn, cbn, std::integral_constant<int, 1 - d> {}, std::integral_constant<int, k0 + kC> {} ); } );
+            const float4 z4 = zq[ i / 4 & 1 ];
+            const float q = xq + ( i % 4 == 0 ? z4.x : i % 4 == 1 ? z4.y : i % 4 == 2 ? z4.z : z4.w );
+            const float p = accP[ d ][ i ], s = accS[ d ][ i ];
+            // exponentials clamped to 1 (a rounded distance below zero counts as 0)
+            const float E0 = __builtin_amdgcn_fmed3f( __builtin_amdgcn_exp2f( fmaf( k2, p, q ) ), 0.f, 1.f );
+            const float E1 = __builtin_amdgcn_fmed3f( __builtin_amdgcn_exp2f( fmaf( k2, s, q ) ), 0.f, 1.f );
+            const float E2 = __builtin_amdgcn_fmed3f( __builtin_amdgcn_exp2f( fmaf( k2n, s, q ) ), 0.f, 1.f );
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
+            {
+                const float2 c = co[ i / PF & 1 ][ i % PF * UMAX + u ];
+                fa[ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ u ] ) );
+                fb[ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ u ] ) );
+                asm volatile( "" : "+v"( fa[ u ] ), "+v"( fb[ u ] )::"memory" );
+            }
+            __builtin_amdgcn_sched_barrier( 0 );
+        } );
+    };
+
+    // Tile tt + 1 is stored between two barriers' reach: its rows (two buffers) replace those of tile
+    // tt - 1, last read before the previous barrier, its norms and coefficients (three) those of tile
+    // tt - 2, as the last block of a tile is contracted after the barrier.
+    constexpr int kBlocks = kTile / 32;
+    typedef std::integral_constant<int, 0> D0;
+    typedef std::integral_constant<int, 1> D1;
+    const int nTiles = (int)( ( G + kTile - 1 ) / kTile );
     if ( nTiles > 0 )
     {
-        loadTile( 0, G < kMfmaTile ? (int)G : kMfmaTile );
+        loadTile( 0 );
         storeTile( 0 );
+        if ( nTiles > 1 )
+            loadTile( 1 );
     }
     __syncthreads();
-#pragma unroll 1
-    for ( int tt = 0; tt < nTiles; tt++ )
-    {
-        const int buf = tt & 1;
-        const int64_t j0 = (int64_t)tt * kMfmaTile;
-        const int nt = ( G - j0 ) < kMfmaTile ? (int)( G - j0 ) : kMfmaTile;
+    auto products = [ & ]( int buf, int cb ) {
+        readGroup( buf, cb, D0 {} );
+        unrollFor<kProducts>( [ & ]( auto kC ) { product( buf, cb, D0 {}, kC ); } );
+    };
+    if ( PIPE && nTiles > 0 )
+        products( 0, 0 );
+    auto advance = [ & ]( int tt ) {
         if ( tt + 1 < nTiles )
-        {
-            const int64_t jn = j0 + kMfmaTile;
-            loadTile( jn, ( G - jn ) < kMfmaTile ? (int)( G - jn ) : kMfmaTile );
-        }
-        const float* zf = sZf[ buf ];
-        const uint16_t* zh = sZh[ buf ];
-        const float* zq = sZn[ buf ];
-        const float2* cc = sC[ buf ];
-
-#pragma unroll 1
-        for ( int cb = 0; cb < nt; cb += 32 )
-        {
-            mf32x16 accP = {}, accS = {};
-            if constexpr ( PREC == PREC_F32 )
-            {
-#pragma unroll
-                for ( int t = 0; t < K / 2; t++ )
-                {
-                    const int k = 2 * t + h;
-                    const float ap = zf[ k * kMfmaTile + cb + col ];
-                    // Zs component k: Im z_k (k < NMAX) or -Re z_(k-NMAX); k < NMAX for t < NMAX/2
-                    const float as = t < NMAX / 2 ? zf[ ( k + NMAX ) * kMfmaTile + cb + col ] : -zf[ ( k - NMAX ) * kMfmaTile + cb + col ];
-                    accP = __builtin_amdgcn_mfma_f32_32x32x2f32( ap, xb[ t ], accP, 0, 0, 0 );
-                    accS = __builtin_amdgcn_mfma_f32_32x32x2f32( as, xb[ t ], accS, 0, 0, 0 );
-                    if ( ( t & 7 ) == 7 )
-                        __builtin_amdgcn_sched_barrier( 0 ); // bound the operand loads in flight (registers)
-                }
-            }
-            else
-            {
-                typedef typename MfmaIn<PREC>::V V;
-                typedef unsigned int u32x4 __attribute__( ( ext_vector_type( 4 ) ) );
-#pragma unroll
-                for ( int t = 0; t < K16 / 16; t++ )
-                {
-                    const int k0 = 16 * t + 8 * h;
-                    const V b = xv[ t ];
-                    const uint16_t* row = zh + ( cb + col ) * RowH;
-                    const V ap = *reinterpret_cast<const V*>( row + k0 );
-                    // Zs: the row shifted by NMAX, second half negated (components past K meet
-                    // zeros of x, so whatever the shifted read holds there does not count)
-                    u32x4 bits;
-                    if constexpr ( NMAX % 8 == 0 )
-                    {
-                        // the lane's 8 components lie in one half: k0 < NMAX gives Im z, else -Re z
-                        const bool lowHalf = k0 < NMAX;
-                        bits = *reinterpret_cast<const u32x4*>( row + ( lowHalf ? k0 + NMAX : k0 - NMAX ) ); // 16-byte aligned
-                        bits ^= lowHalf ? 0u : 0x80008000u;
-                    }
-                    else
-                    {
-                        // NMAX = 4: components 0..3 are Im z (row + 4), 4..7 are -Re z (row + 0);
-                        // the lane with k0 = 8 is past K
-                        typedef unsigned int u32x2 __attribute__( ( ext_vector_type( 2 ) ) );
-                        const u32x2 lo = *reinterpret_cast<const u32x2*>( row + k0 + 4 );
-                        const u32x2 hi = *reinterpret_cast<const u32x2*>( row + k0 ) ^ 0x80008000u;
-                        bits = u32x4 { lo.x, lo.y, hi.x, hi.y };
-                    }
-                    const V as = __builtin_bit_cast( V, bits );
-                    accP = MfmaIn<PREC>::mma( ap, b, accP );
-                    accS = MfmaIn<PREC>::mma( as, b, accS );
-                    if ( ( t & 1 ) == 1 )
-                        __builtin_amdgcn_sched_barrier( 0 );
-                }
-            }
-#pragma unroll
-            for ( int v = 0; v < 16; v++ )
-            {
-                const int e = cb + 8 * ( v / 4 ) + 4 * h + ( v % 4 ); // entry within the tile
-                const float q = xq + zq[ e ];
-                const float p = accP[ v ], s = accS[ v ];
-                // exp2 of a clamped non-positive argument (a rounded distance below zero counts as 0)
-                const float E0 = __builtin_amdgcn_exp2f( fminf( fmaf( k2, p, q ), 0.f ) );
-                const float E1 = __builtin_amdgcn_exp2f( fminf( fmaf( k2, s, q ), 0.f ) );
-                const float E2 = __builtin_amdgcn_exp2f( fminf( fmaf( -k2, s, q ), 0.f ) );
-#pragma unroll
-                for ( int u = 0; u < UMAX; u++ )
-                {
-                    const float2 c = cc[ u * kMfmaTile + e ];
-                    fa[ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ u ] ) );
-                    fb[ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ u ] ) );
-                }
-                // bound the coefficient loads in flight; measured: helps up to 32 antennas, at 64 the
-                // scheduler then serialises the loads ahead of the math and spills
-                if ( NMAX <= 32 )
-                    __builtin_amdgcn_sched_barrier( 0 );
-            }
-        }
-        if ( tt + 1 < nTiles )
-            storeTile( buf ^ 1 ); // the other buffer was released by the previous iteration's barrier
+            storeTile( tt + 1 );
+        if ( tt + 2 < nTiles )
+            loadTile( tt + 2 );
         __syncthreads();
+    };
+    // (the products past the last block read what the buffers hold, and are not used)
+    if constexpr ( !PIPE )
+    {
+#pragma unroll 1
+        for ( int tt = 0; tt < nTiles; tt++ )
+        {
+#pragma unroll 1
+            for ( int cb = 0; cb < kTile; cb += 32 )
+            {
+                products( tt & 1, cb );
+                phase( tt % 3, cb, 0, 0, D0 {} );
+            }
+            advance( tt );
+        }
     }
+    else if constexpr ( kBlocks == 1 )
+    {
+#pragma unroll 1
+        for ( int tt = 0; tt < nTiles; tt += 2 )
+        {
+            advance( tt );
+            phase( tt % 3, 0, ( tt + 1 ) & 1, 0, D0 {} );
+            if ( tt + 1 < nTiles )
+            {
+                advance( tt + 1 );
+                phase( ( tt + 1 ) % 3, 0, tt & 1, 0, D1 {} );
+            }
+        }
+    }
+    else
+    {
+#pragma unroll 1
+        for ( int tt = 0; tt < nTiles; tt++ )
+        {
+#pragma unroll
+            for ( int b = 0; b + 2 < kBlocks; b += 2 )
+            {
+                phase( tt % 3, 32 * b, tt & 1, 32 * b + 32, D0 {} );
+                phase( tt % 3, 32 * b + 32, tt & 1, 32 * b + 64, D1 {} );
+            }
+            phase( tt % 3, kTile - 64, tt & 1, kTile - 32, D0 {} );
+            advance( tt );
+            phase( tt % 3, kTile - 32, ( tt + 1 ) & 1, 0, D1 {} );
+        }
+    }
+    __syncthreads(); // a following tile stores over what other waves may still read
 
-    // the two lane halves saw disjoint entries of the same sample
+    // the two lane halves saw disjoint entries of the same sample; f = wL theta . x + wG (Gaussian
+    // part), x read again
 #pragma unroll
     for ( int u = 0; u < UMAX; u++ )
     {
         fa[ u ] += __shfl_xor( fa[ u ], 32 );
         fb[ u ] += __shfl_xor( fb[ u ], 32 );
     }
-    if ( !valid || h != 0 )
-        return;
-#pragma unroll
-    for ( int u = 0; u < UMAX; u++ )
+    if ( valid && h == 0 )
     {
-        if ( u < U )
+        float la[ UMAX ], lb[ UMAX ];
+#pragma unroll
+        for ( int u = 0; u < UMAX; u++ )
+            la[ u ] = lb[ u ] = 0.f;
+#pragma unroll 4
+        for ( int n = 0; n < N; n++ )
         {
-            const float* th = theta + u * L;
-            float la = 0.f, lb = 0.f;
-            for ( int n = 0; n < N; n++ )
+            const float2 x = reinterpret_cast<const float2*>( rx )[ (int64_t)n * M + m ];
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
             {
-                const float2 x = reinterpret_cast<const float2*>( rx )[ (int64_t)n * M + m ];
-                la += th[ n ] * x.x + th[ N + n ] * x.y;
-                lb += th[ n ] * x.y - th[ N + n ] * x.x;
+                const float* th = theta + ( u < U ? u : 0 ) * L;
+                la[ u ] += fmaf( th[ n ], x.x, th[ N + n ] * x.y );
+                lb[ u ] += fmaf( th[ n ], x.y, -th[ N + n ] * x.x );
             }
-            reinterpret_cast<float2*>( est )[ (int64_t)u * M + m ] = make_float2( wL * la + wG * fa[ u ], wL * lb + wG * fb[ u ] );
         }
+#pragma unroll
+        for ( int u = 0; u < UMAX; u++ )
+            if ( u < U )
+                reinterpret_cast<float2*>( est )[ (int64_t)u * M + m ] = make_float2( wL * la[ u ] + wG * fa[ u ], wL * lb[ u ] + wG * fb[ u ] );
     }
 }
 
+// Two workgroups of four waves per CU at least: 256 registers per wave, which also keeps the matrix
+// results in vector registers (the compiler moves them through accumulation registers otherwise).
 template <int NMAX, int UMAX, int PREC>
-__global__ void __launch_bounds__( kMfmaThreads ) apsm_detect_mfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
-                                                                   const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
-                                                                   const float* __restrict__ theta, int64_t G, int U, float wL, float wG,
-                                                                   float g2, float* __restrict__ est, int N )
+__global__ void __launch_bounds__( kMfmaThreads, 2 ) apsm_detect_mfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
+                                                                      const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
+                                                                      const float* __restrict__ theta, int64_t G, int U, float wL, float wG,
+                                                                      float g2, float* __restrict__ est, int N )
 {
     detectTileMfma<NMAX, UMAX, PREC>( rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, blockIdx.x );
 }
@@ -312,7 +508,7 @@ __global__ void __launch_bounds__( kMfmaThreads ) apsm_detect_mfma( const float*
 // Persistent batched detect over a work list (all items of one launch share NMAX and UMAX),
 // workgroups of WAVES waves, tiles of 32 * WAVES samples.
 template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0>
-__global__ void __launch_bounds__( 64 * WAVES ) batch_detect_mfma( const DetDesc* __restrict__ d, const WorkItem* __restrict__ items,
+__global__ void __launch_bounds__( 64 * WAVES, WAVES <= 4 ? 8 / WAVES : 1 ) batch_detect_mfma( const DetDesc* __restrict__ d, const WorkItem* __restrict__ items,
                                                                    int nItems )
 {
     for ( int w = blockIdx.x; w < nItems; w += gridDim.x )
@@ -330,9 +526,8 @@ template <int PREC, int NMAX, int UMAX>
 hipError_t launchMfmaNU( hipStream_t s, const float* rx, int64_t M, const float* Z, const float* Zn, const float* C, int64_t ldC,
                          const float* theta, int64_t G, int U, float wL, float wG, float g2, float* est, int N )
 {
-    const int64_t grid = ( M + kMfmaSamples - 1 ) / kMfmaSamples;
-    hipLaunchKernelGGL( ( apsm_detect_mfma<NMAX, UMAX, PREC> ), dim3( (unsigned)grid ), dim3( kMfmaThreads ), 0, s, rx, M, Z, Zn, C, ldC,
-                        theta, G, U, wL, wG, g2, est, N );
+    hipLaunchKernelGGL( ( apsm_detect_mfma<NMAX, UMAX, PREC> ), dim3( (unsigned)( ( M + kMfmaSamples - 1 ) / kMfmaSamples ) ),
+                        dim3( kMfmaThreads ), 0, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N );
     return hipGetLastError();
 }
 
