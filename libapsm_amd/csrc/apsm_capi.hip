@@ -6,6 +6,7 @@
 
 #include "apsm_capi.h"
 #include "apsm_device.h"
+#include "apsm_lls.h"
 #include "apsm_train2.h"
 #include "apsm_train_win.h"
 #include "apsm_train_nc.h"
@@ -168,7 +169,7 @@ struct lls_handle
     bool ownStream = true; // false when the caller lent its stream (lls_create_on_stream)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     DevBuf<float> w, part, rx, tx, est;
-    DevBuf<double> gram, sums;
+    DevBuf<double> gram, pairs, sums;
     DevBuf<int> status;
     int nW = 0; // unknowns of the last solve (2N for the embedding, num_input_dims for the low-level call)
     bool trained = false;
@@ -176,37 +177,52 @@ struct lls_handle
 
 namespace {
 
-// FP64 sum of the nPart partial normal equations of n unknowns, then the FP64 Cholesky solve
-// into h->w (first n entries) and h->status.
-void llsReduceSolve( lls_handle* h, int nPart, int n )
+template <int NB>
+void launchLlsSolveNB( const double* gram, int n, float* w, int* status, hipStream_t st )
+{
+    const size_t lds = apsm::llsSolveLds( n );
+    if ( lds > 64 * 1024 )
+        HIP_OR_THROW( hipFuncSetAttribute( (const void*)apsm::lls_solve<NB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds ) );
+    hipLaunchKernelGGL( apsm::lls_solve<NB>, dim3( 1 ), dim3( apsm::kSolveThreads ), lds, st, gram, n, w, status );
+    HIP_OR_THROW( hipGetLastError() );
+}
+
+void launchLlsSolve( const double* gram, int n, float* w, int* status, hipStream_t st )
+{
+    switch ( apsm::llsSolveBlocks( n ) )
+    {
+    case 1: return launchLlsSolveNB<1>( gram, n, w, status, st );
+    case 2: return launchLlsSolveNB<2>( gram, n, w, status, st );
+    case 4: return launchLlsSolveNB<4>( gram, n, w, status, st );
+    default: return launchLlsSolveNB<8>( gram, n, w, status, st );
+    }
+}
+
+// FP64 sum of nPart FP32 partial normal equations of n unknowns, then the FP64 solve.
+void launchLlsReduceSolve( const float* part, int nPart, int n, double* gram, float* w, int* status, hipStream_t st )
 {
     const int E = n * ( n + 1 );
-    h->nW = n;
-    h->gram.ensure( (size_t)E );
-    hipLaunchKernelGGL( apsm::lls_reduce_partials, dim3( gridFor( E, 256 ) ), dim3( 256 ), 0, h->stream, h->part.ptr, nPart, E,
-                        h->gram.ptr );
+    hipLaunchKernelGGL( apsm::lls_reduce_partials, dim3( gridFor( E, 64 ) ), dim3( apsm::kLlsSumThreads ), 0, st, part, nPart, E, gram );
     HIP_OR_THROW( hipGetLastError() );
-    const size_t ldsSolve = (size_t)E * sizeof( double );
-    if ( ldsSolve > 64 * 1024 )
-        HIP_OR_THROW( hipFuncSetAttribute( (const void*)apsm::lls_solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsSolve ) );
-    hipLaunchKernelGGL( apsm::lls_solve, dim3( 1 ), dim3( apsm::kSolveThreads ), ldsSolve, h->stream, h->gram.ptr, n, h->w.ptr,
-                        h->status.ptr );
-    HIP_OR_THROW( hipGetLastError() );
+    launchLlsSolve( gram, n, w, status, st );
 }
 
 void llsTrainDev( lls_handle* h, const float* d_rx, const float* d_tx, int64_t T )
 {
     ARG_CHECK( T > 0, "LLS train needs at least one pilot" );
-    const int L = h->L;
-    const int E = L * ( L + 1 );
-    const int64_t chunk = std::max<int64_t>( 1, (int64_t)( apsm::kLlsLdsBudget / ( 2 * ( L + 1 ) * sizeof( float ) ) ) );
-    const int nPart = (int)( ( T + chunk - 1 ) / chunk );
-    h->part.ensure( (size_t)nPart * E );
-    const size_t lds = 2 * (size_t)chunk * ( L + 1 ) * sizeof( float );
-    hipLaunchKernelGGL( apsm::lls_normal_partial, dim3( nPart ), dim3( apsm::kLlsThreads ), lds, h->stream, d_rx, d_tx, h->N,
-                        T, chunk, h->part.ptr );
+    const int L = h->L, tasks = apsm::llsTasks( h->N );
+    const int64_t share = apsm::llsShare( T );
+    const int nPart = (int)( ( T + share - 1 ) / share );
+    h->pairs.ensure( (size_t)nPart * tasks * apsm::kLlsPairEntries );
+    h->gram.ensure( (size_t)L * ( L + 1 ) );
+    h->nW = L;
+    hipLaunchKernelGGL( apsm::lls_normal_pairs, dim3( nPart, tasks ), dim3( apsm::kLlsPairThreads ), 0, h->stream, d_rx, d_tx, h->N, T,
+                        share, h->pairs.ptr );
     HIP_OR_THROW( hipGetLastError() );
-    llsReduceSolve( h, nPart, L );
+    hipLaunchKernelGGL( apsm::lls_reduce_pairs, dim3( tasks, apsm::kLlsPairEntries / 64 ), dim3( apsm::kLlsSumThreads ), 0, h->stream,
+                        h->pairs.ptr, nPart, h->N, h->gram.ptr );
+    HIP_OR_THROW( hipGetLastError() );
+    launchLlsSolve( h->gram.ptr, L, h->w.ptr, h->status.ptr, h->stream );
 }
 
 // General column-major A (m x n, ld m), target y (m): trainLowLevel's operands.
@@ -224,7 +240,9 @@ void llsTrainColMajor( lls_handle* h, const float* d_A, const float* d_y, int n,
     hipLaunchKernelGGL( apsm::lls_normal_colmajor, dim3( nPart ), dim3( apsm::kLlsThreads ), lds, h->stream, d_A, d_y, n, m, chunk,
                         h->part.ptr );
     HIP_OR_THROW( hipGetLastError() );
-    llsReduceSolve( h, nPart, n );
+    h->gram.ensure( (size_t)E );
+    h->nW = n;
+    launchLlsReduceSolve( h->part.ptr, nPart, n, h->gram.ptr, h->w.ptr, h->status.ptr, h->stream );
 }
 
 // ---- least squares without allocation (lls_train_lowlevel_noalloc) ----
@@ -1666,14 +1684,7 @@ int lls_train_lowlevel_noalloc( const float* d_A, const float* d_y, int32_t num_
         hipLaunchKernelGGL( apsm::lls_normal_colmajor, dim3( sp.nPart ), dim3( apsm::kLlsThreads ),
                             (size_t)sp.chunk * ( n + 1 ) * sizeof( float ), st, d_A, d_y, n, m, sp.chunk, part );
         HIP_OR_THROW( hipGetLastError() );
-        hipLaunchKernelGGL( apsm::lls_reduce_partials, dim3( gridFor( sp.E, 256 ) ), dim3( 256 ), 0, st, part, sp.nPart, sp.E, gram );
-        HIP_OR_THROW( hipGetLastError() );
-        const size_t ldsSolve = (size_t)sp.E * sizeof( double );
-        if ( ldsSolve > 64 * 1024 )
-            HIP_OR_THROW(
-                hipFuncSetAttribute( (const void*)apsm::lls_solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsSolve ) );
-        hipLaunchKernelGGL( apsm::lls_solve, dim3( 1 ), dim3( apsm::kSolveThreads ), ldsSolve, st, gram, n, d_w, d_status );
-        HIP_OR_THROW( hipGetLastError() );
+        launchLlsReduceSolve( part, sp.nPart, n, gram, d_w, d_status, st );
     } );
 }
 

@@ -500,140 +500,12 @@ __global__ void __launch_bounds__( kDetThreads ) apsm_detect_kernel( const float
 }
 
 // ---------------------------------------------------------------------------------------
-// LLS (cpp/lib/noma/lls_detector.cu:136-218): min_w |A w - y| over the real embedding.
-// Normal equations A^T A w = A^T y: per-workgroup FP32 partial sums over a contiguous
-// chunk of samples, then one workgroup adds the partials in FP64 and solves by Cholesky
-// in FP64.
+// Low-level LLS (cpp/lib/noma/lls_detector.cu:136-218): normal equations A^T A w = A^T y of a general
+// real matrix as per-workgroup FP32 partial sums over a contiguous chunk of rows; apsm_lls.h adds
+// them in FP64 and solves.
 // ---------------------------------------------------------------------------------------
 constexpr int kLlsThreads = 256;
 constexpr size_t kLlsLdsBudget = 64 * 1024; // bytes of LDS per workgroup for one chunk of samples
-
-// part[b][i*(L+1) + j] for j < L: sum a_i a_j + b_i b_j; j == L: sum a_i y_re + b_i y_im,
-// over samples [b*chunk, (b+1)*chunk). The whole chunk sits in LDS; each thread owns
-// entries e = tid + o*256 and accumulates one at a time over the chunk.
-__global__ void __launch_bounds__( kLlsThreads ) lls_normal_partial( const float* __restrict__ rx, const float* __restrict__ tx,
-                                                                   int N, int64_t T, int64_t chunk, float* __restrict__ part )
-{
-    const int L = 2 * N;
-    const int ld = L + 1;
-    const int E = L * ld;
-    extern __shared__ float sA[]; // [chunk][L+1] rows a (+ y_re), then [chunk][L+1] rows b (+ y_im)
-    const int64_t k0 = (int64_t)blockIdx.x * chunk;
-    const int nt = (int)( ( k0 + chunk ) < T ? chunk : T - k0 );
-    float* sBr = sA + (int64_t)chunk * ld;
-    for ( int i = threadIdx.x; i < nt * N; i += kLlsThreads )
-    {
-        const int n = i / nt, t = i % nt; // consecutive threads read consecutive samples
-        float2 v = reinterpret_cast<const float2*>( rx )[ (int64_t)n * T + k0 + t ];
-        sA[ t * ld + n ] = v.x;
-        sA[ t * ld + N + n ] = v.y;
-        sBr[ t * ld + n ] = v.y;
-        sBr[ t * ld + N + n ] = -v.x;
-    }
-    for ( int t = threadIdx.x; t < nt; t += kLlsThreads )
-    {
-        float2 y = reinterpret_cast<const float2*>( tx )[ k0 + t ];
-        sA[ t * ld + L ] = y.x;
-        sBr[ t * ld + L ] = y.y;
-    }
-    __syncthreads();
-    for ( int e = threadIdx.x; e < E; e += kLlsThreads )
-    {
-        const int i = e / ld, j = e % ld;
-        float s = 0.f;
-        for ( int t = 0; t < nt; t++ )
-            s += sA[ t * ld + i ] * sA[ t * ld + j ] + sBr[ t * ld + i ] * sBr[ t * ld + j ];
-        part[ (int64_t)blockIdx.x * E + e ] = s;
-    }
-}
-
-// G[e] = sum over partials in FP64.
-__global__ void lls_reduce_partials( const float* __restrict__ part, int nPart, int E, double* __restrict__ G )
-{
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( e >= E )
-        return;
-    double s = 0.0;
-    for ( int b = 0; b < nPart; b++ )
-        s += (double)part[ (int64_t)b * E + e ];
-    G[ e ] = s;
-}
-
-// Cholesky-factor the normal matrix G = R R^T in FP64 (LDS-resident, L <= 128), solve
-// R R^T w = r, write w (FP32) and the status (0 ok, -1 not positive definite).
-constexpr int kSolveThreads = 256;
-__global__ void __launch_bounds__( kSolveThreads ) lls_solve( const double* __restrict__ Gin, int L, float* __restrict__ w,
-                                                            int* __restrict__ status )
-{
-    const int ld = L + 1;
-    const int E = L * ld;
-    extern __shared__ double Gm[]; // [L][L+1], 132 KB at L = 128
-    for ( int e = threadIdx.x; e < E; e += kSolveThreads )
-        Gm[ e ] = Gin[ e ];
-    __shared__ int bad;
-    if ( threadIdx.x == 0 )
-        bad = 0;
-    __syncthreads();
-    for ( int j = 0; j < L; j++ )
-    {
-        if ( threadIdx.x == 0 )
-        {
-            double d = Gm[ j * ld + j ];
-            if ( !( d > 0.0 ) )
-                bad = 1;
-            Gm[ j * ld + j ] = d > 0.0 ? sqrt( d ) : 1.0;
-        }
-        __syncthreads();
-        const double djj = Gm[ j * ld + j ];
-        for ( int i = j + 1 + threadIdx.x; i < L; i += kSolveThreads )
-            Gm[ i * ld + j ] /= djj;
-        __syncthreads();
-        const int rem = L - j - 1;
-        for ( int e = threadIdx.x; e < rem * rem; e += kSolveThreads )
-        {
-            const int i = j + 1 + e / rem, k = j + 1 + e % rem;
-            if ( k <= i )
-                Gm[ i * ld + k ] -= Gm[ i * ld + j ] * Gm[ k * ld + j ];
-        }
-        __syncthreads();
-    }
-    if ( threadIdx.x == 0 )
-    {
-        for ( int i = 0; i < L; i++ )
-        {
-            double s = Gm[ i * ld + L ];
-            for ( int k = 0; k < i; k++ )
-                s -= Gm[ i * ld + k ] * Gm[ k * ld + L ];
-            Gm[ i * ld + L ] = s / Gm[ i * ld + i ];
-        }
-        for ( int i = L - 1; i >= 0; i-- )
-        {
-            double s = Gm[ i * ld + L ];
-            for ( int k = i + 1; k < L; k++ )
-                s -= Gm[ k * ld + i ] * Gm[ k * ld + L ];
-            Gm[ i * ld + L ] = s / Gm[ i * ld + i ];
-        }
-        for ( int i = 0; i < L; i++ )
-            w[ i ] = (float)Gm[ i * ld + L ];
-        *status = bad ? -1 : 0;
-    }
-}
-
-// est[m] = (a_m . w, b_m . w)  (lls_detector.cu:207-218, a GEMV over the embedding).
-__global__ void lls_apply( const float* __restrict__ rx, int N, int64_t M, const float* __restrict__ w, float* __restrict__ est )
-{
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if ( m >= M )
-        return;
-    float ea = 0.f, eb = 0.f;
-    for ( int n = 0; n < N; n++ )
-    {
-        float2 v = reinterpret_cast<const float2*>( rx )[ (int64_t)n * M + m ];
-        ea += v.x * w[ n ] + v.y * w[ N + n ];
-        eb += v.y * w[ n ] - v.x * w[ N + n ];
-    }
-    reinterpret_cast<float2*>( est )[ m ] = make_float2( ea, eb );
-}
 
 // Low-level LLS over a general column-major real matrix A (m x n, leading dimension m) and
 // target y (m), as trainLowLevel / detectLowLevel take them (lls_detector.cu:157-179,207-218).
