@@ -414,9 +414,10 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
     // so only launch shapes of the same arithmetic compete.
     std::map<std::array<int, 3>, std::vector<int>> dBuckets;
     for ( int i = 0; i < n; i++ )
-        dBuckets[ { detectKernelOf( B->inst[ i ]->p.detect_precision, (uint32_t)det[ i ].N ), nmaxOf( det[ i ].N ),
-                    umaxOf( det[ i ].U ) } ]
-            .push_back( i );
+    {
+        const int kernel = detectKernelOf( B->inst[ i ]->p.detect_precision, (uint32_t)det[ i ].N );
+        dBuckets[ { kernel, nmaxOf( det[ i ].N ), detectUmaxOf( kernel, det[ i ].U ) } ].push_back( i );
+    }
     const size_t detOff = arena.add( det );
     struct DetBucket
     {

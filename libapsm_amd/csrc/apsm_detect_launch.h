@@ -156,7 +156,7 @@ struct WorkItem
     int tile;
 };
 
-// Single-handle detect of M samples; nmax in {4, 8, 16, 32, 64}, umax in {1, 2, 4, 8, 12, 16}.
+// Single-handle detect of M samples; nmax in {4, 8, 16, 32, 64}, umax 1 or even, up to 16.
 hipError_t launchDetectMfma( int prec, int nmax, int umax, hipStream_t s, const float* rx, int64_t M, const float* Z,
                              const float* Zn, const float* C, int64_t ldC, const float* theta, int64_t G, int U, float wL,
                              float wG, float g2, float* est, int N );

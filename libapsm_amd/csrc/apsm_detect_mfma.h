@@ -26,7 +26,7 @@
 // the clock falls from 2.1 GHz to 1.6 to 1.75. Detect calls before (FP32 products on
 // v_mfma_f32_32x32x2_f32, one block's products and exponentials after each other) and now:
 //   8 antennas, 685 centres, 3840 samples              60 -> 33 us
-//   16 antennas, 10 users, 4096 centres, 500k samples  5.69 -> 3.75 ms
+//   16 antennas, 10 users, 4096 centres, 500k samples  5.69 -> 3.39 ms
 //   32 antennas, 3690 centres, 49999 samples           678 -> 280 us
 //   64 antennas, 12 users, 16384 centres, 400k samples, bf16  16.1 -> 12.9 ms
 // or per block of 32 x 32 and SIMD, in cycles as if at 2.4 GHz: 1460 (8 antennas), 2070 (16), 3340 (32), 6880 (64).
@@ -577,8 +577,11 @@ struct MfmaTable
         case 1: return one<1>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
         case 2: return one<2>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
         case 4: return one<4>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
+        case 6: return one<6>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
         case 8: return one<8>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
+        case 10: return one<10>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
         case 12: return one<12>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
+        case 14: return one<14>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
         case 16: return one<16>( batch, s, rx, M, Z, Zn, C, ldC, theta, G, U, wL, wG, g2, est, N, d, items, nItems, grid, shape );
         default: return hipErrorInvalidValue;
         }

@@ -437,8 +437,8 @@ bool serverLaunchDetect( apsm_server* S )
     {
         apsm_handle* h = S->links[ f->f.link ].h;
         det.push_back( detectDescOf( h, f->dRxD, f->f.n_data, f->dEst ) );
-        dBuckets[ { detectKernelOf( h->p.detect_precision, (uint32_t)h->N ), nmaxOf( h->N ), umaxOf( h->U ) } ].push_back(
-            (int)det.size() - 1 );
+        const int kernel = detectKernelOf( h->p.detect_precision, (uint32_t)h->N );
+        dBuckets[ { kernel, nmaxOf( h->N ), detectUmaxOf( kernel, h->U ) } ].push_back( (int)det.size() - 1 );
         f->detectBatch = id;
     }
     const size_t detOff = arena.add( det );

@@ -59,6 +59,6 @@ def test_tile_edges(require_gpu, mode, N, G):
 
 
 @pytest.mark.parametrize("M", [1, 31, 33, 128, 257])
-@pytest.mark.parametrize("N,users", [(5, 2), (8, 3), (16, 5), (32, 8), (64, 10), (21, 16)])
+@pytest.mark.parametrize("N,users", [(5, 2), (8, 3), (16, 5), (32, 8), (64, 10), (21, 16), (8, 9), (16, 13)])
 def test_samples_and_user_groups(require_gpu, M, N, users):
     check("fp32-matrix", N, 70, M, users)
