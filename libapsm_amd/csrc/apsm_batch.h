@@ -66,7 +66,7 @@ __global__ void __launch_bounds__( winThreads( TP ) ) batch_train_win( const Seq
 __global__ void batch_theta( const ThetaDesc* __restrict__ d )
 {
     const ThetaDesc& t = d[ blockIdx.y ];
-    if ( (int)blockIdx.x >= t.U )
+    if ( (int)blockIdx.x >= t.U * 2 * t.N )
         return;
     thetaFullBody( t.Z, t.C, t.thOld, t.theta, t.N, t.j0, t.j1, t.ldC, blockIdx.x );
 }

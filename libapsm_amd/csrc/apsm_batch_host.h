@@ -143,7 +143,7 @@ void launchRoundPre( hipStream_t s, const PreLaunch& pl, const char* base, const
         HIP_OR_THROW( apsm::launchBatchBlockPre( o.first.first, o.first.second, s, (const apsm::PreDesc*)( base + o.second ),
                                                  (int)pl.buckets.at( o.first ).size(), pl.maxWg.at( o.first ) ) );
     if ( nComb > 0 )
-        HIP_OR_THROW( apsm::launchBatchEntryCombine( s, (const apsm::EntryMfmaDesc*)( base + combOff ), nComb, ( pl.maxCombine + 255 ) / 256 ) );
+        HIP_OR_THROW( apsm::launchBatchEntryCombine( s, (const apsm::EntryMfmaDesc*)( base + combOff ), nComb, ( pl.maxCombine + 63 ) / 64 ) );
 }
 
 // The same for a batch round: the (NMAX, UMAX) buckets are independent launches, run side by
@@ -172,7 +172,7 @@ void launchRoundPreForked( apsm_batch* B, const PreLaunch& pl, const char* base,
         HIP_OR_THROW( hipStreamWaitEvent( B->stream, B->join[ k ], 0 ) );
     }
     if ( nComb > 0 )
-        HIP_OR_THROW( apsm::launchBatchEntryCombine( B->stream, (const apsm::EntryMfmaDesc*)( base + combOff ), nComb, ( pl.maxCombine + 255 ) / 256 ) );
+        HIP_OR_THROW( apsm::launchBatchEntryCombine( B->stream, (const apsm::EntryMfmaDesc*)( base + combOff ), nComb, ( pl.maxCombine + 63 ) / 64 ) );
 }
 
 void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT, const uint32_t* T, const float* const* rxD, const uint32_t* M,
@@ -397,12 +397,12 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
                          } } );
     }
     {
-        int maxU = 1;
+        int maxUL = 1;
         for ( auto& t : theta )
-            maxU = std::max( maxU, t.U );
+            maxUL = std::max( maxUL, t.U * 2 * t.N );
         const size_t off = arena.add( theta );
         pend.push_back( { 0, [ = ]( const char* base ) {
-                             hipLaunchKernelGGL( apsm::batch_theta, dim3( maxU, n ), dim3( 256 ), 0, B->stream,
+                             hipLaunchKernelGGL( apsm::batch_theta, dim3( maxUL, n ), dim3( 256 ), 0, B->stream,
                                                  (const apsm::ThetaDesc*)( base + off ) );
                              HIP_OR_THROW( hipGetLastError() );
                          } } );

@@ -929,7 +929,7 @@ void trainDev( apsm_handle* h, const float* d_rx, const float* d_tx, int64_t T, 
         return; // the norm-constraint sequencer keeps theta explicitly and wrote it
     const int64_t newUsedC = (int64_t)( h->used / 2 );
     const int64_t lo = h->blocked ? std::min<int64_t>( h->a0Next / 2, newUsedC ) : std::max<int64_t>( 0, newUsedC - h->Hc );
-    hipLaunchKernelGGL( apsm::apsm_theta_full, dim3( U ), dim3( 256 ), 0, h->stream, nb.Z.ptr, nb.C.ptr, h->thOld.ptr,
+    hipLaunchKernelGGL( apsm::apsm_theta_full, dim3( U * h->L ), dim3( 256 ), 0, h->stream, nb.Z.ptr, nb.C.ptr, h->thOld.ptr,
                         h->theta.ptr, N, lo - h->bufBaseC, newUsedC - h->bufBaseC, ld );
     HIP_OR_THROW( hipGetLastError() );
 }

@@ -113,14 +113,15 @@ __host__ __device__ inline I gramRow( I i )
     return 3 * ( i * ( i + 1 ) / 2 ) + 6 * ( i >> 2 ) + ( ( 0x6310 >> ( 4 * ( i & 3 ) ) ) & 15 );
 }
 
-__host__ __device__ inline int64_t gramBlocks( int64_t nA )
+// Blocks of the lower triangle, one wave each: 16 x 16 for the window sequencer, 32 x 32 otherwise.
+__host__ __device__ inline int64_t gramBlocks( const GramArgs& a )
 {
-    const int64_t nb = ( nA + 31 ) / 32;
+    const int64_t nb = a.Wc ? ( a.nA + 15 ) / 16 : ( a.nA + 31 ) / 32;
     return nb * ( nb + 1 ) / 2;
 }
 
 // One train block's precompute as one launch: the entry-share chunks (entryWg workgroups), the
-// Gram blocks (gramWg workgroups of four 32 x 32 blocks) and the eviction shares (evWg
+// Gram blocks (gramWg workgroups of four blocks) and the eviction shares (evWg
 // workgroups of 256 threads), each workgroup taking one role; the chunk combine follows.
 struct PreDesc
 {
@@ -134,7 +135,7 @@ struct PreDesc
 inline void preShape( PreDesc& d )
 {
     d.entryWg = d.e.nChunks * entryTiles( d.e.a.nNewC );
-    d.gramWg = (int)( ( gramBlocks( d.g.a.nA ) + 3 ) / 4 );
+    d.gramWg = (int)( ( gramBlocks( d.g.a ) + 3 ) / 4 );
     d.evWg = d.hasEv ? (int)( ( (int64_t)d.v.a.nSteps * ( d.v.a.w2 / 2 ) + 255 ) / 256 ) : 0;
 }
 

@@ -99,18 +99,19 @@ __device__ __forceinline__ void unrollFor( F f )
     unrollSeq( f, std::make_integer_sequence<int, N> {} );
 }
 
-// WAVES: waves per workgroup (32 samples each); ETILE: dictionary entries per LDS tile (0:
-// mfmaTileOf).
-template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0>
-__device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
-                                                const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
-                                                const float* __restrict__ theta, int64_t G, int U, float wL, float wG, float g2,
-                                                float* __restrict__ est, int N, const int64_t tile )
+// The Gaussian part of f for 32 samples per wave over the dictionary entries [0, G) of Z, Zn, C:
+// load( n ) is antenna n of this lane's sample (zero for none), finish( fa, fb ) takes every user's sums
+// of the lane half h (the two halves of a wave hold disjoint entries of the same samples and are
+// not yet added). MASK: entries below first( j0 ), counted within the tile from j0, do not count.
+// WAVES: waves per workgroup; ETILE: dictionary entries per LDS tile (0: mfmaTileOf).
+template <int NMAX, int UMAX, int PREC, int WAVES, int ETILE, bool MASK, class LOAD, class FIRST, class FINISH>
+__device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const float* __restrict__ Zn, const float* __restrict__ C,
+                                              int64_t ldC, int64_t G, int U, float g2, int N, LOAD load, FIRST first, FINISH finish )
 {
     constexpr int K = 2 * NMAX, K16 = K < 16 ? 16 : K, T = K16 / 16; // components, padded; steps of 16
     constexpr int NS = PREC == PREC_F32 ? 3 : 1;
     constexpr int kTile = ETILE ? ETILE : mfmaTileOf( NMAX, PREC );
-    constexpr int kThreads = 64 * WAVES, kSamples = 32 * WAVES;
+    constexpr int kThreads = 64 * WAVES;
     constexpr int RowH = K16 + 8; // rows padded by 16 bytes against LDS bank conflicts of the 16-byte reads
     constexpr int kAllQuads = K16 / 4 * kTile, kQuads = ( kAllQuads + kThreads - 1 ) / kThreads; // groups of four components staged per thread
     constexpr int kCLoads = ( UMAX * kTile + kThreads - 1 ) / kThreads;
@@ -123,10 +124,8 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
     __shared__ __attribute__( ( aligned( 16 ) ) ) float sZn[ 3 ][ kTile ];
     __shared__ __attribute__( ( aligned( 16 ) ) ) float2 sC[ 3 ][ kTile * UMAX ]; // [entry][user]
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int col = lane & 31, h = lane >> 5;
-    const int64_t m = tile * kSamples + wave * 32 + col; // this lane's sample
-    const bool valid = m < M;
     const int L = 2 * N;
 
     // This lane's half of the sample as B operands: step t holds components 16t + 8h + i of X and Xs.
@@ -140,7 +139,6 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
     float xq; // -g2 |x|^2
     {
         float xn = 0.f;
-        const float2* r2 = reinterpret_cast<const float2*>( rx );
         if constexpr ( HALVES )
         {
 #pragma unroll
@@ -155,7 +153,7 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
                     for ( int e = 0; e < 2; e++ )
                     {
                         const int ant = 16 * t + 8 * h + i + e;
-                        v[ e ] = valid && ant < N ? r2[ (int64_t)ant * M + m ] : make_float2( 0.f, 0.f );
+                        v[ e ] = load( ant );
                         xn += v[ e ].x * v[ e ].x + v[ e ].y * v[ e ].y;
                     }
                     uint32_t pr[ NS ], pi[ NS ];
@@ -191,7 +189,7 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
                 for ( int e = 0; e < 2; e++ )
                 {
                     const int ant = ( i + e ) % NMAX;
-                    const float2 v = valid && ant < N ? r2[ (int64_t)ant * M + m ] : make_float2( 0.f, 0.f );
+                    const float2 v = load( ant );
                     if ( NMAX == 8 || i < 4 )
                         xn += v.x * v.x + v.y * v.y;
                     const bool lo = NMAX == 8 ? h == 0 : i < 4; // component of Re x
@@ -306,8 +304,9 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
     constexpr int kLvls = NS == 3 ? 3 : 1, kGroups = kLvls * T;
     constexpr int kProducts = ( NS == 3 ? 12 : 2 ) * T;
     // The next block's products run under this one's exponentials, into a second set of accumulators
-    // (one set, and one after the other, where two do not fit the registers).
-    constexpr bool PIPE = !SUBTRACT;
+    // (one set, and one after the other, where two do not fit the registers, and for the entering
+    // pilots' chunks of one or two blocks).
+    constexpr bool PIPE = !SUBTRACT && !MASK;
     mf32x16 accP[ PIPE ? 2 : 1 ], accS[ PIPE ? 2 : 1 ], accM;
     V az[ 2 ][ NS ];
     auto readGroup = [ & ]( int buf, int cb, auto gC ) {
@@ -342,7 +341,7 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
     // coefficient slot `slot`), between them the products of the next block (entries cbn of buffer
     // bufn) into the other set. The fences keep the two streams interleaved entry by entry.
     constexpr int PF = UMAX <= 2 ? 4 : 1; // entries whose coefficients are read ahead together
-    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC ) {
+    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, int rel = 0 ) {
         constexpr int d = dC;
         float2 co[ 2 ][ PF * UMAX ];
         float4 zq[ 2 ];
@@ -368,7 +367,9 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
             if constexpr ( PIPE )
                 unrollFor<k1 - k0>( [ & ]( auto kC ) { product( bufn, cbn, std::integral_constant<int, 1 - d> {}, std::integral_constant<int, k0 + kC> {} ); } );
             const float4 z4 = zq[ i / 4 & 1 ];
-            const float q = xq + ( i % 4 == 0 ? z4.x : i % 4 == 1 ? z4.y : i % 4 == 2 ? z4.z : z4.w );
+            float q = xq + ( i % 4 == 0 ? z4.x : i % 4 == 1 ? z4.y : i % 4 == 2 ? z4.z : z4.w );
+            if constexpr ( MASK ) // arithmetic, as a select of the results costs the scheduler its freedom
+                q -= entryOf( i ) >= rel ? 0.f : 1.0e30f;
             const float p = accP[ d ][ i ], s = accS[ d ][ i ];
             // exponentials clamped to 1 (a rounded distance below zero counts as 0)
             const float E0 = __builtin_amdgcn_fmed3f( __builtin_amdgcn_exp2f( fmaf( k2, p, q ) ), 0.f, 1.f );
@@ -423,8 +424,10 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
 #pragma unroll 1
             for ( int cb = 0; cb < kTile; cb += 32 )
             {
+                if ( (int64_t)tt * kTile + cb >= G )
+                    break;
                 products( tt & 1, cb );
-                phase( tt % 3, cb, 0, 0, D0 {} );
+                phase( tt % 3, cb, 0, 0, D0 {}, MASK ? first( (int64_t)tt * kTile ) : 0 );
             }
             advance( tt );
         }
@@ -461,37 +464,55 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
     }
     __syncthreads(); // a following tile stores over what other waves may still read
 
-    // the two lane halves saw disjoint entries of the same sample; f = wL theta . x + wG (Gaussian
-    // part), x read again
-#pragma unroll
-    for ( int u = 0; u < UMAX; u++ )
-    {
-        fa[ u ] += __shfl_xor( fa[ u ], 32 );
-        fb[ u ] += __shfl_xor( fb[ u ], 32 );
-    }
-    if ( valid && h == 0 )
-    {
-        float la[ UMAX ], lb[ UMAX ];
-#pragma unroll
-        for ( int u = 0; u < UMAX; u++ )
-            la[ u ] = lb[ u ] = 0.f;
-#pragma unroll 4
-        for ( int n = 0; n < N; n++ )
-        {
-            const float2 x = reinterpret_cast<const float2*>( rx )[ (int64_t)n * M + m ];
+    finish( fa, fb );
+}
+
+// One tile of 32 * WAVES data samples of a detect.
+template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0>
+__device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
+                                                const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
+                                                const float* __restrict__ theta, int64_t G, int U, float wL, float wG, float g2,
+                                                float* __restrict__ est, int N, const int64_t tile )
+{
+    const int h = ( threadIdx.x >> 5 ) & 1;
+    const int64_t m = tile * ( 32 * WAVES ) + ( threadIdx.x >> 6 ) * 32 + ( threadIdx.x & 31 ); // this lane's sample
+    const bool valid = m < M;
+    const float2* x = reinterpret_cast<const float2*>( rx ) + m;
+    gaussianMfma<NMAX, UMAX, PREC, WAVES, ETILE, false>(
+        Z, Zn, C, ldC, G, U, g2, N, [ & ]( int n ) { return valid && n < N ? x[ (int64_t)n * M ] : make_float2( 0.f, 0.f ); },
+        []( int64_t ) { return 0; },
+        [ & ]( float( &fa )[ UMAX ], float( &fb )[ UMAX ] ) {
+            // f = wL theta . x + wG (Gaussian part), x read again
 #pragma unroll
             for ( int u = 0; u < UMAX; u++ )
             {
-                const float* th = theta + ( u < U ? u : 0 ) * L;
-                la[ u ] += fmaf( th[ n ], x.x, th[ N + n ] * x.y );
-                lb[ u ] += fmaf( th[ n ], x.y, -th[ N + n ] * x.x );
+                fa[ u ] += __shfl_xor( fa[ u ], 32 );
+                fb[ u ] += __shfl_xor( fb[ u ], 32 );
             }
-        }
+            if ( !valid || h != 0 )
+                return;
+            float la[ UMAX ], lb[ UMAX ];
 #pragma unroll
-        for ( int u = 0; u < UMAX; u++ )
-            if ( u < U )
-                reinterpret_cast<float2*>( est )[ (int64_t)u * M + m ] = make_float2( wL * la[ u ] + wG * fa[ u ], wL * lb[ u ] + wG * fb[ u ] );
-    }
+            for ( int u = 0; u < UMAX; u++ )
+                la[ u ] = lb[ u ] = 0.f;
+#pragma unroll 4
+            for ( int n = 0; n < N; n++ )
+            {
+                const float2 v = x[ (int64_t)n * M ];
+#pragma unroll
+                for ( int u = 0; u < UMAX; u++ )
+                {
+                    const float* th = theta + ( u < U ? u : 0 ) * 2 * N;
+                    la[ u ] += fmaf( th[ n ], v.x, th[ N + n ] * v.y );
+                    lb[ u ] += fmaf( th[ n ], v.y, -th[ N + n ] * v.x );
+                }
+            }
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
+                if ( u < U )
+                    reinterpret_cast<float2*>( est )[ (int64_t)u * M + m ] =
+                        make_float2( wL * la[ u ] + wG * fa[ u ], wL * lb[ u ] + wG * fb[ u ] );
+        } );
 }
 
 // Two workgroups of four waves per CU at least: 256 registers per wave, which also keeps the matrix

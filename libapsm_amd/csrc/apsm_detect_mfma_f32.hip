@@ -22,13 +22,13 @@ hipError_t launchEntryCombine( hipStream_t s, const float* Z, const float* thF, 
                                int nChunks )
 {
     const int n = a.U * a.nNewC;
-    hipLaunchKernelGGL( apsm_entry_combine, dim3( ( n + 255 ) / 256 ), dim3( 256 ), 0, s, Z, thF, part, P, a, nChunks );
+    hipLaunchKernelGGL( apsm_entry_combine, dim3( ( n + 63 ) / 64 ), dim3( kCombineThreads ), 0, s, Z, thF, part, P, a, nChunks );
     return hipGetLastError();
 }
 
 hipError_t launchBatchEntryCombine( hipStream_t s, const EntryMfmaDesc* d, int n, int gridX )
 {
-    hipLaunchKernelGGL( batch_entry_combine, dim3( gridX, n ), dim3( 256 ), 0, s, d );
+    hipLaunchKernelGGL( batch_entry_combine, dim3( gridX, n ), dim3( kCombineThreads ), 0, s, d );
     return hipGetLastError();
 }
 

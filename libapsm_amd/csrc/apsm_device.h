@@ -341,39 +341,39 @@ __global__ void __launch_bounds__( kSeqThreads ) apsm_train_seq( const float* __
         thOld[ u * L + i ] = sTh[ i ];
 }
 
-// theta = thOld + sum over dictionary rows of c_j x_j (one workgroup of 256 threads per user u).
+// theta = thOld + sum over dictionary rows of c_j x_j: one workgroup of 256 threads per user and
+// component, wg = u L + d (one workgroup per user took 2 N rounds of loads and barriers).
 __device__ __forceinline__ void thetaFullBody( const float* __restrict__ Z, const float* __restrict__ C, const float* __restrict__ thOld,
-                                               float* __restrict__ theta, int N, int64_t j0, int64_t j1, int64_t ldC, const int u )
+                                               float* __restrict__ theta, int N, int64_t j0, int64_t j1, int64_t ldC, const int wg )
 {
-    const int L = 2 * N;
-    __shared__ float red[ 4 ][ 256 ];
+    const int L = 2 * N, u = wg / L, d = wg % L;
+    __shared__ float red[ 4 ];
     const float* Cu = C + u * ldC;
-    for ( int d = 0; d < L; d++ )
+    const int db = d < N ? N + d : d - N;
+    const float sign = d < N ? 1.f : -1.f;
+    float acc = 0.f;
+#pragma unroll 8
+    for ( int64_t j = j0 + threadIdx.x; j < j1; j += 256 )
     {
-        float acc = 0.f;
-        for ( int64_t j = j0 + threadIdx.x; j < j1; j += blockDim.x )
-        {
-            const float* zj = Z + j * L;
-            float bd = d < N ? zj[ N + d ] : -zj[ d - N ];
-            acc += Cu[ 2 * j ] * zj[ d ] + Cu[ 2 * j + 1 ] * bd;
-        }
-        acc = waveSum( acc );
-        if ( ( threadIdx.x & 63 ) == 0 )
-            red[ threadIdx.x / 64 ][ d & 255 ] = acc;
-        __syncthreads();
-        if ( threadIdx.x == 0 )
-        {
-            float s = thOld[ u * L + d ];
-            for ( int w = 0; w < (int)( blockDim.x / 64 ); w++ )
-                s += red[ w ][ d & 255 ];
-            theta[ u * L + d ] = s;
-        }
-        __syncthreads();
+        const float* zj = Z + j * L;
+        acc += Cu[ 2 * j ] * zj[ d ] + Cu[ 2 * j + 1 ] * ( sign * zj[ db ] );
+    }
+    acc = waveSum( acc );
+    if ( ( threadIdx.x & 63 ) == 0 )
+        red[ threadIdx.x / 64 ] = acc;
+    __syncthreads();
+    if ( threadIdx.x == 0 )
+    {
+        float s = thOld[ wg ];
+        for ( int w = 0; w < 4; w++ )
+            s += red[ w ];
+        theta[ wg ] = s;
     }
 }
 
-__global__ void apsm_theta_full( const float* __restrict__ Z, const float* __restrict__ C, const float* __restrict__ thOld,
-                                 float* __restrict__ theta, int N, int64_t j0, int64_t j1, int64_t ldC )
+__global__ void __launch_bounds__( 256 ) apsm_theta_full( const float* __restrict__ Z, const float* __restrict__ C,
+                                                         const float* __restrict__ thOld, float* __restrict__ theta, int N, int64_t j0,
+                                                         int64_t j1, int64_t ldC )
 {
     thetaFullBody( Z, C, thOld, theta, N, j0, j1, ldC, blockIdx.x );
 }

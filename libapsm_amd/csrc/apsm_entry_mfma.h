@@ -7,9 +7,7 @@
 // dictionary's lower end when sample i enters (the FIFO may already have dropped entries).
 // The frozen range is cut into chunks of kEntryChunk entries counted from its top (chunk 0 holds
 // the most recently frozen entries); one workgroup takes one chunk
-// for all (at most 128) entering samples, with the layout of the matrix-core detect (4 waves x
-// 32 samples, lane l holds sample l % 32 and entries 8(v/4) + 4(l/32) + v%4 of each 32-entry
-// block), masks the entries below j0(i), and writes its partial sums. A second kernel adds the
+// for 128 entering samples, as the matrix-core detect (4 waves x 32 samples) does, masks the entries below j0(i), and writes its partial sums. A second kernel adds the
 // chunks in order and the linear share: P_u(i) = wL thF_u.x_i + wG g_u(i).
 #pragma once
 
@@ -25,18 +23,10 @@ __device__ __forceinline__ void entryChunkMfma( const float* __restrict__ Z, con
 {
     // work item = (tile of kMfmaSamples entering samples, chunk of the frozen range)
     const int chunk = work % nChunks, mBase = ( work / nChunks ) * kMfmaSamples;
-    constexpr int K = 2 * NMAX;
-    constexpr int kTile = NMAX >= 64 ? 32 : 64;
-    __shared__ float sZf[ 2 * K * kTile ];
-    __shared__ float sZn[ kTile ];
-    __shared__ float2 sC[ UMAX * kTile ];
-
-    const int N = a.N, L = a.L, U = a.U;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int col = lane & 31, h = lane >> 5;
-    const int m = mBase + wave * 32 + col; // entering sample of this lane
+    const int N = a.N, L = a.L;
+    const int h = ( threadIdx.x >> 5 ) & 1;
+    const int m = mBase + ( threadIdx.x >> 6 ) * 32 + ( threadIdx.x & 31 ); // entering sample of this lane
     const bool valid = m < a.nNewC;
-    const float g2 = a.g2;
 
     // dictionary lower end when sample m enters (entries below it are masked)
     const int64_t tc = a.newC0 + m;
@@ -46,163 +36,108 @@ __device__ __forceinline__ void entryChunkMfma( const float* __restrict__ Z, con
     const int64_t jlo = ( lo - a.rowBase ) / 2;
     const int64_t j1 = ( a.a0 - a.rowBase ) / 2;
 
-    float xb[ K / 2 ];
-    float xn = 0.f;
-#pragma unroll
-    for ( int t = 0; t < K / 2; t++ )
-    {
-        const int k = 2 * t + h;
-        const int ant = k < NMAX ? k : k - NMAX;
-        float v = 0.f;
-        if ( valid && ant < N )
-            v = Z[ tc * L + ( k < NMAX ? ant : N + ant ) ];
-        xb[ t ] = v;
-        xn += v * v;
-    }
-    xn += __shfl_xor( xn, 32 );
-    const float xq = -g2 * xn, k2 = 2.f * g2;
-
-    float fa[ UMAX ], fb[ UMAX ];
-#pragma unroll
-    for ( int u = 0; u < UMAX; u++ )
-        fa[ u ] = fb[ u ] = 0.f;
-
     // chunks from the top of the frozen range: chunk 0 holds the most recently frozen entries
     const int64_t c1 = j1 - (int64_t)chunk * kEntryChunk;
     const int64_t c0 = ( c1 - kEntryChunk ) > jBeg ? c1 - kEntryChunk : jBeg;
-    for ( int64_t j0 = c0; j0 < c1; j0 += kTile )
-    {
-        const int nt = ( c1 - j0 ) < kTile ? (int)( c1 - j0 ) : kTile;
-        __syncthreads();
-#pragma unroll 2
-        for ( int i = tid; i < K * kTile; i += kMfmaThreads )
-        {
-            const int k = i / kTile, e = i % kTile;
-            const int n = k < NMAX ? k : k - NMAX;
-            float zr = 0.f, zi = 0.f;
-            if ( e < nt && n < N )
+    const float* x = Z + tc * L;
+    gaussianMfma<NMAX, UMAX, PREC_F32, kMfmaThreads / 64, 0, true>(
+        Z + c0 * L, Zn + c0, C + 2 * c0, a.ldYC, c1 - c0, a.U, a.g2, N,
+        [ & ]( int n ) { return valid && n < N ? make_float2( x[ n ], x[ N + n ] ) : make_float2( 0.f, 0.f ); },
+        [ & ]( int64_t j0 ) { // entries of the tile from j0 that the FIFO dropped before this lane's sample entered
+            const int64_t d = jlo - c0 - j0;
+            return d < 0 ? 0 : d > kEntryChunk ? (int)kEntryChunk : (int)d;
+        },
+        [ & ]( float( &fa )[ UMAX ], float( &fb )[ UMAX ] ) {
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
             {
-                zr = Z[ ( j0 + e ) * L + n ];
-                zi = Z[ ( j0 + e ) * L + N + n ];
+                fa[ u ] += __shfl_xor( fa[ u ], 32 );
+                fb[ u ] += __shfl_xor( fb[ u ], 32 );
             }
-            sZf[ k * kTile + e ] = k < NMAX ? zr : zi;
-            sZf[ K * kTile + k * kTile + e ] = k < NMAX ? zi : -zr;
-        }
-        for ( int i = tid; i < kTile; i += kMfmaThreads )
-            sZn[ i ] = i < nt ? -g2 * Zn[ j0 + i ] : 0.f;
-        for ( int i = tid; i < UMAX * kTile; i += kMfmaThreads )
-        {
-            const int u = i / kTile, e = i % kTile;
-            sC[ i ] = ( u < U && e < nt ) ? make_float2( C[ u * a.ldYC + 2 * ( j0 + e ) ], C[ u * a.ldYC + 2 * ( j0 + e ) + 1 ] )
-                                          : make_float2( 0.f, 0.f );
-        }
-        __syncthreads();
-        // first entry of this tile the lane's sample may use (the FIFO dropped those below)
-        const int rel = jlo <= j0 ? 0 : ( jlo - j0 >= kTile ? kTile : (int)( jlo - j0 ) );
-
-#pragma unroll 1
-        for ( int cb = 0; cb < nt; cb += 32 )
-        {
-            mf32x16 accP = {}, accS = {};
+            if ( !valid || h != 0 )
+                return;
 #pragma unroll
-            for ( int t = 0; t < K / 2; t++ )
-            {
-                const int k = 2 * t + h;
-                const float ap = sZf[ k * kTile + cb + col ];
-                const float as = sZf[ K * kTile + k * kTile + cb + col ];
-                accP = __builtin_amdgcn_mfma_f32_32x32x2f32( ap, xb[ t ], accP, 0, 0, 0 );
-                accS = __builtin_amdgcn_mfma_f32_32x32x2f32( as, xb[ t ], accS, 0, 0, 0 );
-                if ( ( t & 7 ) == 7 )
-                    __builtin_amdgcn_sched_barrier( 0 );
-            }
-#pragma unroll
-            for ( int v = 0; v < 16; v++ )
-            {
-                const int e = cb + 8 * ( v / 4 ) + 4 * h + ( v % 4 );
-                // entries the FIFO dropped before this sample entered contribute nothing: their
-                // exponent argument is pushed to -1e30 (an arithmetic mask; a select here costs
-                // the scheduler its freedom and doubles the register count)
-                const float q = xq + sZn[ e ] - ( e >= rel ? 0.f : 1.0e30f );
-                const float p = accP[ v ], s = accS[ v ];
-                const float E0 = __builtin_amdgcn_exp2f( fminf( fmaf( k2, p, q ), 0.f ) );
-                const float E1 = __builtin_amdgcn_exp2f( fminf( fmaf( k2, s, q ), 0.f ) );
-                const float E2 = __builtin_amdgcn_exp2f( fminf( fmaf( -k2, s, q ), 0.f ) );
-#pragma unroll
-                for ( int u = 0; u < UMAX; u++ )
-                {
-                    const float2 c = sC[ u * kTile + e ];
-                    fa[ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ u ] ) );
-                    fb[ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ u ] ) );
-                }
-                if ( NMAX <= 32 )
-                    __builtin_amdgcn_sched_barrier( 0 );
-            }
-        }
-    }
-#pragma unroll
-    for ( int u = 0; u < UMAX; u++ )
-    {
-        fa[ u ] += __shfl_xor( fa[ u ], 32 );
-        fb[ u ] += __shfl_xor( fb[ u ], 32 );
-    }
-    if ( !valid || h != 0 )
-        return;
-#pragma unroll
-    for ( int u = 0; u < UMAX; u++ )
-        if ( u < U )
-            reinterpret_cast<float2*>( part )[ ( (int64_t)u * nChunks + chunk ) * a.nNewC + m ] = make_float2( fa[ u ], fb[ u ] );
+            for ( int u = 0; u < UMAX; u++ )
+                if ( u < a.U )
+                    reinterpret_cast<float2*>( part )[ ( (int64_t)u * nChunks + chunk ) * a.nNewC + m ] = make_float2( fa[ u ], fb[ u ] );
+        } );
 }
 
-// P_u(i) = wL thF_u.x_i + wG (chunk partials added in chunk order); one thread per (u, i).
+// P_u(i) = wL thF_u.x_i + wG (sum of the chunk partials): 64 (u, i) per workgroup, 16 slices of the
+// antennas and of the chunks, whose sums are added in order. (One thread per (u, i) waited for
+// the chunks one after another.)
+constexpr int kCombineSlices = 16, kCombineThreads = 64 * kCombineSlices;
 __device__ __forceinline__ void entryCombineBody( const float* __restrict__ Z, const float* __restrict__ thF, const float* __restrict__ part,
-                                                  float* __restrict__ P, const EntryArgs& a, const int nChunks, const int idx )
+                                                  float* __restrict__ P, const EntryArgs& a, const int nChunks, const int wg )
 {
-    if ( idx >= a.U * a.nNewC )
-        return;
-    const int u = idx / a.nNewC, i = idx % a.nNewC;
+    __shared__ float4 sum[ kCombineSlices ][ 64 ];
+    const int col = threadIdx.x & 63, slice = threadIdx.x >> 6;
+    const int idx = wg * 64 + col;
     const int N = a.N;
-    const float* x = Z + ( a.newC0 + i ) * a.L;
-    const float* th = thF + (int64_t)u * a.L;
-    float la = 0.f, lb = 0.f;
-    for ( int n = 0; n < N; n++ )
+    float la = 0.f, lb = 0.f, ga = 0.f, gb = 0.f;
+    if ( idx < a.U * a.nNewC )
     {
-        const float xr = x[ n ], xi = x[ N + n ];
-        la += th[ n ] * xr + th[ N + n ] * xi;
-        lb += th[ n ] * xi - th[ N + n ] * xr;
-    }
-    float ga = 0.f, gb = 0.f;
-    const float2* pp = reinterpret_cast<const float2*>( part ) + (int64_t)u * nChunks * a.nNewC + i;
+        const int u = idx / a.nNewC, i = idx % a.nNewC;
+        const float* x = Z + ( a.newC0 + i ) * a.L;
+        const float* th = thF + (int64_t)u * a.L;
+#pragma unroll 4
+        for ( int n = slice; n < N; n += kCombineSlices )
+        {
+            const float xr = x[ n ], xi = x[ N + n ];
+            la += fmaf( th[ n ], xr, th[ N + n ] * xi );
+            lb += fmaf( th[ n ], xi, -th[ N + n ] * xr );
+        }
+        const float2* pp = reinterpret_cast<const float2*>( part ) + (int64_t)u * nChunks * a.nNewC + i;
 #pragma unroll 8
-    for ( int c = 0; c < nChunks; c++ )
-    {
-        const float2 v = pp[ (int64_t)c * a.nNewC ];
-        ga += v.x;
-        gb += v.y;
+        for ( int c = slice; c < nChunks; c += kCombineSlices )
+        {
+            const float2 v = pp[ (int64_t)c * a.nNewC ];
+            ga += v.x;
+            gb += v.y;
+        }
     }
-    P[ ( (int64_t)u * a.nNewC + i ) * 2 + 0 ] = a.wL * la + a.wG * ga;
-    P[ ( (int64_t)u * a.nNewC + i ) * 2 + 1 ] = a.wL * lb + a.wG * gb;
+    sum[ slice ][ col ] = make_float4( la, lb, ga, gb );
+    __syncthreads();
+    if ( slice != 0 || idx >= a.U * a.nNewC )
+        return;
+#pragma unroll
+    for ( int k = 1; k < kCombineSlices; k++ )
+    {
+        const float4 v = sum[ k ][ col ];
+        la += v.x;
+        lb += v.y;
+        ga += v.z;
+        gb += v.w;
+    }
+    reinterpret_cast<float2*>( P )[ idx ] = make_float2( a.wL * la + a.wG * ga, a.wL * lb + a.wG * gb );
 }
 
 template <int NMAX, int UMAX>
-__global__ void __launch_bounds__( kMfmaThreads ) apsm_entry_mfma( const float* __restrict__ Z, const float* __restrict__ Zn,
+__global__ void __launch_bounds__( kMfmaThreads, 2 ) apsm_entry_mfma( const float* __restrict__ Z, const float* __restrict__ Zn,
                                                                   const float* __restrict__ C, float* __restrict__ part, const EntryArgs a,
                                                                   int64_t jBeg, int nChunks, int chunk0 )
 {
     entryChunkMfma<NMAX, UMAX>( Z, Zn, C, part, a, jBeg, nChunks, chunk0 + blockIdx.x );
 }
 
-__global__ void apsm_entry_combine( const float* __restrict__ Z, const float* __restrict__ thF, const float* __restrict__ part,
+__global__ void __launch_bounds__( kCombineThreads ) apsm_entry_combine( const float* __restrict__ Z, const float* __restrict__ thF, const float* __restrict__ part,
                                     float* __restrict__ P, const EntryArgs a, int nChunks )
 {
-    entryCombineBody( Z, thF, part, P, a, nChunks, blockIdx.x * blockDim.x + threadIdx.x );
+    entryCombineBody( Z, thF, part, P, a, nChunks, blockIdx.x );
 }
 
-__global__ void batch_entry_combine( const EntryMfmaDesc* __restrict__ d )
+__global__ void __launch_bounds__( kCombineThreads ) batch_entry_combine( const EntryMfmaDesc* __restrict__ d )
 {
     const EntryMfmaDesc& e = d[ blockIdx.y ];
-    entryCombineBody( e.Z, e.thF, e.part, e.P, e.a, e.nChunks, blockIdx.x * blockDim.x + threadIdx.x );
+    if ( (int)blockIdx.x * 64 < e.a.U * e.a.nNewC )
+        entryCombineBody( e.Z, e.thF, e.part, e.P, e.a, e.nChunks, blockIdx.x );
 }
 
+// What a further block of a train call costs besides its steps (precompute, combine, launches; 8
+// antennas, at windowSize 20 / 40 / 80 / 160): 17 / 24 / 25 / 36 us with FP32 products of 32 x 32 blocks, one load
+// at a time and a serial combine, 11 / 12 / 13 / 21 us now. Latency bounds it: a few hundred waves, each
+// one chain.
+//
 // One block's precompute, workgroup b: entry work item (the first entryWg workgroups), Gram
 // blocks (the next gramWg) or eviction shares (the last evWg); batched: gridX = the largest sum.
 template <int NMAX, int UMAX>
@@ -217,7 +152,7 @@ __device__ __forceinline__ void blockPreBody( const PreDesc& d, int b )
     if ( b < d.gramWg )
     {
         const int64_t blk = (int64_t)b * ( kMfmaThreads / 64 ) + ( threadIdx.x >> 6 );
-        if ( blk < gramBlocks( d.g.a.nA ) )
+        if ( blk < gramBlocks( d.g.a ) )
         {
             if ( d.g.a.Wc )
                 gramWinMfma<NMAX>( d.g.Z, d.g.Zn, d.g.Gact, d.g.a, blk );
@@ -232,13 +167,13 @@ __device__ __forceinline__ void blockPreBody( const PreDesc& d, int b )
 }
 
 template <int NMAX, int UMAX>
-__global__ void __launch_bounds__( kMfmaThreads ) apsm_block_pre( const PreDesc d )
+__global__ void __launch_bounds__( kMfmaThreads, 2 ) apsm_block_pre( const PreDesc d )
 {
     blockPreBody<NMAX, UMAX>( d, blockIdx.x );
 }
 
 template <int NMAX, int UMAX>
-__global__ void __launch_bounds__( kMfmaThreads ) batch_block_pre( const PreDesc* __restrict__ d )
+__global__ void __launch_bounds__( kMfmaThreads, 2 ) batch_block_pre( const PreDesc* __restrict__ d )
 {
     const PreDesc& x = d[ blockIdx.y ];
     if ( (int)blockIdx.x >= x.entryWg + x.gramWg + x.evWg )

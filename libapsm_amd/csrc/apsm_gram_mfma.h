@@ -10,6 +10,8 @@
 
 namespace apsm {
 
+typedef float f32x4 __attribute__( ( ext_vector_type( 4 ) ) );
+
 template <int NMAX>
 __device__ __forceinline__ void gramBlockMfma( const float* __restrict__ Z, const float* __restrict__ Zn, float* __restrict__ Gact,
                                                const GramArgs& a, const int64_t blk )
@@ -78,57 +80,63 @@ __device__ __forceinline__ void gramBlockMfma( const float* __restrict__ Z, cons
 // The same values in the window sequencer's layout (apsm_train_win.h). Here the rows i are the A
 // operand and the rows j the B operand, so that the lanes of a store run along j, which is along
 // an image's slots: the stores are contiguous but for the slots' wrap.
+//
+// Few waves, each a chain of loads, products, exponentials and stores, bound this: blocks of 16 x 16
+// (v_mfma_f32_16x16x4_f32, four pairs per lane) give four times the waves of 32 x 32 ones, and all loads
+// are issued before the first use.
 template <int NMAX>
 __device__ __forceinline__ void gramWinMfma( const float* __restrict__ Z, const float* __restrict__ Zn, float* __restrict__ Gact,
                                              const GramArgs& a, const int64_t blk )
 {
-    constexpr int K = 2 * NMAX;
+    constexpr int T = NMAX / 4; // steps of four antennas
     const int N = a.N, L = a.L, Wc = a.Wc, tp = a.tp, nA = (int)a.nA, newRel0 = a.newRel0;
     const int lane = threadIdx.x & 63;
-    const int col = lane & 31, h = lane >> 5;
+    const int r = lane & 15, g = lane >> 4;
     int bi = (int)( ( sqrtf( 8.f * (float)blk + 1.f ) - 1.f ) * 0.5f );
     while ( ( bi + 1 ) * ( bi + 2 ) / 2 <= blk )
         bi++;
     while ( bi * ( bi + 1 ) / 2 > blk )
         bi--;
     const int bj = (int)blk - bi * ( bi + 1 ) / 2;
-    const int ir = bi * 32 + col; // the row this lane supplies as A operand
-    const int j = bj * 32 + col; // this lane's B operand column
+    const int ir = bi * 16 + r; // the row this lane supplies as A operand
+    const int j = bj * 16 + r; // this lane's B operand column
     const bool vi = ir < nA, vj = j < nA;
     const float* xi = Z + ( a.c0 + ir ) * L;
     const float* zj = Z + ( a.c0 + j ) * L;
-    float xv[ K / 2 ], zr[ K / 2 ], zim[ K / 2 ];
+    float xr[ T ], xm[ T ], zr[ T ], zm[ T ], ni[ 4 ];
 #pragma unroll
-    for ( int t = 0; t < K / 2; t++ )
+    for ( int t = 0; t < T; t++ )
     {
-        const int k = 2 * t + h;
-        const int ant = k < NMAX ? k : k - NMAX;
-        xv[ t ] = ( ant < N && vi ) ? xi[ k < NMAX ? ant : N + ant ] : 0.f;
-        zr[ t ] = ( ant < N && vj ) ? zj[ ant ] : 0.f;
-        zim[ t ] = ( ant < N && vj ) ? zj[ N + ant ] : 0.f;
+        const int n = 4 * t + g;
+        xr[ t ] = n < N && vi ? xi[ n ] : 0.f;
+        xm[ t ] = n < N && vi ? xi[ N + n ] : 0.f;
+        zr[ t ] = n < N && vj ? zj[ n ] : 0.f;
+        zm[ t ] = n < N && vj ? zj[ N + n ] : 0.f;
     }
-    mf32x16 accP = {}, accS = {};
+    const int i0 = bi * 16 + 4 * g; // this lane's pairs: (i0 + v, j)
 #pragma unroll
-    for ( int t = 0; t < K / 2; t++ )
+    for ( int v = 0; v < 4; v++ )
+        ni[ v ] = Zn[ a.c0 + ( i0 + v < nA ? i0 + v : nA - 1 ) ];
+    const float nj = Zn[ a.c0 + ( vj ? j : nA - 1 ) ];
+    f32x4 accP = { 0.f, 0.f, 0.f, 0.f }, accS = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+    for ( int t = 0; t < T; t++ )
     {
-        const bool re = 2 * t + h < NMAX;
-        const float zp = re ? zr[ t ] : zim[ t ]; // Zp row = [Re z | Im z]
-        const float zs = re ? zim[ t ] : -zr[ t ]; // Zs row = [Im z | -Re z]
-        accP = __builtin_amdgcn_mfma_f32_32x32x2f32( xv[ t ], zp, accP, 0, 0, 0 );
-        accS = __builtin_amdgcn_mfma_f32_32x32x2f32( xv[ t ], zs, accS, 0, 0, 0 );
+        accP = __builtin_amdgcn_mfma_f32_16x16x4f32( xr[ t ], zr[ t ], accP, 0, 0, 0 );
+        accS = __builtin_amdgcn_mfma_f32_16x16x4f32( xr[ t ], zm[ t ], accS, 0, 0, 0 );
+        accP = __builtin_amdgcn_mfma_f32_16x16x4f32( xm[ t ], zm[ t ], accP, 0, 0, 0 );
+        accS = __builtin_amdgcn_mfma_f32_16x16x4f32( -xm[ t ], zr[ t ], accS, 0, 0, 0 );
     }
     const int img = winImg( tp ), part = winPart( tp ), tpq = winTpq( tp );
     const float g2 = a.g2, k2 = 2.f * g2;
-    const float qj = vj ? -g2 * Zn[ a.c0 + j ] : 0.f;
+    const float qj = -g2 * nj;
     const int sj = ( a.cMod + j ) % Wc;
     const int oj = ( sj / tp ) * part + sj % tp; // this column's place in an image
 #pragma unroll
-    for ( int v = 0; v < 16; v++ )
+    for ( int v = 0; v < 4; v++ )
     {
-        const int i = bi * 32 + 8 * ( v / 4 ) + 4 * h + ( v % 4 );
-        if ( j > i || i >= nA )
-            continue;
-        const float q = qj - g2 * Zn[ a.c0 + i ];
+        const int i = i0 + v;
+        const float q = qj - g2 * ni[ v ];
         const float p = accP[ v ], s = accS[ v ];
         const float E0 = __builtin_amdgcn_exp2f( fminf( fmaf( k2, p, q ), 0.f ) );
         const float E1 = __builtin_amdgcn_exp2f( fminf( fmaf( k2, s, q ), 0.f ) );
@@ -136,6 +144,8 @@ __device__ __forceinline__ void gramWinMfma( const float* __restrict__ Z, const 
         const float kA = a.wL * p + a.wG * E0; // kappa(a_i,a_j) = kappa(b_i,b_j)
         const float kB = a.wL * s + a.wG * E1; // kappa(a_i,b_j)
         const float kC = -a.wL * s + a.wG * E2; // kappa(b_i,a_j)
+        if ( j > i || i >= nA )
+            continue;
         if ( i < newRel0 )
         {
             // both in the window at the block start: the image of j (t = i) and the image of i (t = j)
@@ -179,28 +189,28 @@ __device__ __forceinline__ void gramWinMfma( const float* __restrict__ Z, const 
         return;
     // what a package row holds besides pairs: zeros in the image for slots without an active sample
     // and past the window, and in the padding of the older planes (all are multiplied by zero
-    // coefficients, so they must be finite)
-    for ( int i = bi * 32; i < bi * 32 + 32 && i < nA; i++ )
+    // coefficients, so they must be finite); 16 lanes per row
+    for ( int i = bi * 16 + g; i < bi * 16 + 16 && i < nA; i += 4 )
     {
         if ( i < newRel0 )
             continue;
         const int e = i - newRel0;
         float* o = Gact + winRow( e, newRel0, Wc, tp );
-        for ( int n = lane; n < Wc - i; n += 64 )
+        for ( int n = r; n < Wc - i; n += 16 )
         {
             const int sl = ( a.cMod + Wc - 1 - n ) % Wc; // relative sample -1 - n
             float* z = o + ( sl / tp ) * part + sl % tp;
             z[ 0 ] = z[ tpq ] = z[ 2 * tpq ] = 0.f;
         }
-        for ( int sl = Wc + lane; sl < 4 * tp; sl += 64 )
+        for ( int sl = Wc + r; sl < 4 * tp; sl += 16 )
         {
             float* z = o + ( sl / tp ) * part + sl % tp;
             z[ 0 ] = z[ tpq ] = z[ 2 * tpq ] = 0.f;
         }
         const int older = winOlder( e, newRel0, Wc ), o4 = ( older + 3 ) & ~3;
-        if ( lane < 3 )
+        if ( r < 3 )
             for ( int n = older; n < o4; n++ )
-                o[ img + 4 + lane * o4 + n ] = 0.f;
+                o[ img + 4 + r * o4 + n ] = 0.f;
     }
 }
 

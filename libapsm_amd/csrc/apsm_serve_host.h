@@ -548,7 +548,7 @@ bool serverLaunchTrainRound( apsm_server* S )
     std::map<std::pair<int, int>, std::vector<apsm::Seq2Desc>> seq;
     std::map<std::pair<int, int>, std::pair<int, size_t>> seqDim;
     std::vector<apsm::ThetaDesc> theta;
-    int maxU = 1;
+    int maxUL = 1;
     for ( auto it = S->training.begin(); it != S->training.end(); )
     {
         ServeFrame* f = *it;
@@ -562,7 +562,7 @@ bool serverLaunchTrainRound( apsm_server* S )
         if ( f->nextBlock == f->plan.blocks.size() )
         {
             theta.push_back( f->plan.theta );
-            maxU = std::max( maxU, f->plan.theta.U );
+            maxUL = std::max( maxUL, f->plan.theta.U * 2 * f->plan.theta.N );
             f->lastRound = rid;
             R.finishing.push_back( f );
             it = S->training.erase( it );
@@ -621,7 +621,7 @@ bool serverLaunchTrainRound( apsm_server* S )
     }
     if ( !theta.empty() )
     {
-        hipLaunchKernelGGL( apsm::batch_theta, dim3( maxU, (unsigned)theta.size() ), dim3( 256 ), 0, st,
+        hipLaunchKernelGGL( apsm::batch_theta, dim3( maxUL, (unsigned)theta.size() ), dim3( 256 ), 0, st,
                             (const apsm::ThetaDesc*)( base + thetaOff ) );
         HIP_OR_THROW( hipGetLastError() );
     }
