@@ -103,8 +103,11 @@ __device__ __forceinline__ void unrollFor( F f )
 // load( n ) is antenna n of this lane's sample (zero for none), finish( fa, fb ) takes every user's sums
 // of the lane half h (the two halves of a wave hold disjoint entries of the same samples and are
 // not yet added). MASK: entries below first( j0 ), counted within the tile from j0, do not count.
-// WAVES: waves per workgroup; ETILE: dictionary entries per LDS tile (0: mfmaTileOf).
-template <int NMAX, int UMAX, int PREC, int WAVES, int ETILE, bool MASK, class LOAD, class FIRST, class FINISH>
+// WAVES: waves per workgroup; ETILE: dictionary entries per LDS tile (0: mfmaTileOf). PARTS > 1: the
+// entries of a tile (32 PARTS) are shared out over PARTS waves of the same samples, wave w taking block
+// w % PARTS, and finish is called for the first of them with the parts added in order. ORDER > 1: a wave
+// takes all entries and keeps the sums of blocks b % ORDER apart, which gives the bits of PARTS = ORDER.
+template <int NMAX, int UMAX, int PREC, int WAVES, int ETILE, bool MASK, int PARTS, int ORDER, class LOAD, class FIRST, class FINISH>
 __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const float* __restrict__ Zn, const float* __restrict__ C,
                                               int64_t ldC, int64_t G, int U, float g2, int N, LOAD load, FIRST first, FINISH finish )
 {
@@ -116,6 +119,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     constexpr int kAllQuads = K16 / 4 * kTile, kQuads = ( kAllQuads + kThreads - 1 ) / kThreads; // groups of four components staged per thread
     constexpr int kCLoads = ( UMAX * kTile + kThreads - 1 ) / kThreads;
     static_assert( kTile <= kThreads && kTile % 32 == 0, "staging shape" );
+    static_assert( PARTS == 1 || ( kTile == 32 * PARTS && WAVES % PARTS == 0 && !MASK ), "one block per wave and tile" );
     typedef typename MfmaIn<PREC>::V V;
     typedef uint32_t u32x4 __attribute__( ( ext_vector_type( 4 ) ) );
     // two tile buffers: the next tile's loads are in flight (in registers) while the current tile
@@ -221,10 +225,12 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     float k2 = 2.f * g2, k2n = -2.f * g2;
     asm( "" : "+v"( k2 ), "+v"( k2n ) );
 
-    float fa[ UMAX ], fb[ UMAX ];
+    float fa[ ORDER ][ UMAX ], fb[ ORDER ][ UMAX ];
 #pragma unroll
-    for ( int u = 0; u < UMAX; u++ )
-        fa[ u ] = fb[ u ] = 0.f;
+    for ( int o = 0; o < ORDER; o++ )
+#pragma unroll
+        for ( int u = 0; u < UMAX; u++ )
+            fa[ o ][ u ] = fb[ o ][ u ] = 0.f;
 
     // tile loads into registers (zeros past the dictionary end, past N and past K): components k to k + 3
     // of entry e, r * kThreads + tid = e * K16/4 + k/4. With N == NMAX rows have no gaps: one 16-byte load.
@@ -341,8 +347,8 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     // coefficient slot `slot`), between them the products of the next block (entries cbn of buffer
     // bufn) into the other set. The fences keep the two streams interleaved entry by entry.
     constexpr int PF = UMAX <= 2 ? 4 : 1; // entries whose coefficients are read ahead together
-    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, int rel = 0 ) {
-        constexpr int d = dC;
+    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, auto oC, int rel = 0 ) {
+        constexpr int d = dC, ord = oC;
         float2 co[ 2 ][ PF * UMAX ];
         float4 zq[ 2 ];
         auto entryOf = [ & ]( int i ) { return cb + 8 * ( i / 4 ) + 4 * h + i % 4; }; // the lane's entry i within the tile
@@ -379,9 +385,9 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
             for ( int u = 0; u < UMAX; u++ )
             {
                 const float2 c = co[ i / PF & 1 ][ i % PF * UMAX + u ];
-                fa[ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ u ] ) );
-                fb[ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ u ] ) );
-                asm volatile( "" : "+v"( fa[ u ] ), "+v"( fb[ u ] )::"memory" );
+                fa[ ord ][ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ ord ][ u ] ) );
+                fb[ ord ][ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ ord ][ u ] ) );
+                asm volatile( "" : "+v"( fa[ ord ][ u ] ), "+v"( fb[ ord ][ u ] )::"memory" );
             }
             __builtin_amdgcn_sched_barrier( 0 );
         } );
@@ -390,7 +396,8 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     // Tile tt + 1 is stored between two barriers' reach: its rows (two buffers) replace those of tile
     // tt - 1, last read before the previous barrier, its norms and coefficients (three) those of tile
     // tt - 2, as the last block of a tile is contracted after the barrier.
-    constexpr int kBlocks = kTile / 32;
+    constexpr int kBlocks = kTile / 32 / PARTS;
+    const int cw = PARTS > 1 ? 32 * ( ( threadIdx.x >> 6 ) % PARTS ) : 0; // the wave's block of a shared-out tile
     typedef std::integral_constant<int, 0> D0;
     typedef std::integral_constant<int, 1> D1;
     const int nTiles = (int)( ( G + kTile - 1 ) / kTile );
@@ -407,7 +414,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         unrollFor<kProducts>( [ & ]( auto kC ) { product( buf, cb, D0 {}, kC ); } );
     };
     if ( PIPE && nTiles > 0 )
-        products( 0, 0 );
+        products( 0, cw );
     auto advance = [ & ]( int tt ) {
         if ( tt + 1 < nTiles )
             storeTile( tt + 1 );
@@ -416,69 +423,112 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         __syncthreads();
     };
     // (the products past the last block read what the buffers hold, and are not used)
+    static_assert( ORDER == 1 || ( !MASK && PARTS == 1 && ( kBlocks == 1 || ORDER % kBlocks == 0 ) ), "whole turns of the sums" );
     if constexpr ( !PIPE )
     {
 #pragma unroll 1
-        for ( int tt = 0; tt < nTiles; tt++ )
-        {
+        for ( int t0 = 0; t0 < nTiles; t0 += ORDER )
+            unrollFor<ORDER>( [ & ]( auto iC ) {
+                const int tt = t0 + iC;
+                if ( tt >= nTiles )
+                    return;
 #pragma unroll 1
-            for ( int cb = 0; cb < kTile; cb += 32 )
-            {
-                if ( (int64_t)tt * kTile + cb >= G )
-                    break;
-                products( tt & 1, cb );
-                phase( tt % 3, cb, 0, 0, D0 {}, MASK ? first( (int64_t)tt * kTile ) : 0 );
-            }
-            advance( tt );
-        }
+                for ( int cb = cw; cb < kTile; cb += 32 * PARTS )
+                {
+                    if ( (int64_t)tt * kTile + cb >= G )
+                        break;
+                    products( tt & 1, cb );
+                    phase( tt % 3, cb, 0, 0, D0 {}, iC, MASK ? first( (int64_t)tt * kTile ) : 0 );
+                }
+                advance( tt );
+            } );
     }
     else if constexpr ( kBlocks == 1 )
     {
+        constexpr int STEP = ORDER > 2 ? ORDER : 2;
 #pragma unroll 1
-        for ( int tt = 0; tt < nTiles; tt += 2 )
-        {
-            advance( tt );
-            phase( tt % 3, 0, ( tt + 1 ) & 1, 0, D0 {} );
-            if ( tt + 1 < nTiles )
-            {
-                advance( tt + 1 );
-                phase( ( tt + 1 ) % 3, 0, tt & 1, 0, D1 {} );
-            }
-        }
+        for ( int t0 = 0; t0 < nTiles; t0 += STEP )
+            unrollFor<STEP>( [ & ]( auto iC ) {
+                const int tt = t0 + iC;
+                if ( tt >= nTiles )
+                    return;
+                advance( tt );
+                phase( tt % 3, cw, ( tt + 1 ) & 1, cw, std::integral_constant<int, iC & 1> {}, std::integral_constant<int, iC % ORDER> {} );
+            } );
     }
     else
     {
+        constexpr int STEP = ORDER > kBlocks ? ORDER / kBlocks : 1;
 #pragma unroll 1
-        for ( int tt = 0; tt < nTiles; tt++ )
-        {
-#pragma unroll
-            for ( int b = 0; b + 2 < kBlocks; b += 2 )
-            {
-                phase( tt % 3, 32 * b, tt & 1, 32 * b + 32, D0 {} );
-                phase( tt % 3, 32 * b + 32, tt & 1, 32 * b + 64, D1 {} );
-            }
-            phase( tt % 3, kTile - 64, tt & 1, kTile - 32, D0 {} );
-            advance( tt );
-            phase( tt % 3, kTile - 32, ( tt + 1 ) & 1, 0, D1 {} );
-        }
+        for ( int t0 = 0; t0 < nTiles; t0 += STEP )
+            unrollFor<STEP>( [ & ]( auto iC ) {
+                const int tt = t0 + iC;
+                if ( tt >= nTiles )
+                    return;
+                unrollFor<kBlocks>( [ & ]( auto bC ) {
+                    constexpr int b = bC, last = b == kBlocks - 1;
+                    if constexpr ( last )
+                        advance( tt );
+                    phase( tt % 3, 32 * b, ( tt + last ) & 1, last ? 0 : 32 * b + 32, std::integral_constant<int, b & 1> {},
+                           std::integral_constant<int, ( iC * kBlocks + b ) % ORDER> {} );
+                } );
+            } );
     }
     __syncthreads(); // a following tile stores over what other waves may still read
 
-    finish( fa, fb );
+    if constexpr ( PARTS > 1 )
+    {
+        const int wave = tid >> 6, part = wave % PARTS;
+        constexpr int kRed = WAVES / PARTS * ( PARTS - 1 ) * UMAX * 64;
+        constexpr bool inTile = sizeof( sZ ) >= kRed * sizeof( float2 );
+        __shared__ float2 sRed[ inTile ? 1 : kRed ];
+        float2* red = ( inTile ? reinterpret_cast<float2*>( sZ ) : sRed ) + wave / PARTS * ( PARTS - 1 ) * UMAX * 64 + lane;
+        if ( part > 0 )
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
+                red[ ( ( part - 1 ) * UMAX + u ) * 64 ] = make_float2( fa[ 0 ][ u ], fb[ 0 ][ u ] );
+        __syncthreads();
+        if ( part == 0 )
+        {
+#pragma unroll
+            for ( int k = 0; k < PARTS - 1; k++ )
+#pragma unroll
+                for ( int u = 0; u < UMAX; u++ )
+                {
+                    const float2 v = red[ ( k * UMAX + u ) * 64 ];
+                    fa[ 0 ][ u ] += v.x;
+                    fb[ 0 ][ u ] += v.y;
+                }
+            finish( fa[ 0 ], fb[ 0 ] );
+        }
+        __syncthreads(); // a following tile stores over what was read
+    }
+    else
+    {
+#pragma unroll
+        for ( int o = 1; o < ORDER; o++ )
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
+            {
+                fa[ 0 ][ u ] += fa[ o ][ u ];
+                fb[ 0 ][ u ] += fb[ o ][ u ];
+            }
+        finish( fa[ 0 ], fb[ 0 ] );
+    }
 }
 
-// One tile of 32 * WAVES data samples of a detect.
-template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0>
+// One tile of 32 * WAVES / PARTS data samples of a detect.
+template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0, int PARTS = 1, int ORDER = 1>
 __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
                                                 const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
                                                 const float* __restrict__ theta, int64_t G, int U, float wL, float wG, float g2,
                                                 float* __restrict__ est, int N, const int64_t tile )
 {
     const int h = ( threadIdx.x >> 5 ) & 1;
-    const int64_t m = tile * ( 32 * WAVES ) + ( threadIdx.x >> 6 ) * 32 + ( threadIdx.x & 31 ); // this lane's sample
+    const int64_t m = tile * ( 32 * WAVES / PARTS ) + ( threadIdx.x >> 6 ) / PARTS * 32 + ( threadIdx.x & 31 ); // this lane's sample
     const bool valid = m < M;
     const float2* x = reinterpret_cast<const float2*>( rx ) + m;
-    gaussianMfma<NMAX, UMAX, PREC, WAVES, ETILE, false>(
+    gaussianMfma<NMAX, UMAX, PREC, WAVES, ETILE, false, PARTS, ORDER>(
         Z, Zn, C, ldC, G, U, g2, N, [ & ]( int n ) { return valid && n < N ? x[ (int64_t)n * M ] : make_float2( 0.f, 0.f ); },
         []( int64_t ) { return 0; },
         [ & ]( float( &fa )[ UMAX ], float( &fb )[ UMAX ] ) {

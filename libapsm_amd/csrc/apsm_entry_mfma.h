@@ -40,7 +40,7 @@ __device__ __forceinline__ void entryChunkMfma( const float* __restrict__ Z, con
     const int64_t c1 = j1 - (int64_t)chunk * kEntryChunk;
     const int64_t c0 = ( c1 - kEntryChunk ) > jBeg ? c1 - kEntryChunk : jBeg;
     const float* x = Z + tc * L;
-    gaussianMfma<NMAX, UMAX, PREC_F32, kMfmaThreads / 64, 0, true>(
+    gaussianMfma<NMAX, UMAX, PREC_F32, kMfmaThreads / 64, 0, true, 1, 1>(
         Z + c0 * L, Zn + c0, C + 2 * c0, a.ldYC, c1 - c0, a.U, a.g2, N,
         [ & ]( int n ) { return valid && n < N ? make_float2( x[ n ], x[ N + n ] ) : make_float2( 0.f, 0.f ); },
         [ & ]( int64_t j0 ) { // entries of the tile from j0 that the FIFO dropped before this lane's sample entered

@@ -62,3 +62,27 @@ def test_tile_edges(require_gpu, mode, N, G):
 @pytest.mark.parametrize("N,users", [(5, 2), (8, 3), (16, 5), (32, 8), (64, 10), (21, 16), (8, 9), (16, 13)])
 def test_samples_and_user_groups(require_gpu, M, N, users):
     check("fp32-matrix", N, 70, M, users)
+
+
+@pytest.mark.parametrize("M", [16384, 16385])
+@pytest.mark.parametrize("N,G,users", [(3, 1, 1), (8, 33, 3), (16, 97, 1), (32, 130, 2), (64, 65, 1), (13, 200, 10)])
+def test_around_the_parts_rule(require_gpu, M, N, G, users):
+    """The last call whose dictionary entries are shared out over waves, and the first that is not."""
+    check("fp32-matrix", N, G, M, users)
+
+
+def test_batch_by_parts_equals_single_handles(require_gpu):
+    """Calls by parts: a batch keeps the parts' sums apart in one wave (up to 4 users) or shares them out."""
+    from libapsm_amd import ApsmBatch, ApsmNomaDetectorFactory
+    shapes = [(2, 1, 40, 70), (8, 1, 200, 300), (16, 3, 150, 64), (30, 9, 260, 129), (32, 4, 33, 31), (64, 2, 100, 257), (64, 12, 70, 65),
+              (16, 1, 90, 17000)]
+    data = [small_problem(N=N, U=max(U, 3), T=T, M=M, seed=N + U) for N, U, T, M in shapes]
+    cfgs = [dict(windowSize=10, dictionarySize=T, eB=0.01, gaussianKernelVariance=0.5) for _, _, T, _ in shapes]
+    b = ApsmBatch(cfgs, [s[0] for s in shapes], [s[1] for s in shapes])
+    b.plan([d["rx_train"] for d in data], [d["tx_train"][:s[1]] for d, s in zip(data, shapes)], [d["rx_data"] for d in data])
+    b.synchronize()
+    for i, ((N, U, T, M), d, cfg) in enumerate(zip(shapes, data, cfgs)):
+        print(f"instance {i}: N {N} users {U} T {T} M {M}", flush=True)
+        det = ApsmNomaDetectorFactory.build(dict(cfg, otype="APSM"), N, U)
+        det.train(d["rx_train"], d["tx_train"][:U] if U > 1 else d["tx_train"][0])
+        np.testing.assert_array_equal(np.atleast_2d(b.estimates(i)), np.atleast_2d(det.detect(d["rx_data"])).astype(np.complex64))
