@@ -14,15 +14,6 @@
 
 namespace apsm {
 
-struct StageDesc
-{
-    const float *rx, *tx;
-    float *Z, *Zn, *Y, *C;
-    int64_t S, ldYC;
-    int N, U;
-};
-
-
 struct Seq2Desc
 {
     const float *Z, *Zn, *Y;
@@ -39,10 +30,9 @@ struct ThetaDesc
     int N, U;
 };
 
-__global__ void batch_stage( const StageDesc* __restrict__ d )
+__global__ void __launch_bounds__( kStageThreads ) batch_stage( const StageDesc* __restrict__ d )
 {
-    const StageDesc& s = d[ blockIdx.y ];
-    stagePilotsBody( s.rx, s.tx, nullptr, s.N, s.U, s.S, s.Z, s.Zn, s.Y, s.C, s.ldYC, (int64_t)blockIdx.x * blockDim.x + threadIdx.x );
+    stagePilotsBody( d[ blockIdx.y ], nullptr, blockIdx.x );
 }
 
 template <int TP, int NEWPER, int PMAX>

@@ -294,9 +294,9 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
                      } } );
     {
         const size_t off = arena.add( stage );
-        const int ns = (int)stage.size(), gx = gridFor( maxS, 256 );
+        const int ns = (int)stage.size(), gx = gridFor( maxS, apsm::kStagePilots );
         pend.push_back( { 0, [ = ]( const char* base ) {
-                             hipLaunchKernelGGL( apsm::batch_stage, dim3( gx, ns ), dim3( 256 ), 0, B->stream,
+                             hipLaunchKernelGGL( apsm::batch_stage, dim3( gx, ns ), dim3( apsm::kStageThreads ), 0, B->stream,
                                                  (const apsm::StageDesc*)( base + off ) );
                              HIP_OR_THROW( hipGetLastError() );
                          } } );

@@ -852,19 +852,6 @@ void trainDev( apsm_handle* h, const float* d_rx, const float* d_tx, int64_t T, 
     const int64_t K = nOld + T;
     nb.ensure( K, N, U );
     const int64_t ld = 2 * nb.capK;
-    if ( nOld > 0 )
-    {
-        StreamBuf& ob = h->buf[ h->cur ];
-        const int64_t off = usedC - nOld - h->bufBaseC;
-        const int64_t ldOld = 2 * ob.capK;
-        HIP_OR_THROW( hipMemcpyAsync( nb.Z.ptr, ob.Z.ptr + off * L, (size_t)nOld * L * sizeof( float ), hipMemcpyDeviceToDevice,
-                                      h->stream ) );
-        HIP_OR_THROW( hipMemcpyAsync( nb.Zn.ptr, ob.Zn.ptr + off, (size_t)nOld * sizeof( float ), hipMemcpyDeviceToDevice, h->stream ) );
-        HIP_OR_THROW( hipMemcpy2DAsync( nb.Y.ptr, ld * sizeof( float ), ob.Y.ptr + 2 * off, ldOld * sizeof( float ),
-                                        2 * nOld * sizeof( float ), U, hipMemcpyDeviceToDevice, h->stream ) );
-        HIP_OR_THROW( hipMemcpy2DAsync( nb.C.ptr, ld * sizeof( float ), ob.C.ptr + 2 * off, ldOld * sizeof( float ),
-                                        2 * nOld * sizeof( float ), U, hipMemcpyDeviceToDevice, h->stream ) );
-    }
     const int32_t* dPerm = nullptr;
     if ( shuffle )
     {
@@ -872,8 +859,19 @@ void trainDev( apsm_handle* h, const float* d_rx, const float* d_tx, int64_t T, 
         HIP_OR_THROW( hipMemcpyAsync( h->perm.ptr, perm.data(), T * sizeof( int32_t ), hipMemcpyHostToDevice, h->stream ) );
         dPerm = h->perm.ptr;
     }
-    hipLaunchKernelGGL( apsm::stage_pilots, dim3( gridFor( T, 256 ) ), dim3( 256 ), 0, h->stream, d_rx, d_tx, dPerm, N, U, T,
-                        nb.Z.ptr + nOld * L, nb.Zn.ptr + nOld, nb.Y.ptr + 2 * nOld, nb.C.ptr + 2 * nOld, ld );
+    apsm::KeepDesc keep {};
+    if ( nOld > 0 )
+    {
+        const StreamBuf& ob = h->buf[ h->cur ];
+        const int64_t off = usedC - nOld - h->bufBaseC;
+        keep = { ob.Z.ptr + off * L, ob.Zn.ptr + off, ob.Y.ptr + 2 * off, ob.C.ptr + 2 * off, nb.Z.ptr, nb.Zn.ptr, nb.Y.ptr, nb.C.ptr, nOld,
+                 2 * ob.capK, ld };
+    }
+    const int stageWg = std::max( gridFor( T, apsm::kStagePilots ), gridFor( nOld * L, apsm::kKeepWg ) );
+    hipLaunchKernelGGL( apsm::stage_call, dim3( stageWg, nOld > 0 ? 3 + 2 * U : 1 ), dim3( apsm::kStageThreads ), 0, h->stream,
+                        apsm::StageDesc { d_rx, d_tx, nb.Z.ptr + nOld * L, nb.Zn.ptr + nOld, nb.Y.ptr + 2 * nOld, nb.C.ptr + 2 * nOld, T, ld,
+                                          N, U },
+                        dPerm, keep );
     HIP_OR_THROW( hipGetLastError() );
 
     apsm::SeqArgs a {};

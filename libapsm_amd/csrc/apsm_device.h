@@ -30,38 +30,107 @@ namespace apsm {
 // Staging: host layout rx [N][S][2] (+ optional permutation) -> stream rows Z [S][2N] and
 // norms; tx [U][S][2] -> Y [U][2S]; C of the new rows cleared.
 // ---------------------------------------------------------------------------------------
-__device__ __forceinline__ void stagePilotsBody( const float* __restrict__ rx, const float* __restrict__ tx, const int32_t* __restrict__ perm,
-                                                 int N, int U, int64_t S, float* __restrict__ Z, float* __restrict__ Zn,
-                                                 float* __restrict__ Y, float* __restrict__ C, int64_t ldYC, const int64_t k )
+// One workgroup per 64 pilots, through LDS: reads run along the pilots, writes along the rows (a
+// thread per pilot wrote 4 bytes of every row it touched, with one load in flight).
+constexpr int kStageThreads = 256, kStagePilots = 64;
+struct StageDesc
 {
-    if ( k >= S )
+    const float *rx, *tx;
+    float *Z, *Zn, *Y, *C;
+    int64_t S, ldYC;
+    int N, U;
+};
+__device__ __forceinline__ void stagePilotsBody( const StageDesc& s, const int32_t* __restrict__ perm, const int64_t wg )
+{
+    __shared__ float tile[ kStagePilots * 129 ]; // [pilot][2N + 1]
+    const int64_t k0 = wg * kStagePilots;
+    if ( k0 >= s.S )
         return;
-    const int64_t src = perm ? perm[ k ] : k;
-    const int L = 2 * N;
-    float nrm = 0.f;
-    for ( int n = 0; n < N; n++ )
+    const int nk = s.S - k0 < kStagePilots ? (int)( s.S - k0 ) : kStagePilots;
+    const int N = s.N, L = 2 * N, ld = L + 1;
+    const int k = threadIdx.x % kStagePilots, part = threadIdx.x / kStagePilots;
+    constexpr int kParts = kStageThreads / kStagePilots;
+    if ( k < nk )
     {
-        float2 v = reinterpret_cast<const float2*>( rx )[ (int64_t)n * S + src ];
-        Z[ k * L + n ] = v.x;
-        Z[ k * L + N + n ] = v.y;
-        nrm += v.x * v.x + v.y * v.y;
+        const int64_t src = perm ? perm[ k0 + k ] : k0 + k;
+        const float2* x = reinterpret_cast<const float2*>( s.rx ) + src;
+#pragma unroll 8
+        for ( int n = part; n < N; n += kParts )
+        {
+            const float2 v = x[ (int64_t)n * s.S ];
+            tile[ k * ld + n ] = v.x;
+            tile[ k * ld + N + n ] = v.y;
+        }
+#pragma unroll 2
+        for ( int u = part; u < s.U; u += kParts )
+        {
+            reinterpret_cast<float2*>( s.Y + u * s.ldYC )[ k0 + k ] = reinterpret_cast<const float2*>( s.tx )[ u * s.S + src ];
+            reinterpret_cast<float2*>( s.C + u * s.ldYC )[ k0 + k ] = make_float2( 0.f, 0.f );
+        }
     }
-    Zn[ k ] = nrm;
-    for ( int u = 0; u < U; u++ )
+    __syncthreads();
+    float* z = s.Z + k0 * L;
+    for ( int i = threadIdx.x; i < nk * L; i += kStageThreads )
+        z[ i ] = tile[ i / L * ld + i % L ];
+    if ( (int)threadIdx.x < nk )
     {
-        float2 t = reinterpret_cast<const float2*>( tx )[ (int64_t)u * S + src ];
-        Y[ u * ldYC + 2 * k ] = t.x;
-        Y[ u * ldYC + 2 * k + 1 ] = t.y;
-        C[ u * ldYC + 2 * k ] = 0.f;
-        C[ u * ldYC + 2 * k + 1 ] = 0.f;
+        float nrm = 0.f;
+        for ( int n = 0; n < N; n++ )
+        {
+            const float re = tile[ threadIdx.x * ld + n ], im = tile[ threadIdx.x * ld + N + n ];
+            nrm += re * re + im * im;
+        }
+        s.Zn[ k0 + threadIdx.x ] = nrm;
     }
 }
 
-__global__ void stage_pilots( const float* __restrict__ rx, const float* __restrict__ tx, const int32_t* __restrict__ perm, int N, int U,
-                              int64_t S, float* __restrict__ Z, float* __restrict__ Zn, float* __restrict__ Y, float* __restrict__ C,
-                              int64_t ldYC )
+// A train call's stream rows in one launch: row y = 0 of the grid stages the new pilots, rows 1 to 2 + 2 U
+// copy what is kept of the previous buffer (Z, Zn, then Y and C of every user), kKeepWg floats
+// per workgroup. Four copies and the staging took a launch each.
+constexpr int kKeepWg = 8 * kStageThreads;
+struct KeepDesc
 {
-    stagePilotsBody( rx, tx, perm, N, U, S, Z, Zn, Y, C, ldYC, (int64_t)blockIdx.x * blockDim.x + threadIdx.x );
+    const float *Z, *Zn, *Y, *C; // first kept row
+    float *Zd, *Znd, *Yd, *Cd;
+    int64_t n, ldSrc, ldDst; // complex rows kept; strides of Y and C
+};
+__global__ void __launch_bounds__( kStageThreads ) stage_call( const StageDesc s, const int32_t* __restrict__ perm, const KeepDesc d )
+{
+    if ( blockIdx.y == 0 )
+    {
+        stagePilotsBody( s, perm, blockIdx.x );
+        return;
+    }
+    const int r = (int)blockIdx.y - 1, u = ( r - 2 ) >> 1;
+    const float* src;
+    float* dst;
+    int64_t n = 2 * d.n;
+    if ( r == 0 )
+    {
+        src = d.Z;
+        dst = d.Zd;
+        n = d.n * 2 * s.N;
+    }
+    else if ( r == 1 )
+    {
+        src = d.Zn;
+        dst = d.Znd;
+        n = d.n;
+    }
+    else
+    {
+        src = ( r & 1 ? d.C : d.Y ) + u * d.ldSrc;
+        dst = ( r & 1 ? d.Cd : d.Yd ) + u * d.ldDst;
+    }
+    const int64_t i0 = (int64_t)blockIdx.x * kKeepWg + threadIdx.x;
+    float v[ 8 ];
+#pragma unroll
+    for ( int e = 0; e < 8; e++ )
+        v[ e ] = i0 + e * kStageThreads < n ? src[ i0 + e * kStageThreads ] : 0.f;
+#pragma unroll
+    for ( int e = 0; e < 8; e++ )
+        if ( i0 + e * kStageThreads < n )
+            dst[ i0 + e * kStageThreads ] = v[ e ];
 }
 
 // ---------------------------------------------------------------------------------------

@@ -599,7 +599,7 @@ bool serverLaunchTrainRound( apsm_server* S )
     }
     if ( !stage.empty() )
     {
-        hipLaunchKernelGGL( apsm::batch_stage, dim3( gridFor( maxS, 256 ), (unsigned)stage.size() ), dim3( 256 ), 0, st,
+        hipLaunchKernelGGL( apsm::batch_stage, dim3( gridFor( maxS, apsm::kStagePilots ), (unsigned)stage.size() ), dim3( apsm::kStageThreads ), 0, st,
                             (const apsm::StageDesc*)( base + stageOff ) );
         HIP_OR_THROW( hipGetLastError() );
     }

@@ -51,3 +51,24 @@ def test_dictionary_near_the_window(require_gpu, oracle, w, dict_size):
 def test_short_and_cut_streams(require_gpu, oracle, w, T, cuts):
     cfg = dict(windowSize=w, dictionarySize=max(w, T // 2), eB=0.01, gaussianKernelVariance=0.1)
     run(oracle, 5, T, cfg, cuts, users=2, seed=T)
+
+
+@pytest.mark.parametrize("N,T,cuts,users", [(1, 129, [64], 1), (16, 200, [63, 65, 130], 3), (21, 300, [128, 257], 2), (64, 260, [1, 65, 193], 1),
+                                            (33, 400, [70, 320], 5)])
+def test_calls_around_the_staging_tiles(require_gpu, oracle, N, T, cuts, users):
+    """Pilots are staged 64 to a workgroup and kept rows copied 2048 floats to a workgroup."""
+    cfg = dict(windowSize=8, dictionarySize=100, eB=0.01, gaussianKernelVariance=0.5)
+    from libapsm_amd import ApsmNomaDetectorFactory
+    d = small_problem(N=N, U=max(users, 3), T=T, M=65, seed=T)
+    det = ApsmNomaDetectorFactory.build(dict(cfg, otype="APSM"), N, users)
+    for a, b in zip([0] + cuts, cuts + [T]):
+        det.train(d["rx_train"][:, a:b], d["tx_train"][:users, a:b])
+    est = np.atleast_2d(det.detect(d["rx_data"]))
+    st = det.getTrainingState()
+    for u in range(users):
+        o = oracle.Apsm(cfg, N)
+        o.train(d["rx_train"], d["tx_train"][u], incremental=True)
+        e = np.abs(to_ri(est[u]) - o.detect(d["rx_data"])).max()
+        c = np.abs(st["coeffs"][u] - o.state()["coeffs"]).max()
+        print(f"N {N} T {T} cuts {cuts} user {u}: soft {e:.2e} coeffs {c:.2e}", flush=True)
+        assert e <= ATOL and c <= ATOL
