@@ -339,6 +339,7 @@ struct apsm_handle
     DevBuf<double> Qn; // norm-constraint path: c^T K c per user
     DevBuf<float> rx, tx, est; // staging for the host entry points
     DevBuf<int32_t> perm;
+    DevBuf<unsigned long long> varHist; // variance heuristic: state and histogram
     lls_handle* lls = nullptr;
     // per-kernel profile (apsm_profile_*): event pairs bracketing launches of a kind
     bool prof = false;
@@ -744,44 +745,36 @@ void trainBlocked( apsm_handle* h, const StreamBuf& b, int64_t usedOld, int64_t 
 // on the device: the k-th smallest pair distance by a three-pass radix select, k as the
 // reference indexes its sorted vector (size * 0.7f in float). The set of pair distances does
 // not depend on the pilot order, so the training shuffle does not enter.
-float varianceHeuristicDevice( hipStream_t stream, const float* d_rx, int N, int64_t T )
+float varianceHeuristicDevice( hipStream_t stream, const float* d_rx, int N, int64_t T, DevBuf<unsigned long long>& buf )
 {
     ARG_CHECK( T >= 2, "variance heuristic needs at least two pilots" );
     const uint64_t P = (uint64_t)T * (uint64_t)( T - 1 ) / 2;
     uint64_t k = (uint64_t)( (float)P * 0.7f );
     if ( k >= P )
         k = P - 1;
-    DevBuf<unsigned long long> hist;
-    hist.ensure( apsm::kVhBins );
-    std::vector<unsigned long long> hh( apsm::kVhBins );
+    static_assert( sizeof( apsm::VhState ) == 2 * sizeof( unsigned long long ), "state before the histogram" );
+    buf.ensure( 2 + apsm::kVhBins );
+    apsm::VhState* state = reinterpret_cast<apsm::VhState*>( buf.ptr );
+    unsigned long long* hist = buf.ptr + 2;
     const int tiles = gridFor( T, apsm::kVhTile );
     ARG_CHECK( tiles <= 65535, "too many pilots for the variance heuristic" );
     const size_t lds = 2 * (size_t)N * apsm::kVhTile * sizeof( float2 );
-    uint32_t prefix = 0;
+    HIP_OR_THROW( hipMemsetAsync( buf.ptr, 0, ( 2 + apsm::kVhBins ) * sizeof( unsigned long long ), stream ) );
     for ( int pass = 0; pass < 3; pass++ )
     {
-        HIP_OR_THROW( hipMemsetAsync( hist.ptr, 0, apsm::kVhBins * sizeof( unsigned long long ), stream ) );
         hipLaunchKernelGGL( apsm::apsm_variance_histogram, dim3( tiles, tiles ), dim3( apsm::kVhThreads ), lds, stream, d_rx, N, T, pass,
-                            prefix, hist.ptr );
+                            state, hist );
         HIP_OR_THROW( hipGetLastError() );
-        HIP_OR_THROW( hipMemcpyAsync( hh.data(), hist.ptr, apsm::kVhBins * sizeof( unsigned long long ), hipMemcpyDeviceToHost, stream ) );
-        HIP_OR_THROW( hipStreamSynchronize( stream ) );
-        const int nb = pass == 2 ? 256 : apsm::kVhBins;
-        uint64_t cum = 0;
-        int b = 0;
-        for ( ; b < nb; b++ )
-        {
-            if ( cum + hh[ b ] > k )
-                break;
-            cum += hh[ b ];
-        }
-        if ( b == nb )
-            throw ApsmError { APSM_ERR_NUMERIC, "variance heuristic: percentile not found" };
-        k -= cum;
-        prefix = pass == 0 ? (uint32_t)b : ( prefix << ( pass == 1 ? 12 : 8 ) ) | (uint32_t)b;
+        hipLaunchKernelGGL( apsm::apsm_variance_select, dim3( 1 ), dim3( apsm::kVhSelectThreads ), 0, stream, hist, state, pass, k );
+        HIP_OR_THROW( hipGetLastError() );
     }
+    apsm::VhState found;
+    HIP_OR_THROW( hipMemcpyAsync( &found, state, sizeof( found ), hipMemcpyDeviceToHost, stream ) );
+    HIP_OR_THROW( hipStreamSynchronize( stream ) );
+    if ( found.found != 3 )
+        throw ApsmError { APSM_ERR_NUMERIC, "variance heuristic: percentile not found" };
     float value;
-    std::memcpy( &value, &prefix, sizeof( value ) );
+    std::memcpy( &value, &found.prefix, sizeof( value ) );
     // float element times a double power, rounded to float, then squared in float
     const float v = (float)( (double)value * std::pow( (double)T, -1. / 5. ) );
     return v * v;
@@ -798,7 +791,7 @@ void trainPrepare( apsm_handle* h, const float* d_rx, const float* d_tx, int64_t
         if ( p.gaussian_kernel_variance != 0.f )
             h->var = p.gaussian_kernel_variance * (float)( N * N );
         else
-            h->var = varianceHeuristicDevice( h->stream, d_rx, N, T );
+            h->var = varianceHeuristicDevice( h->stream, d_rx, N, T, h->varHist );
         h->varSet = true;
     }
     const float wL = p.linear_kernel_weight;

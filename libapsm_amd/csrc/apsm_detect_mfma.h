@@ -399,7 +399,6 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     constexpr int kBlocks = kTile / 32 / PARTS;
     const int cw = PARTS > 1 ? 32 * ( ( threadIdx.x >> 6 ) % PARTS ) : 0; // the wave's block of a shared-out tile
     typedef std::integral_constant<int, 0> D0;
-    typedef std::integral_constant<int, 1> D1;
     const int nTiles = (int)( ( G + kTile - 1 ) / kTile );
     if ( nTiles > 0 )
     {
