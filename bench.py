@@ -30,12 +30,12 @@ PEAK_FP32_TFLOPS = 157.3
 # HBM bytes of one train call of a workload (all its dispatches: sequencer, block precompute,
 # combine, staging, theta), from two rocprofv3 --pmc passes over `bench.py --steps 1 --warmup 0
 # --no-cpu-baseline --no-lls --no-batched --no-mixed --no-serving --no-small`: FETCH_SIZE
-# 6 603 568 KiB x 2.000 (a 1 GiB device copy, `bench.py --only copy`, reads 524 315 KiB of
-# FETCH_SIZE) + WRITE_SIZE 4 593 643 KiB x 1.000 (the copy reads 1 048 576 KiB).
-TRAIN_HBM_BYTES = {"plain-16ant-16qam": (6603568 * 2.000 + 4593643 * 1.000) * 1024}
-# HBM bytes of one apsm_train_seq2 launch, from the same calibrated passes restricted to the
-# sequencer kernel: FETCH_SIZE 8 717.1 KiB x 2.000 + WRITE_SIZE 53.7 KiB x 1.000 per dispatch.
-SEQ_HBM_BYTES_PER_LAUNCH = {"plain-16ant-16qam": (8717.1 * 2.000 + 53.7 * 1.000) * 1024}
+# 7 157 311 KiB x 2.000 (a 1 GiB device copy, `bench.py --only copy`, reads 524 315 KiB of
+# FETCH_SIZE) + WRITE_SIZE 4 759 622 KiB x 1.000 (the copy reads 1 048 576 KiB).
+TRAIN_HBM_BYTES = {"plain-16ant-16qam": (7157311 * 2.000 + 4759622 * 1.000) * 1024}
+# HBM bytes of one apsm_train_win launch, from the same calibrated passes restricted to the
+# sequencer kernel: FETCH_SIZE 8 597.9 KiB x 2.000 + WRITE_SIZE 226.8 KiB x 1.000 per dispatch.
+SEQ_HBM_BYTES_PER_LAUNCH = {"plain-16ant-16qam": (8597.9 * 2.000 + 226.8 * 1.000) * 1024}
 
 
 def parse():
@@ -660,7 +660,7 @@ def main():
     seq_tf = seq_flops / (seq_us * 1e-6) / 1e12
     cus = 256
     roofline = {"bound": f"fp32-valu latency chain, {U}/{cus} CUs (one workgroup per user, one projection step after another)",
-                "kernel": "apsm_train_seq2", "achieved": seq_tf, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
+                "kernel": "apsm_train_win", "achieved": seq_tf, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                 "frac": seq_tf / PEAK_FP32_TFLOPS,
                 "frac_of_occupied_cus": seq_tf / (PEAK_FP32_TFLOPS * U / cus),
                 "avg_launch_us": seq_us, "launches_per_step": seq_n / args.steps, "flops_per_launch": seq_flops,
@@ -670,12 +670,11 @@ def main():
                 "train_call_traffic": TRAIN_HBM_BYTES.get(args.workload),
                 "share_of_step": seq_ms / args.steps / ms_step}
     # per-step floor of the chain: the window-Gram product's vector-ALU issue on the busiest SIMD
-    # (4 TP FMA per thread, wave64 at 16 lanes per cycle, packed FP32 off) at 2.4 GHz
-    Wc = w["window"]
-    parts = 1024 // Wc
-    tp = -(-Wc // parts)
-    waves_per_simd = -(-(-(-parts * Wc // 64)) // 4)
-    floor_us = waves_per_simd * 4 * tp * 4 / 2.4e9 * 1e6
+    # (4 TP FMA per lane on ceil(4 TP / 16) waves, a wave64 FMA in 2 cycles at best, packed FP32 off)
+    # at 2.4 GHz
+    tp = next(t for t in (5, 10, 16, 20, 28, 40) if w["window"] <= 4 * t)
+    waves_per_simd = -(-(-(-4 * tp // 16)) // 4)
+    floor_us = waves_per_simd * 4 * tp * 2 / 2.4e9 * 1e6
     roofline["per_step_floor_us"] = floor_us
     roofline["frac_of_per_step_floor"] = floor_us / roofline["us_per_projection_step"]
     det_flops = M * G * (8.0 * N + 8.0 * U) + M * U * 8.0 * N
@@ -704,7 +703,7 @@ def main():
         "kernels_ms": {"train": tr_ms, "detect": dt_ms, "sequencer": seq_ms / args.steps,
                        "block_pre": pre_ms / args.steps},
         "secondary_rooflines": [
-            {"kernel": "apsm_detect_mfma<16,12,fp32>", "bound": "fp32 mfma cross terms + vector-ALU exp and contraction",
+            {"kernel": "apsm_detect_mfma<16,10,fp32>", "bound": "vector-ALU exp and contraction beside three-part bf16 mfma cross terms",
              "achieved": det_tf, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": det_tf / PEAK_FP32_TFLOPS,
              "avg_launch_us": det_us, "flops_per_launch": det_flops, "exp_per_s": 3.0 * M * G / (det_us * 1e-6)},
             {"kernel": "apsm_block_pre + apsm_entry_combine", "avg_launch_us": pre_us,

@@ -123,7 +123,7 @@ int apsm_kernel_times(apsm_handle* h, float* train_ms, float* detect_ms);
 /* Per-kernel device time of the handle's launches (no counterpart in the reference, whose
  * timer covers the whole train loop or detect kernel). While enabled, pairs of HIP events on
  * the handle's stream bracket every launch of the train sequencer (APSM_PROFILE_SEQUENCER,
- * apsm_train_seq2, one per train block), every block precompute (APSM_PROFILE_BLOCK_PRE: the
+ * apsm_train_win or apsm_train_seq2, one per train block), every block precompute (APSM_PROFILE_BLOCK_PRE: the
  * entry/Gram/eviction launch and the entry combine of a block) and every detect
  * (APSM_PROFILE_DETECT) of the blocked train path and the detect entry points.
  * apsm_profile_read waits for the recorded events and returns, per kind, the summed device

@@ -12,7 +12,8 @@
 //            A = kappa(a_t,a_j) = kappa(b_t,b_j), Bv = kappa(a_t,b_j), Cv = kappa(b_t,a_j).
 //   eviction shares    wG*sum_e c_e K(e,u) for the rows e leaving the dictionary at each
 //          step and the window rows u that were already in the window.
-//   apsm_train_seq2    one workgroup per user runs the block's steps: f of an entering row
+//   apsm_train_seq2    (two samples enter per step; apsm_train_win.h runs one per step)
+//          one workgroup per user runs the block's steps: f of an entering row
 //          is P_t + sum over active rows of c_j kappa(j,t); the sliding window Gram matrix
 //          lives in registers (complex-block form) and f, beta, c of the active rows in LDS,
 //          so a step touches global memory only through a prefetch of the next step's inputs.
@@ -44,8 +45,8 @@ __host__ __device__ constexpr int seq2PmaxOfTp( int tp )
 // and P with the eviction shares (2 * NEWPER + w2 floats, w2 <= 2 * TP * PMAX, copied in
 // 64-float chunks). Up to TP = 10 (at most 64 registers), rounded up to 256 floats, so that two
 // workgroups fit in a CU's LDS. Beyond, where the registers allow one workgroup per CU anyway,
-// the rows plus a whole kSeqThreads-float spare, in kSeqThreads units (3072 floats at TP = 27:
-// measured 1 % faster there than the tight 2048).
+// the rows plus a whole kSeqThreads-float spare, in kSeqThreads units (1 % faster at TP = 27
+// than tight buffers, measured with one sample entering per step).
 __host__ __device__ constexpr int seq2PkCap( int newPer, int tp, int pmax )
 {
     return tp <= 10 ? ( newPer * 3 * kActMax + ( ( 2 * newPer + 2 * tp * pmax + 63 ) & ~63 ) + 255 ) & ~255
@@ -210,7 +211,7 @@ __device__ __forceinline__ void seq2Body( const float* __restrict__ Z, const flo
                 int off = 0;
                 if ( e < NEWPER * rowFloats )
                 {
-                    const int i = NEWPER == 1 ? 0 : e / rowFloats;
+                    const int i = e / rowFloats;
                     off = gramRow( c0 + i ) + ( e - i * rowFloats );
                     off = off > gEnd4Off ? gEnd4Off : off;
                 }
