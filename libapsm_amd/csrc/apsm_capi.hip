@@ -1982,6 +1982,8 @@ void apsm_server_destroy( apsm_server* S )
         if ( D.detected )
             (void)hipEventDestroy( D.detected );
     }
+    for ( hipEvent_t ev : S->uploadEv )
+        (void)hipEventDestroy( ev );
     for ( ServeLink& L : S->links )
         apsm_destroy( L.h );
     for ( int k = 0; k < kServeSideStreams; k++ )

@@ -16,7 +16,8 @@
 // waiting for the trains, and its train joins the next round. A link takes its next frame once
 // the round with its previous frame's last block has completed. Frame buffers come from a
 // device arena of fixed size: a frame waits until the arena has room (first fit, in arrival
-// order).
+// order). Frames that wait for their link or for a batch slot are uploaded meanwhile
+// (serverUploadAhead).
 #pragma once
 
 #include <chrono>
@@ -220,6 +221,7 @@ struct ServeFrame
     size_t nextBlock = 0;
     int64_t detectBatch = -1, lastRound = -1;
     int32_t status = APSM_OK;
+    int upload = -1; // uploaded ahead of its admission: index of the event after its copies
 };
 
 // Pinned host staging and device copy of one launch's descriptors.
@@ -297,7 +299,11 @@ struct apsm_server
     size_t batchFrames = kServeBatchFrames, batchBytes = kServeBatchBytes; // a detect batch closes here
     std::deque<int64_t> roundsInFlight, detectsInFlight; // ids, oldest first
     int64_t nextRound = 0, nextDetect = 0;
-    std::deque<ServeFrame*> waiting; // arrival order
+    std::deque<ServeFrame*> waiting; // arrival order; those uploaded ahead come first
+    std::vector<hipEvent_t> uploadEv; // one per frame uploaded ahead at a time
+    std::vector<int> uploadEvFree;
+    size_t aheadBytes = 0; // arena bytes of waiting frames that are uploaded
+    hipEvent_t upLast = nullptr, upPrev = nullptr; // after the last two groups of copies on the upload stream
     std::vector<ServeFrame*> pendingTrain; // detected (enqueued), train not started
     std::vector<ServeFrame*> training; // trains in progress (blocks left)
     std::vector<ServeFrame*> finished; // completed, not yet reported by poll
@@ -383,13 +389,88 @@ void serverRetire( apsm_server* S )
     }
 }
 
+void serveUploaded( apsm_server* S, hipEvent_t ev )
+{
+    HIP_OR_THROW( hipEventRecord( ev, S->ustream ) );
+    S->upPrev = S->upLast;
+    S->upLast = ev;
+}
+
+// Arena room for a frame and its buffers in it; false where there is none now.
+bool servePlace( apsm_server* S, ServeFrame* f )
+{
+    size_t off = 0;
+    if ( !S->arenaAlloc.alloc( f->arenaBytes, off ) )
+        return false;
+    f->arenaOff = off;
+    char* base = S->arena.ptr + off;
+    const apsm_handle* h = S->links[ f->f.link ].h;
+    const size_t N = (size_t)h->N, U = (size_t)h->U;
+    f->dRxD = (float*)base;
+    base += alignUp256( N * f->f.n_data * 8 );
+    f->dRxP = (float*)base;
+    base += alignUp256( N * f->f.n_pilots * 8 );
+    f->dTxP = (float*)base;
+    base += alignUp256( U * f->f.n_pilots * 8 );
+    f->dEst = (float*)base;
+    return true;
+}
+
+// The large copies of a frame, on the upload stream.
+void serveUpload( apsm_server* S, const ServeFrame* f )
+{
+    const size_t N = (size_t)S->links[ f->f.link ].h->N;
+    HIP_OR_THROW( hipMemcpyAsync( f->dRxD, f->f.rx_data, N * f->f.n_data * 8, hipMemcpyHostToDevice, S->ustream ) );
+    if ( f->f.n_pilots > 0 )
+        HIP_OR_THROW( hipMemcpyAsync( f->dRxP, f->f.rx_pilots, N * f->f.n_pilots * 8, hipMemcpyHostToDevice, S->ustream ) );
+}
+
+// Uploads waiting frames (busy link, or no batch slot) in arrival order, so that the copy engine,
+// which bounds a saturated server, does not idle until a link's train completes (64 frames of 32 links, 24
+// antennas, 211 MB: 7.0 -> 6.0 ms). Only while at most one group of copies is queued, so that a frame of an
+// idle link waits for two frames' copies at most (with the queue kept full a saturated replay of
+// 2048 links was 5 % slower), and only a batch's bytes and a quarter of the arena. Uploaded frames
+// precede all others in `waiting`, so a frame without room never stands before them.
+void serverUploadAhead( apsm_server* S )
+{
+    const size_t most = std::min<size_t>( S->batchBytes, (size_t)S->cfg.frame_arena / 4 );
+    for ( ServeFrame* f : S->waiting )
+    {
+        if ( f->upload >= 0 )
+            continue;
+        if ( S->aheadBytes + f->arenaBytes > most )
+            break;
+        if ( S->upPrev )
+        {
+            const hipError_t e = hipEventQuery( S->upPrev );
+            if ( e == hipErrorNotReady )
+                break;
+            HIP_OR_THROW( e );
+        }
+        if ( !servePlace( S, f ) )
+            break;
+        S->aheadBytes += f->arenaBytes;
+        if ( S->uploadEvFree.empty() )
+        {
+            hipEvent_t ev = nullptr;
+            HIP_OR_THROW( hipEventCreateWithFlags( &ev, hipEventDisableTiming ) );
+            S->uploadEvFree.push_back( (int)S->uploadEv.size() );
+            S->uploadEv.push_back( ev );
+        }
+        f->upload = S->uploadEvFree.back();
+        S->uploadEvFree.pop_back();
+        serveUpload( S, f );
+        serveUploaded( S, S->uploadEv[ f->upload ] );
+    }
+}
+
 // Admits waiting frames and launches their detect batch on the detect stream; returns whether
 // it launched one.
 bool serverLaunchDetect( apsm_server* S )
 {
     if ( S->waiting.empty() || (int)S->detectsInFlight.size() >= S->detectSlots )
         return false;
-    const double now = serverNow( S );
+    const double t = serverNow( S );
     // arrival order; a frame whose link is busy waits, a frame without arena room stops admission
     std::vector<ServeFrame*> admitted;
     size_t batchBytes = 0;
@@ -404,20 +485,9 @@ bool serverLaunchDetect( apsm_server* S )
             ++it;
             continue;
         }
-        size_t off = 0;
-        if ( !S->arenaAlloc.alloc( f->arenaBytes, off ) )
+        if ( f->upload < 0 && !servePlace( S, f ) )
             break;
-        f->arenaOff = off;
-        char* base = S->arena.ptr + off;
-        const size_t N = (size_t)L.h->N, U = (size_t)L.h->U;
-        f->dRxD = (float*)base;
-        base += alignUp256( N * f->f.n_data * 8 );
-        f->dRxP = (float*)base;
-        base += alignUp256( N * f->f.n_pilots * 8 );
-        f->dTxP = (float*)base;
-        base += alignUp256( U * f->f.n_pilots * 8 );
-        f->dEst = (float*)base;
-        f->admit = now;
+        f->admit = t;
         L.busy = true;
         batchBytes += f->arenaBytes;
         admitted.push_back( f );
@@ -467,21 +537,35 @@ bool serverLaunchDetect( apsm_server* S )
     // the large copies (data and pilot samples) go on the upload stream; the small ones
     // (descriptors, transmitted pilots) on the detect stream, where the runtime's copy kernel
     // for them does not interleave with the upload stream's engine copies
-    hipStream_t st = S->dstream, up = S->ustream;
+    hipStream_t st = S->dstream;
     const char* base = D.desc.upload( arena, st );
-    for ( const ServeFrame* f : admitted )
+    bool now = false; // a frame is uploaded here: the event after it covers those uploaded ahead
+    for ( ServeFrame* f : admitted )
     {
-        const apsm_handle* h = S->links[ f->f.link ].h;
-        const size_t N = (size_t)h->N, U = (size_t)h->U;
-        HIP_OR_THROW( hipMemcpyAsync( f->dRxD, f->f.rx_data, N * f->f.n_data * 8, hipMemcpyHostToDevice, up ) );
-        if ( f->f.n_pilots > 0 )
+        if ( f->upload < 0 )
         {
-            HIP_OR_THROW( hipMemcpyAsync( f->dRxP, f->f.rx_pilots, N * f->f.n_pilots * 8, hipMemcpyHostToDevice, up ) );
-            HIP_OR_THROW( hipMemcpyAsync( f->dTxP, f->f.tx_pilots, U * f->f.n_pilots * 8, hipMemcpyHostToDevice, st ) );
+            serveUpload( S, f );
+            now = true;
         }
+        if ( f->f.n_pilots > 0 )
+            HIP_OR_THROW( hipMemcpyAsync( f->dTxP, f->f.tx_pilots, (size_t)S->links[ f->f.link ].h->U * f->f.n_pilots * 8,
+                                          hipMemcpyHostToDevice, st ) );
     }
-    HIP_OR_THROW( hipEventRecord( D.uploaded, up ) );
-    HIP_OR_THROW( hipStreamWaitEvent( st, D.uploaded, 0 ) );
+    hipEvent_t last = nullptr; // they were uploaded in arrival order
+    for ( ServeFrame* f : admitted )
+        if ( f->upload >= 0 )
+        {
+            last = S->uploadEv[ f->upload ];
+            S->uploadEvFree.push_back( f->upload );
+            S->aheadBytes -= f->arenaBytes;
+            f->upload = -1;
+        }
+    if ( now )
+    {
+        last = D.uploaded;
+        serveUploaded( S, last );
+    }
+    HIP_OR_THROW( hipStreamWaitEvent( st, last, 0 ) );
     const apsm::DetDesc* dd = (const apsm::DetDesc*)( base + detOff );
     for ( const DetL& d : detL )
     {
@@ -642,6 +726,7 @@ void serverProgress( apsm_server* S )
     serverRetire( S );
     serverLaunchDetect( S );
     serverLaunchTrainRound( S );
+    serverUploadAhead( S );
 }
 
 // Throws APSM_ERR_ARG for a frame the server cannot take; enqueues nothing.
@@ -724,6 +809,11 @@ void serverAbort( apsm_server* S )
     S->roundsInFlight.clear();
     S->detectsInFlight.clear();
     S->arenaAlloc.reset( (size_t)S->cfg.frame_arena );
+    S->aheadBytes = 0;
+    S->upLast = S->upPrev = nullptr;
+    S->uploadEvFree.clear();
+    for ( size_t k = 0; k < S->uploadEv.size(); k++ )
+        S->uploadEvFree.push_back( (int)k );
     for ( ServeLink& L : S->links )
         L.busy = false;
 }
