@@ -175,7 +175,7 @@ int apsm_train_history(apsm_handle* h, const float* rx, const float* tx, uint32_
                        float* history, uint32_t history_cap, uint32_t* num_steps, float* ms);
 
 /* LLS detector: replaces LlsNomaDetector (cpp/lib/noma/lls_detector.cu:97-218).
- * Normal equations accumulated on the device in FP32, solved by an FP64 Cholesky on the
+ * Normal equations accumulated on the device in FP64, solved by an FP64 factorization on the
  * device; detect is est = A w. lls_get_weights replaces getWeightMat() (2N floats). */
 int lls_create(uint32_t num_antennas, lls_handle** out);
 void lls_destroy(lls_handle* h);

@@ -415,7 +415,7 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
     std::map<std::array<int, 4>, std::vector<int>> dBuckets;
     for ( int i = 0; i < n; i++ )
     {
-        const int kernel = detectKernelOf( B->inst[ i ]->p.detect_precision, (uint32_t)det[ i ].N );
+        const int kernel = detectKernelOf( B->inst[ i ]->p.detect_precision );
         const bool parts = apsm::detectByParts( kernel, det[ i ].M );
         dBuckets[ { kernel, nmaxOf( det[ i ].N ), detectUmaxOf( kernel, det[ i ].U, parts ), parts } ].push_back( i );
     }

@@ -141,10 +141,6 @@ int umaxOf( int U ) { return U <= 1 ? 1 : U <= 2 ? 2 : U <= 4 ? 4 : U <= 8 ? 8 :
 int detectUmaxOf( int kernel, int U, bool parts ) { return kernel < 0 || parts ? umaxOf( U ) : U <= 1 ? 1 : std::min( 16, U + U % 2 ); }
 
 
-// APSM_PRECISION_FP32 runs the cross terms on the matrix cores from this many antennas on
-// (below, the vector-ALU kernel is at least as fast).
-constexpr uint32_t kMatrixFp32MinAntennas = 1;
-
 // Permutation of the reference shuffle (cpp/lib/noma/noma_detector.cu:59-74).
 std::vector<int32_t> shufflePermutation( int64_t T )
 {
@@ -164,7 +160,7 @@ int gridFor( int64_t n, int threads ) { return (int)( ( n + threads - 1 ) / thre
 // ---------------------------------------------------------------------------------------
 // LLS
 // ---------------------------------------------------------------------------------------
-constexpr int kLlsMaxDims = 128; // unknowns of one least-squares solve (the FP64 Cholesky is LDS-resident)
+constexpr int kLlsMaxDims = 128; // unknowns of one least-squares solve (the FP64 factor is LDS-resident)
 
 struct lls_handle
 {
@@ -954,9 +950,9 @@ void launchDetectU( apsm_handle* h, const float* d_rx, int64_t M, float* d_est, 
         launchDetect<NMAX, 16>( h, d_rx, M, d_est, Z, Zn, C, ldC, theta, G, U );
 }
 
-// The detect kernel of a precision mode for N antennas: -1 for the vector-ALU kernel, else the
+// The detect kernel of a precision mode: -1 for the vector-ALU kernel, else the
 // matrix-core input precision (apsm::PREC_*).
-int detectKernelOf( int32_t precision, uint32_t N )
+int detectKernelOf( int32_t precision )
 {
     switch ( precision )
     {
@@ -964,7 +960,7 @@ int detectKernelOf( int32_t precision, uint32_t N )
     case APSM_PRECISION_FP32_MATRIX: return apsm::PREC_F32;
     case APSM_PRECISION_BF16: return apsm::PREC_BF16;
     case APSM_PRECISION_FP16: return apsm::PREC_F16;
-    default: return N >= kMatrixFp32MinAntennas ? apsm::PREC_F32 : -1;
+    default: return apsm::PREC_F32; // faster than the vector ALUs for every antenna count
     }
 }
 
@@ -991,7 +987,7 @@ void detectDev( apsm_handle* h, const float* d_rx, int64_t M, float* d_est )
         const float* Cg = C ? C + (int64_t)u0 * ld : nullptr;
         const float* th = h->theta.ptr + (size_t)u0 * h->L;
         float* est = d_est + (size_t)u0 * M * 2;
-        const int kernel = detectKernelOf( h->p.detect_precision, h->N );
+        const int kernel = detectKernelOf( h->p.detect_precision );
         const float g2 = 0.5f / h->var * kLog2e;
         if ( apsm::detectByParts( kernel, M ) )
             HIP_OR_THROW( apsm::launchDetectParts( nmaxOf( (int)h->N ), detectUmaxOf( kernel, Ug, true ), h->stream,

@@ -507,7 +507,7 @@ bool serverLaunchDetect( apsm_server* S )
     {
         apsm_handle* h = S->links[ f->f.link ].h;
         det.push_back( detectDescOf( h, f->dRxD, f->f.n_data, f->dEst ) );
-        const int kernel = detectKernelOf( h->p.detect_precision, (uint32_t)h->N );
+        const int kernel = detectKernelOf( h->p.detect_precision );
         const bool parts = apsm::detectByParts( kernel, f->f.n_data );
         dBuckets[ { kernel, nmaxOf( h->N ), detectUmaxOf( kernel, h->U, parts ), parts } ].push_back( (int)det.size() - 1 );
         f->detectBatch = id;

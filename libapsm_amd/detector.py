@@ -307,7 +307,7 @@ class ApsmNomaDetectorFactory:
 
 
 class LlsNomaDetector(NomaDetector):
-    """Least-squares linear detector (FP32 normal equations, FP64 Cholesky, on the GPU)."""
+    """Least-squares linear detector (normal equations and solve in FP64 on the GPU)."""
 
     def __init__(self, numAntennas):
         self.numAntennas = int(numAntennas)
