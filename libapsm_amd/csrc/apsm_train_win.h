@@ -385,9 +385,8 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             float hs = h[ 0 ] + h[ 1 ];
             if constexpr ( NH > 2 )
                 hs += h[ 2 ];
-            f -= a.hasEv ? evv : 0.f;
-            f += isP ? hs : 0.f;
-            f += x;
+            // (one rounding at f's size: the shares are added up among themselves first)
+            f += x + ( ( isP ? hs : 0.f ) - ( a.hasEv ? evv : 0.f ) );
             const float res = y - f;
             const float bb = res - __builtin_amdgcn_fmed3f( res, -a.eB, a.eB );
             const float beta = bb * ( iw * inv );
