@@ -16,8 +16,9 @@
 // previous sample leaves (its f is no longer needed, only its beta), the new sample's Gram column is
 // loaded into the slot's lanes, and product k - 1 already adds the share of beta_{k-1}. H_k then only
 // needs the coefficients after projection k - 2, and helper waves have the whole interval between
-// barriers k - 2 and k - 1 to sum it: one takes the window's rows and P_k, one the active rows that have
-// left the window. A further helper (the last one, where registers allow only two) streams the
+// barriers k - 2 and k - 1 to sum it: one takes the window's rows, one the active rows that have
+// left the window. P_k is the slot's f from the takeover on (one rounding at its size fewer in every f;
+// at TP = 40, where the register it is read ahead into costs 2 %, the first helper adds it). A further helper (the last one, where registers allow only two) streams the
 // steps' packages into LDS (global -> LDS DMA, BUFS buffers). The t-slot is taken over at step k itself: the lanes of
 // the 16-lane row that holds t-slot p write kappa(p, v) into register p % TP (VGPR index mode).
 //
@@ -202,11 +203,11 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
     float* sB = sPk + BUFS * PKCAP; // [2][SB]
     float* sCw = sB + 2 * SB; // [2][2 VS]: coefficients of the window after a projection, by slot
     float* sC = sCw + 4 * VS; // [2 kActMax]: coefficients of the active rows that have left the window
-    // [kActMax + 2][4]: per step the next sample's targets (a, b) and projection weight
-    // 1 / (wL|x|^2 + wG), and 1 / W of the step itself
+    constexpr bool FROZEN = TP < 40; // P_k at the takeover
+    // [kActMax + 2][6]: per step the next sample's targets (a, b) and projection weight
+    // 1 / (wL|x|^2 + wG), 1 / W of the step itself, and the next sample's frozen shares (a, b)
     float* sStep = sC + 2 * kActMax;
-    float* sP = sStep + 4 * ( kActMax + 2 ); // [2 K]: frozen shares of the entering samples
-    float* sH = sP + 2 * ( kActMax + 2 ); // [2][NH][2]: entering shares (window rows and P, left rows)
+    float* sH = sStep + 6 * ( kActMax + 2 ); // [2][NH][2]: entering shares (window rows, left rows)
 
     const float* Yu = Y + u * a.ldYC;
     float* Cu = C + u * a.ldYC;
@@ -237,16 +238,16 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
         sB[ i ] = 0.f;
     for ( int i = tid; i < 2 * kActMax; i += THREADS )
         sC[ i ] = 0.f;
-    for ( int i = tid; i < 2 * K; i += THREADS )
-        sP[ i ] = Pu[ i ];
     for ( int i = tid; i <= K; i += THREADS ) // record i: step i - 1's next sample is sample i
     {
         const int rel = newRel0 + ( i < K ? i : K - 1 );
         const int W = a.sFirstRel + 2 * i;
-        sStep[ 4 * i ] = Yu[ 2 * rel ];
-        sStep[ 4 * i + 1 ] = Yu[ 2 * rel + 1 ];
-        sStep[ 4 * i + 2 ] = 1.f / ( a.wL * Zn[ rel ] + a.wG );
-        sStep[ 4 * i + 3 ] = 1.f / (float)( a.ramp && W < w2 ? W : w2 );
+        sStep[ 6 * i ] = Yu[ 2 * rel ];
+        sStep[ 6 * i + 1 ] = Yu[ 2 * rel + 1 ];
+        sStep[ 6 * i + 2 ] = 1.f / ( a.wL * Zn[ rel ] + a.wG );
+        sStep[ 6 * i + 3 ] = 1.f / (float)( a.ramp && W < w2 ? W : w2 );
+        sStep[ 6 * i + 4 ] = i < K ? Pu[ 2 * i ] : 0.f;
+        sStep[ 6 * i + 5 ] = i < K ? Pu[ 2 * i + 1 ] : 0.f;
     }
 
     const int kLast = newRel0 - 1; // newest sample before the block
@@ -340,8 +341,8 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
         // of the image, which there holds the leaving sample)
         float selfA = 0.f, selfC = 0.f;
         bool isP = v == p;
-        auto takeOver = [ & ]( const float* pk, float ny, float ninv ) {
-            f = 0.f;
+        auto takeOver = [ & ]( const float* pk, float ny, float ninv, float frozen ) {
+            f = frozen;
             c = 0.f;
             y = ny;
             inv = ninv;
@@ -351,10 +352,10 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
         };
         // step 0's sample takes its u-slot over (later ones do so one step early)
         if ( isP )
-            takeOver( sPk, sStep[ pt ], sStep[ 2 ] );
+            takeOver( sPk, sStep[ pt ], sStep[ 2 ], FROZEN ? sStep[ 4 + pt ] : 0.f );
         // read one step ahead: eviction share, kappa(entering, v) for t-slot p, the entering shares,
         // the weight 1 / W, and target and weight of the sample after it
-        float evv, rA, rC, rB, h[ NH ], yn, invn, iw;
+        float evv, rA, rC, rB, h[ NH ], yn, invn, fn = 0.f, iw;
         const float* sRec = sStep; // record of the step read ahead
         auto readAhead = [ & ]( const float* pk, int par ) {
             evv = pk[ evAt ];
@@ -366,9 +367,11 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             for ( int i = 0; i < NH; i++ )
                 h[ i ] = sH[ ( par * NH + i ) * 2 + pt ];
             iw = sRec[ 3 ];
-            yn = sRec[ 4 + pt ];
-            invn = sRec[ 6 ];
-            sRec += 4;
+            yn = sRec[ 6 + pt ];
+            invn = sRec[ 8 ];
+            if ( FROZEN )
+                fn = sRec[ 10 + pt ];
+            sRec += 6;
         };
         readAhead( sPk, 0 );
         float x = 0.f; // this row's product of the previous step
@@ -408,7 +411,7 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             // ---- u-slot pn: the sample of the next step (the reads need not end before the barrier;
             //      after the last step it takes a stale package, whose slot nothing reads) ----
             if ( leave )
-                takeOver( pkn, yn, invn );
+                takeOver( pkn, yn, invn, FROZEN ? fn : 0.f );
             isP = leave;
             asm volatile( "s_barrier" ::: "memory" );
             // ---- product, with the next step's reads in flight ----
@@ -421,6 +424,8 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             x = __uint_as_float( s2[ 0 ] ) + __uint_as_float( s2[ 1 ] );
             // (the reads ahead are not moved behind the product)
             asm volatile( "" : "+v"( evv ), "+v"( rA ), "+v"( rC ), "+v"( rB ), "+v"( h[ 0 ] ), "+v"( h[ 1 ] ), "+v"( yn ), "+v"( invn ), "+v"( iw ) );
+            if ( FROZEN )
+                asm volatile( "" : "+v"( fn ) );
             p = pn;
             jp++;
             if ( jp == TP || p == 0 )
@@ -457,7 +462,7 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
         // ================= helper waves =================
         // Interval k (after barrier k): the packages' wave issues package k + BUFS into the buffer step k
         // released; the entering share H_{k+2} is summed.
-        // window rows and P in H_m, coefficients as after projection m - 2 (buffer cw)
+        // window rows in H_m, coefficients as after projection m - 2 (buffer cw)
         int tOff[ ( 4 * TP + 63 ) / 64 ];
 #pragma unroll
         for ( int i = 0; i < ( 4 * TP + 63 ) / 64; i++ )
@@ -480,10 +485,9 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
                 ea += ok ? sa : 0.f;
                 eb += ok ? sb : 0.f;
             }
-            const float pv = sP[ 2 * m + ( lane >> 5 ) ];
             const float s = waveSumPair( ea, eb );
             if ( ( lane & 31 ) == 0 )
-                sH[ ( m & 1 ) * NH * 2 + ( lane >> 5 ) ] = s + pv;
+                sH[ ( m & 1 ) * NH * 2 + ( lane >> 5 ) ] = FROZEN ? s : s + sStep[ 6 * m + 4 + ( lane >> 5 ) ];
         };
         // the active rows that have left the window by step m - 1 (LEFT * 256 of them from `base` on);
         // their kappa planes come from memory through a ring of register sets
