@@ -537,7 +537,7 @@ void reserveBlockedScratch( apsm_handle* h, int64_t steps )
     if ( newPer == 1 )
     {
         h->Gact.ensure( (size_t)apsm::winGactFloats( h->w2 / 2, (int)steps ) );
-        h->EvF.ensure( (size_t)h->U * steps * apsm::winEvStride( h->w2 ) + 256 ); // whole 256-float copies
+        h->EvF.ensure( (size_t)apsm::winEvFloats( h->U, steps, h->w2 ) );
     }
     else
     {

@@ -227,7 +227,7 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
         for ( int d = 0; d < PKG / 256; d++ )
             dmaDwordx4( src + d * 256, 16u * (uint32_t)lane, __builtin_amdgcn_readfirstlane( dst + (uint32_t)d * 1024u ) );
 #pragma unroll
-        for ( int d = 0; d < ( PKCAP - PKG ) / 256; d++ )
+        for ( int d = 0; d < winPkEv( TP ) / 256; d++ )
             dmaDwordx4( ev + d * 256, 16u * (uint32_t)lane, __builtin_amdgcn_readfirstlane( dst + (uint32_t)( PKG + d * 256 ) * 4u ) );
     };
     if ( wave == NP )

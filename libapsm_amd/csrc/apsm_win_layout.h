@@ -69,7 +69,14 @@ __host__ __device__ inline int winEvStride( int w2 ) { return ( w2 + 3 ) & ~3; }
 // Package buffer in LDS: the image with the self entries, then the eviction shares, both in whole
 // 256-float copies (the left rows' planes are not copied: their helper reads them from memory).
 __host__ __device__ constexpr int winPkGram( int tp ) { return ( winImg( tp ) + 4 + 255 ) & ~255; }
-__host__ __device__ constexpr int winPkCap( int tp ) { return winPkGram( tp ) + ( ( 8 * tp + 255 ) & ~255 ); }
+__host__ __device__ constexpr int winPkEv( int tp ) { return ( 8 * tp + 255 ) & ~255; }
+__host__ __device__ constexpr int winPkCap( int tp ) { return winPkGram( tp ) + winPkEv( tp ); }
+// Floats of the eviction shares of U users in a block of `steps` steps, plus what the last row's copy
+// reads beyond it: a row is shorter than the copy (228 floats against two pieces at windowSize 113).
+inline int64_t winEvFloats( int64_t U, int64_t steps, int w2 )
+{
+    return U * steps * winEvStride( w2 ) + winPkEv( winTp( w2 / 2 ) );
+}
 // Beta pairs by t-slot, each 16-lane row's run padded to 16 bytes and so that the four rows' reads
 // fall into different LDS banks; one more pair takes the writes of lanes without a t-slot.
 __host__ __device__ constexpr int winBetaRun( int tp ) { return ( ( tp + 1 ) & ~1 ) + ( ( ( tp + 1 ) & ~1 ) % 16 == 0 ? 2 : 0 ); }
