@@ -391,7 +391,8 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             // (one rounding at f's size: the shares are added up among themselves first)
             f += x + ( ( isP ? hs : 0.f ) - ( a.hasEv ? evv : 0.f ) );
             const float res = y - f;
-            const float bb = res - __builtin_amdgcn_fmed3f( res, -a.eB, a.eB );
+            // (compared, so that a residual that is not a number, an unknown target's, projects nothing)
+            const float bb = __builtin_fabsf( res ) > a.eB ? res - __builtin_amdgcn_fmed3f( res, -a.eB, a.eB ) : 0.f;
             const float beta = bb * ( iw * inv );
             c += beta;
             // (the two upper rows of a wave write what the two lower ones write)
