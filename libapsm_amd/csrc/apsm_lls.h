@@ -8,6 +8,8 @@
 
 #include "apsm_common.h"
 
+#include <type_traits>
+
 namespace apsm {
 
 typedef double f64x4 __attribute__( ( ext_vector_type( 4 ) ) );
@@ -211,79 +213,90 @@ __global__ void __launch_bounds__( kSolveThreads ) lls_solve( const double* __re
     __shared__ double sInv[ 16 * NB ], sFloor[ 16 * NB ];
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     double a[ NB ][ NB ], z[ NB ];
+    auto factor = [ & ]( auto floorC ) {
 #pragma unroll
-    for ( int p = 0; p < NB; p++ )
+        for ( int p = 0; p < NB; p++ )
 #pragma unroll
-        for ( int q = 0; q <= p; q++ )
-        {
-            const int i = ty + 16 * p, k = tx + 16 * q;
-            a[ p ][ q ] = i < L && k <= i ? Gin[ i * ( L + 1 ) + k ] : 0.0;
-            if ( p == q && tx == ty )
-                sFloor[ i ] = kSolveFloor * a[ p ][ q ];
-        }
-#pragma unroll
-    for ( int q = 0; q < NB; q++ )
-        z[ q ] = tx + 16 * q < L ? Gin[ ( tx + 16 * q ) * ( L + 1 ) + L ] : 0.0;
-    bool bad = false;
-    int dependent = 0;
-#pragma unroll
-    for ( int jb = 0; jb < NB; jb++ )
-#pragma unroll 1
-        for ( int jj = 0; jj < 16; jj++ )
-        {
-            const int j = 16 * jb + jj;
-            if ( j >= L )
-                break;
-            double* cj = col + j * ld;
-            if ( tx == jj )
+            for ( int q = 0; q <= p; q++ )
             {
+                const int i = ty + 16 * p, k = tx + 16 * q;
+                a[ p ][ q ] = i < L && k <= i ? Gin[ i * ( L + 1 ) + k ] : 0.0;
+                if ( p == q && tx == ty )
+                    sFloor[ i ] = a[ p ][ q ] > 0.0 ? kSolveFloor * a[ p ][ q ] : -1.0; // negative: an empty column
+            }
+#pragma unroll
+        for ( int q = 0; q < NB; q++ )
+            z[ q ] = tx + 16 * q < L ? Gin[ ( tx + 16 * q ) * ( L + 1 ) + L ] : 0.0;
+#pragma unroll
+        for ( int jb = 0; jb < NB; jb++ )
+#pragma unroll 1
+            for ( int jj = 0; jj < 16; jj++ )
+            {
+                const int j = 16 * jb + jj;
+                if ( j >= L )
+                    break;
+                double* cj = col + j * ld;
+                if ( tx == jj )
+                {
+#pragma unroll
+                    for ( int p = jb; p < NB; p++ )
+                        cj[ ty + 16 * p ] = a[ p ][ jb ];
+                    if ( ty == 0 )
+                        cj[ ld - 1 ] = z[ jb ];
+                }
+                __syncthreads();
+                double d = cj[ j ], zj = cj[ ld - 1 ], ci[ NB ], ck[ NB ];
 #pragma unroll
                 for ( int p = jb; p < NB; p++ )
-                    cj[ ty + 16 * p ] = a[ p ][ jb ];
-                if ( ty == 0 )
-                    cj[ ld - 1 ] = z[ jb ];
-            }
-            __syncthreads();
-            double d = cj[ j ], least = sFloor[ j ], zj = cj[ ld - 1 ], ci[ NB ], ck[ NB ];
+                {
+                    ci[ p ] = cj[ ty + 16 * p ];
+                    ck[ p ] = cj[ tx + 16 * p ];
+                }
+                if constexpr ( floorC )
+                    d = fmax( d, fabs( sFloor[ j ] ) );
+                double inv = __builtin_amdgcn_rcp( d ); // and two Newton steps
+                inv = fma( fma( -d, inv, 1.0 ), inv, inv );
+                inv = fma( fma( -d, inv, 1.0 ), inv, inv );
+                if ( threadIdx.x == 0 )
+                    sInv[ j ] = inv;
+                // (rows and columns up to j of block jb are finished: what these get is not used)
 #pragma unroll
-            for ( int p = jb; p < NB; p++ )
-            {
-                ci[ p ] = cj[ ty + 16 * p ];
-                ck[ p ] = cj[ tx + 16 * p ];
-            }
-            dependent += d < least ? 1 : 0;
-            bad |= !( d >= -least && least > 0.0 ) || dependent > 2;
-            d = bad ? 1.0 : fmax( d, least );
-            double inv = __builtin_amdgcn_rcp( d ); // and two Newton steps
-            inv = fma( fma( -d, inv, 1.0 ), inv, inv );
-            inv = fma( fma( -d, inv, 1.0 ), inv, inv );
-            if ( threadIdx.x == 0 )
-                sInv[ j ] = inv;
-            // (rows and columns up to j of block jb are finished: what these get is not used)
+                for ( int q = jb; q < NB; q++ )
+                {
+                    const double f = -ck[ q ] * inv;
+                    z[ q ] = fma( f, zj, z[ q ] );
 #pragma unroll
-            for ( int q = jb; q < NB; q++ )
-            {
-                const double f = -ck[ q ] * inv;
-                z[ q ] = fma( f, zj, z[ q ] );
-#pragma unroll
-                for ( int p = q; p < NB; p++ )
-                    a[ p ][ q ] = fma( f, ci[ p ], a[ p ][ q ] );
+                    for ( int p = q; p < NB; p++ )
+                        a[ p ][ q ] = fma( f, ci[ p ], a[ p ][ q ] );
+                }
             }
-        }
-    __syncthreads();
+        __syncthreads();
+    };
+    // The pivots are looked at afterwards, off the chain; a system with one below its floor is factored
+    // once more with the floors.
+    auto below = [ & ]( int k ) { return k < L && !( col[ k * ld + k ] >= sFloor[ k ] && sFloor[ k ] > 0.0 ); };
+    factor( std::false_type {} );
+    if ( __syncthreads_or( below( threadIdx.x ) ) )
+        factor( std::true_type {} );
     if ( threadIdx.x < 64 )
     {
         // w_j = (z_j - sum_{i > j} col_j[i] w_i) / d_j: lane k keeps unknowns k and k + 64
         constexpr int H = NB > 4 ? 2 : 1;
         const int lane = threadIdx.x;
         double acc[ H ], x[ H ];
+        bool bad = false;
+        int dependent = 0;
 #pragma unroll
         for ( int h = 0; h < H; h++ )
         {
             const int k = lane + 64 * h < L ? lane + 64 * h : 0;
             acc[ h ] = col[ k * ld + ld - 1 ];
             x[ h ] = 0.0;
+            const double d = col[ k * ld + k ], least = sFloor[ k ];
+            bad |= least < 0.0 || !( d >= -least );
+            dependent += __popcll( __ballot( lane + 64 * h < L && d < least ) );
         }
+        bad = __ballot( bad ) != 0 || dependent > 2;
 #pragma unroll
         for ( int hj = H - 1; hj >= 0; hj-- )
         {
