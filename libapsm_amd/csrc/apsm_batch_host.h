@@ -409,21 +409,19 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
     }
     const size_t trainLaunches = pend.size();
 
-    // detect buckets by (kernel, NMAX, UMAX, by parts); work items for every candidate tile size. The
+    // detect buckets by (kernel, NMAX, UMAX); work items for every candidate tile size. The
     // kernel (vector ALU or a matrix-core precision) is the one the instance's own handle runs,
     // so only launch shapes of the same arithmetic compete.
-    std::map<std::array<int, 4>, std::vector<int>> dBuckets;
+    std::map<std::array<int, 3>, std::vector<int>> dBuckets;
     for ( int i = 0; i < n; i++ )
     {
         const int kernel = detectKernelOf( B->inst[ i ]->p.detect_precision );
-        const bool parts = apsm::detectByParts( kernel, det[ i ].M );
-        dBuckets[ { kernel, nmaxOf( det[ i ].N ), detectUmaxOf( kernel, det[ i ].U, parts ), parts } ].push_back( i );
+        dBuckets[ { kernel, nmaxOf( det[ i ].N ), detectUmaxOf( kernel, det[ i ].U ) } ].push_back( i );
     }
     const size_t detOff = arena.add( det );
     struct DetBucket
     {
         int kernel, nmax, umax, nCand;
-        bool parts;
         int threads[ kTuneCands ], shape[ kTuneCands ];
         size_t itemOff[ kTuneCands ];
         int nItems[ kTuneCands ];
@@ -435,11 +433,8 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
         db.kernel = kv.first[ 0 ];
         db.nmax = kv.first[ 1 ];
         db.umax = kv.first[ 2 ];
-        db.parts = kv.first[ 3 ];
         db.nCand = 0;
-        if ( db.parts )
-            db.threads[ db.nCand++ ] = apsm::batchPartsThreads( db.nmax, db.umax );
-        else if ( db.kernel < 0 )
+        if ( db.kernel < 0 )
             for ( int t : kTuneThreads )
             {
                 db.threads[ db.nCand ] = t;
@@ -454,9 +449,7 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
                 }
         for ( int c = 0; c < db.nCand; c++ )
         {
-            const int tileSamples = db.parts ? apsm::batchPartsSamples( db.umax )
-                : db.kernel < 0              ? db.threads[ c ]
-                                             : apsm::mfmaShapeSamples( db.shape[ c ] );
+            const int tileSamples = db.kernel < 0 ? db.threads[ c ] : apsm::mfmaShapeSamples( db.shape[ c ] );
             // instances with the largest dictionaries first (a tile's cost is proportional to
             // G): the workgroups of the persistent launch end on cheap tiles, not on a tail of
             // expensive ones
@@ -497,11 +490,8 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
     {
         const apsm::DetDesc* dd = (const apsm::DetDesc*)( base + detOff );
         const int kernel = db.kernel, nmax = db.nmax, umax = db.umax;
-        const bool parts = db.parts;
         auto launch = [ = ]( hipStream_t st, int threads, int shape, const apsm::WorkItem* it, int nItems, int grid ) {
-            if ( parts )
-                HIP_OR_THROW( apsm::launchBatchDetectParts( nmax, umax, st, dd, it, nItems, grid ) );
-            else if ( kernel < 0 )
+            if ( kernel < 0 )
                 launchBatchDetectAny( st, nmax, umax, threads, dd, it, nItems, grid );
             else
                 HIP_OR_THROW( apsm::launchBatchDetectMfma( kernel, nmax, umax, st, dd, it, nItems, grid, shape ) );
@@ -542,12 +532,8 @@ void batchPlan( apsm_batch* B, const float* const* rxT, const float* const* txT,
         const apsm::WorkItem* it = (const apsm::WorkItem*)( base + db.itemOff[ bc ] );
         detLaunches.push_back( [ = ]( hipStream_t st ) { launch( st, threads, shape, it, nItems, grid ); } );
         B->tuning.push_back( { nmax, umax, threads, bb, nItems, kernel,
-                               parts            ? apsm::batchPartsEntries( nmax, umax )
-                                   : kernel < 0 ? apsm::kDetTile
-                                                : apsm::mfmaShapeEntries( shape, nmax, kernel ),
-                               parts            ? apsm::batchPartsSamples( umax )
-                                   : kernel < 0 ? threads
-                                                : apsm::mfmaShapeSamples( shape ) } );
+                               kernel < 0 ? apsm::kDetTile : apsm::mfmaShapeEntries( shape, nmax, kernel ),
+                               kernel < 0 ? threads : apsm::mfmaShapeSamples( shape ) } );
     }
     // the buckets run side by side (their tails overlap instead of draining the GPU in turn)
     B->launches.push_back( [ B, detLaunches ]() {

@@ -138,7 +138,7 @@ int nmaxOf( int N ) { return N <= 4 ? 4 : N <= 8 ? 8 : N <= 16 ? 16 : N <= 32 ? 
 int umaxOf( int U ) { return U <= 1 ? 1 : U <= 2 ? 2 : U <= 4 ? 4 : U <= 8 ? 8 : U <= 12 ? 12 : 16; }
 // The matrix-core detect has every even bucket: a padded user costs its share of the contraction (16
 // antennas, 4096 centres, 500k samples: 10 users 3.75 ms as 12, 3.39 as 10).
-int detectUmaxOf( int kernel, int U, bool parts ) { return kernel < 0 || parts ? umaxOf( U ) : U <= 1 ? 1 : std::min( 16, U + U % 2 ); }
+int detectUmaxOf( int kernel, int U ) { return kernel < 0 ? umaxOf( U ) : U <= 1 ? 1 : std::min( 16, U + U % 2 ); }
 
 
 // Permutation of the reference shuffle (cpp/lib/noma/noma_detector.cu:59-74).
@@ -990,12 +990,12 @@ void detectDev( apsm_handle* h, const float* d_rx, int64_t M, float* d_est )
         const int kernel = detectKernelOf( h->p.detect_precision );
         const float g2 = 0.5f / h->var * kLog2e;
         if ( apsm::detectByParts( kernel, M ) )
-            HIP_OR_THROW( apsm::launchDetectParts( nmaxOf( (int)h->N ), detectUmaxOf( kernel, Ug, true ), h->stream,
+            HIP_OR_THROW( apsm::launchDetectParts( nmaxOf( (int)h->N ), umaxOf( Ug ), h->stream,
                                                    apsm::DetDesc { d_rx, Z, Zn, Cg, th, est, M, ld, G, Ug, (int)h->N,
                                                                    h->p.linear_kernel_weight, h->p.gaussian_kernel_weight, g2 } ) );
         else if ( kernel >= 0 )
         {
-            HIP_OR_THROW( apsm::launchDetectMfma( kernel, nmaxOf( (int)h->N ), detectUmaxOf( kernel, Ug, false ), h->stream, d_rx, M, Z, Zn, Cg, ld,
+            HIP_OR_THROW( apsm::launchDetectMfma( kernel, nmaxOf( (int)h->N ), detectUmaxOf( kernel, Ug ), h->stream, d_rx, M, Z, Zn, Cg, ld,
                                                   th, G, Ug, h->p.linear_kernel_weight, h->p.gaussian_kernel_weight, g2, est,
                                                   (int)h->N ) );
         }

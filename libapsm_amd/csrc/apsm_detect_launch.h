@@ -157,13 +157,14 @@ struct WorkItem
     int tile;
 };
 
-// FP32 detects of few samples add a dictionary's entries by parts: 32-entry block b belongs to part
-// b % partsOf(nmax), and the parts are added in order (apsm_detect_mfma_parts.hip). One workgroup per compute
-// unit takes 64 samples by parts, so up to 256 * 64 samples the parts of a call run at once (8
-// antennas, 685 centres, 4000 samples 14.5 us against 22.6, 16384 samples 16.0 against 23.5; 4096 centres
-// 51 / 103 and 57 / 108); beyond, whole dictionaries per wave are as fast or faster (24000
-// samples: 26.7 against 23.7; 105 / 110). The rule reads the call's samples only: a detect gives the same bits
-// alone, in a batch, served, and for every number of users.
+// FP32 detects add a dictionary's entries by parts: 32-entry block b belongs to part b % partsOf(nmax), and
+// the parts are added in order. A call of few samples shares the parts out over waves
+// (apsm_detect_mfma_parts.hip), a longer one, and those of a batch or a server, which fill the chip together,
+// takes them one after another in a wave: the same bits, however a recording is cut into calls.
+// One workgroup per compute unit takes 64 samples by parts, so up to 256 * 64 samples the parts of a call run
+// at once (8 antennas, 685 centres, 4000 samples 14.5 us against 22.6, 16384 samples 16.0 against 23.5; 4096
+// centres 51 / 103 and 57 / 108); beyond, whole dictionaries per wave are as fast or faster (24000
+// samples: 26.7 against 23.7; 105 / 110).
 constexpr int64_t kPartsMaxSamples = 16384;
 constexpr int kPartsSamples = 64; // per workgroup
 __host__ __device__ constexpr int partsEntries( int nmax ) { return nmax > 32 ? 64 : 128; } // per LDS tile
@@ -171,15 +172,6 @@ __host__ __device__ constexpr int partsOf( int nmax ) { return partsEntries( nma
 __host__ __device__ constexpr int partsThreads( int nmax ) { return 64 * partsOf( nmax ) * kPartsSamples / 32; }
 inline bool detectByParts( int kernel, int64_t M ) { return kernel == PREC_F32 && M <= kPartsMaxSamples; }
 hipError_t launchDetectParts( int nmax, int umax, hipStream_t s, const DetDesc& x );
-// The batched launch fills the chip with other calls, where waves that stage for 128 samples are
-// faster: up to 4 users a wave takes whole dictionaries and keeps the parts' sums apart (the same
-// bits); for more users their registers do not suffice.
-inline bool batchWholeParts( int umax ) { return umax <= 4; }
-inline int batchPartsThreads( int nmax, int umax ) { return batchWholeParts( umax ) ? kMfmaThreads : partsThreads( nmax ); }
-inline int batchPartsSamples( int umax ) { return batchWholeParts( umax ) ? kMfmaSamples : kPartsSamples; }
-inline int batchPartsEntries( int nmax, int umax ) { return batchWholeParts( umax ) ? mfmaTileOf( nmax, PREC_F32 ) : partsEntries( nmax ); }
-hipError_t launchBatchDetectParts( int nmax, int umax, hipStream_t s, const DetDesc* d, const WorkItem* items, int nItems, int grid );
-
 // Single-handle detect of M samples; nmax in {4, 8, 16, 32, 64}, umax 1 or even, up to 16.
 hipError_t launchDetectMfma( int prec, int nmax, int umax, hipStream_t s, const float* rx, int64_t M, const float* Z,
                              const float* Zn, const float* C, int64_t ldC, const float* theta, int64_t G, int U, float wL,

@@ -101,12 +101,14 @@ __device__ __forceinline__ void unrollFor( F f )
 
 // The Gaussian part of f for 32 samples per wave over the dictionary entries [0, G) of Z, Zn, C:
 // load( n ) is antenna n of this lane's sample (zero for none), finish( fa, fb ) takes every user's sums
-// of the lane half h (the two halves of a wave hold disjoint entries of the same samples and are
-// not yet added). MASK: entries below first( j0 ), counted within the tile from j0, do not count.
+// (for the lanes of the first half; the two halves of a wave hold disjoint entries of the same samples
+// and have been added). MASK: entries below first( j0 ), counted within the tile from j0, do not count.
 // WAVES: waves per workgroup; ETILE: dictionary entries per LDS tile (0: mfmaTileOf). PARTS > 1: the
 // entries of a tile (32 PARTS) are shared out over PARTS waves of the same samples, wave w taking block
 // w % PARTS, and finish is called for the first of them with the parts added in order. ORDER > 1: a wave
-// takes all entries and keeps the sums of blocks b % ORDER apart, which gives the bits of PARTS = ORDER.
+// takes all entries in the order 0, ORDER, 2 ORDER, ..., 1, ORDER + 1, ... of the 32-entry blocks and adds
+// each of the ORDER runs up by itself, which gives the bits of PARTS = ORDER. From 6 users on the sums of
+// the finished runs wait in LDS, for the registers' sake.
 template <int NMAX, int UMAX, int PREC, int WAVES, int ETILE, bool MASK, int PARTS, int ORDER, class LOAD, class FIRST, class FINISH>
 __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const float* __restrict__ Zn, const float* __restrict__ C,
                                               int64_t ldC, int64_t G, int U, float g2, int N, LOAD load, FIRST first, FINISH finish )
@@ -120,6 +122,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     constexpr int kCLoads = ( UMAX * kTile + kThreads - 1 ) / kThreads;
     static_assert( kTile <= kThreads && kTile % 32 == 0, "staging shape" );
     static_assert( PARTS == 1 || ( kTile == 32 * PARTS && WAVES % PARTS == 0 && !MASK ), "one block per wave and tile" );
+    static_assert( ORDER == 1 || ( !MASK && PARTS == 1 ), "runs of blocks are one wave's" );
     typedef typename MfmaIn<PREC>::V V;
     typedef uint32_t u32x4 __attribute__( ( ext_vector_type( 4 ) ) );
     // two tile buffers: the next tile's loads are in flight (in registers) while the current tile
@@ -127,6 +130,8 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     __shared__ __attribute__( ( aligned( 16 ) ) ) uint16_t sZ[ 2 ][ NS ][ kTile * RowH ];
     __shared__ __attribute__( ( aligned( 16 ) ) ) float sZn[ 3 ][ kTile ];
     __shared__ __attribute__( ( aligned( 16 ) ) ) float2 sC[ 3 ][ kTile * UMAX ]; // [entry][user]
+    constexpr bool SUMLDS = ORDER > 1 && UMAX > 4;
+    __shared__ float sSum[ SUMLDS ? UMAX * 64 * WAVES : 1 ]; // [user][lane]: sums of the finished runs
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int col = lane & 31, h = lane >> 5;
@@ -225,21 +230,53 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     float k2 = 2.f * g2, k2n = -2.f * g2;
     asm( "" : "+v"( k2 ), "+v"( k2n ) );
 
-    float fa[ ORDER ][ UMAX ], fb[ ORDER ][ UMAX ];
-#pragma unroll
-    for ( int o = 0; o < ORDER; o++ )
+    float fa[ UMAX ], fb[ UMAX ];
+    auto addHalves = [ & ]() {
 #pragma unroll
         for ( int u = 0; u < UMAX; u++ )
-            fa[ o ][ u ] = fb[ o ][ u ] = 0.f;
+        {
+            fa[ u ] += __shfl_xor( fa[ u ], 32 );
+            fb[ u ] += __shfl_xor( fb[ u ], 32 );
+        }
+    };
+    float sum[ SUMLDS ? 1 : UMAX ]; // sums of the finished runs, fa's in lane half 0 and fb's in 1
+    float* const sums = sSum + ( SUMLDS ? tid : 0 );
+#pragma unroll
+    for ( int u = 0; u < UMAX; u++ )
+    {
+        fa[ u ] = fb[ u ] = 0.f;
+        if ( SUMLDS )
+            sums[ u * 64 * WAVES ] = 0.f;
+        else
+            sum[ u ] = 0.f;
+    }
+
+    const int nBlocks = (int)( ( G + 31 ) / 32 );
 
     // tile loads into registers (zeros past the dictionary end, past N and past K): components k to k + 3
     // of entry e, r * kThreads + tid = e * K16/4 + k/4. With N == NMAX rows have no gaps: one 16-byte load.
+    // A tile holds the next blocks of the order taken.
+    constexpr int kTileBlocks = kTile / 32;
+    static_assert( kTileBlocks <= 2 || kTileBlocks == 4, "blockOf" );
+    int bLoad = 0, runLoad = 0; // next block to load, its run
+    auto nextBlock = [ & ]() { // of the runs
+        const int b = bLoad;
+        bLoad += ORDER;
+        if ( bLoad >= nBlocks )
+        {
+            runLoad++;
+            bLoad = runLoad < ORDER ? runLoad : nBlocks;
+        }
+        return b;
+    };
     float4 zreg[ kQuads ];
     float zn;
     float2 creg[ kCLoads ];
     const bool whole = N == NMAX && K == K16 && ( reinterpret_cast<uintptr_t>( Z ) & 15 ) == 0;
-    auto loadTile = [ & ]( int tt ) {
-        const int64_t j0 = (int64_t)tt * kTile;
+    auto loadRows = [ & ]() { // a tile of consecutive rows
+        const int64_t j0 = (int64_t)( ORDER > 1 ? nextBlock() : bLoad ) * 32;
+        if ( ORDER == 1 )
+            bLoad += kTileBlocks;
         const int nt = ( G - j0 ) < kTile ? (int)( G - j0 ) : kTile;
         if ( whole )
         {
@@ -277,6 +314,54 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
                 ? make_float2( C[ u * ldC + 2 * ( j0 + e ) ], C[ u * ldC + 2 * ( j0 + e ) + 1 ] )
                 : make_float2( 0.f, 0.f );
         }
+    };
+    auto loadBlocks = [ & ]() { // a tile of the next blocks of the runs
+        int blk[ kTileBlocks ];
+        unrollFor<kTileBlocks>( [ & ]( auto iC ) { blk[ iC ] = nextBlock(); } );
+        // (of values: selects of elements would keep the array in memory)
+        const int b0 = blk[ 0 ], b1 = blk[ kTileBlocks > 1 ? 1 : 0 ], b2 = blk[ kTileBlocks > 2 ? 2 : 0 ], b3 = blk[ kTileBlocks - 1 ];
+        auto blockOf = [ & ]( int i ) { // block i of the tile
+            const int lo = i < 1 ? b0 : b1, hi = i < 3 ? b2 : b3;
+            return kTileBlocks < 4 || i < 2 ? lo : hi;
+        };
+        constexpr int kBlockQuads = 8 * K16; // a wave's quads lie in one block
+#pragma unroll
+        for ( int r = 0; r < kQuads; r++ )
+        {
+            const int bi = __builtin_amdgcn_readfirstlane( ( r * kThreads + tid ) / kBlockQuads ), i = r * kThreads + tid - bi * kBlockQuads;
+            const int e = i / ( K16 / 4 ), b = __builtin_amdgcn_readfirstlane( blockOf( bi ) );
+            const int64_t j0 = (int64_t)b * 32;
+            const int nt = kAllQuads % kThreads != 0 && bi >= kTileBlocks ? 0 : G - j0 < 32 ? (int)( G - j0 ) : 32;
+            if ( whole )
+                zreg[ r ] = e < nt ? reinterpret_cast<const float4*>( Z + j0 * L )[ i ] : make_float4( 0.f, 0.f, 0.f, 0.f );
+            else
+            {
+                const int k = 4 * ( i % ( K16 / 4 ) );
+                const int n = k < NMAX ? k : k - NMAX;
+                const float* z = Z + ( j0 + e ) * L + ( k < NMAX ? n : N + n );
+                const int have = e < nt && k < K ? N - n : 0;
+                zreg[ r ].x = have > 0 ? z[ 0 ] : 0.f;
+                zreg[ r ].y = have > 1 ? z[ 1 ] : 0.f;
+                zreg[ r ].z = have > 2 ? z[ 2 ] : 0.f;
+                zreg[ r ].w = have > 3 ? z[ 3 ] : 0.f;
+            }
+        }
+        static_assert( kThreads % kTile == 0, "a thread stages one entry's norm and coefficients" );
+        const int64_t j = (int64_t)blockOf( tid % kTile / 32 ) * 32 + tid % 32;
+        zn = tid < kTile && j < G ? -g2 * Zn[ j ] : 0.f;
+#pragma unroll
+        for ( int r = 0; r < kCLoads; r++ )
+        {
+            const int u = r * ( kThreads / kTile ) + tid / kTile;
+            // (C and ldC are even numbers of floats from an allocation's start)
+            creg[ r ] = u < UMAX && u < U && j < G ? *reinterpret_cast<const float2*>( C + u * ldC + 2 * j ) : make_float2( 0.f, 0.f );
+        }
+    };
+    auto loadTile = [ & ]() {
+        if constexpr ( ORDER > 1 && ( kTileBlocks > 1 || UMAX > 8 || ( NMAX >= 64 && UMAX > 2 ) ) ) // (scalar addresses: fewer spills)
+            loadBlocks();
+        else
+            loadRows();
     };
     auto storeTile = [ & ]( int tt ) {
         const int buf = tt & 1, slot = tt % 3;
@@ -347,8 +432,9 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     // coefficient slot `slot`), between them the products of the next block (entries cbn of buffer
     // bufn) into the other set. The fences keep the two streams interleaved entry by entry.
     constexpr int PF = UMAX <= 2 ? 4 : 1; // entries whose coefficients are read ahead together
-    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, auto oC, int rel = 0 ) {
-        constexpr int d = dC, ord = oC;
+    int run = 0, runLeft = ( nBlocks + ORDER - 1 ) / ORDER; // run of the next phase, blocks left in it
+    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, int rel = 0 ) {
+        constexpr int d = dC;
         float2 co[ 2 ][ PF * UMAX ];
         float4 zq[ 2 ];
         auto entryOf = [ & ]( int i ) { return cb + 8 * ( i / 4 ) + 4 * h + i % 4; }; // the lane's entry i within the tile
@@ -385,12 +471,25 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
             for ( int u = 0; u < UMAX; u++ )
             {
                 const float2 c = co[ i / PF & 1 ][ i % PF * UMAX + u ];
-                fa[ ord ][ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ ord ][ u ] ) );
-                fb[ ord ][ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ ord ][ u ] ) );
-                asm volatile( "" : "+v"( fa[ ord ][ u ] ), "+v"( fb[ ord ][ u ] )::"memory" );
+                fa[ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ u ] ) );
+                fb[ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ u ] ) );
+                asm volatile( "" : "+v"( fa[ u ] ), "+v"( fb[ u ] )::"memory" );
             }
             __builtin_amdgcn_sched_barrier( 0 );
         } );
+        if constexpr ( ORDER > 1 )
+            if ( --runLeft == 0 ) // the run ends with this block
+            {
+#pragma unroll
+                for ( int u = 0; u < UMAX; u++ )
+                {
+                    const auto s = __builtin_amdgcn_permlane32_swap( __float_as_uint( fa[ u ] ), __float_as_uint( fb[ u ] ), false, false );
+                    ( SUMLDS ? sums[ u * 64 * WAVES ] : sum[ SUMLDS ? 0 : u ] ) += __uint_as_float( s[ 0 ] ) + __uint_as_float( s[ 1 ] );
+                    fa[ u ] = fb[ u ] = 0.f;
+                }
+                run++;
+                runLeft = ( nBlocks - run + ORDER - 1 ) / ORDER;
+            }
     };
 
     // Tile tt + 1 is stored between two barriers' reach: its rows (two buffers) replace those of tile
@@ -402,10 +501,10 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     const int nTiles = (int)( ( G + kTile - 1 ) / kTile );
     if ( nTiles > 0 )
     {
-        loadTile( 0 );
+        loadTile();
         storeTile( 0 );
         if ( nTiles > 1 )
-            loadTile( 1 );
+            loadTile();
     }
     __syncthreads();
     auto products = [ & ]( int buf, int cb ) {
@@ -418,59 +517,47 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         if ( tt + 1 < nTiles )
             storeTile( tt + 1 );
         if ( tt + 2 < nTiles )
-            loadTile( tt + 2 );
+            loadTile();
         __syncthreads();
     };
     // (the products past the last block read what the buffers hold, and are not used)
-    static_assert( ORDER == 1 || ( !MASK && PARTS == 1 && ( kBlocks == 1 || ORDER % kBlocks == 0 ) ), "whole turns of the sums" );
     if constexpr ( !PIPE )
     {
 #pragma unroll 1
-        for ( int t0 = 0; t0 < nTiles; t0 += ORDER )
-            unrollFor<ORDER>( [ & ]( auto iC ) {
-                const int tt = t0 + iC;
-                if ( tt >= nTiles )
-                    return;
+        for ( int tt = 0; tt < nTiles; tt++ )
+        {
 #pragma unroll 1
-                for ( int cb = cw; cb < kTile; cb += 32 * PARTS )
-                {
-                    if ( (int64_t)tt * kTile + cb >= G )
-                        break;
-                    products( tt & 1, cb );
-                    phase( tt % 3, cb, 0, 0, D0 {}, iC, MASK ? first( (int64_t)tt * kTile ) : 0 );
-                }
-                advance( tt );
-            } );
+            for ( int cb = cw; cb < kTile; cb += 32 * PARTS )
+            {
+                if ( (int64_t)tt * kTile + cb >= G )
+                    break;
+                products( tt & 1, cb );
+                phase( tt % 3, cb, 0, 0, D0 {}, MASK ? first( (int64_t)tt * kTile ) : 0 );
+            }
+            advance( tt );
+        }
     }
     else if constexpr ( kBlocks == 1 )
     {
-        constexpr int STEP = ORDER > 2 ? ORDER : 2;
 #pragma unroll 1
-        for ( int t0 = 0; t0 < nTiles; t0 += STEP )
-            unrollFor<STEP>( [ & ]( auto iC ) {
+        for ( int t0 = 0; t0 < nTiles; t0 += 2 )
+            unrollFor<2>( [ & ]( auto iC ) {
                 const int tt = t0 + iC;
                 if ( tt >= nTiles )
                     return;
                 advance( tt );
-                phase( tt % 3, cw, ( tt + 1 ) & 1, cw, std::integral_constant<int, iC & 1> {}, std::integral_constant<int, iC % ORDER> {} );
+                phase( tt % 3, cw, ( tt + 1 ) & 1, cw, std::integral_constant<int, iC> {} );
             } );
     }
     else
     {
-        constexpr int STEP = ORDER > kBlocks ? ORDER / kBlocks : 1;
 #pragma unroll 1
-        for ( int t0 = 0; t0 < nTiles; t0 += STEP )
-            unrollFor<STEP>( [ & ]( auto iC ) {
-                const int tt = t0 + iC;
-                if ( tt >= nTiles )
-                    return;
-                unrollFor<kBlocks>( [ & ]( auto bC ) {
-                    constexpr int b = bC, last = b == kBlocks - 1;
-                    if constexpr ( last )
-                        advance( tt );
-                    phase( tt % 3, 32 * b, ( tt + last ) & 1, last ? 0 : 32 * b + 32, std::integral_constant<int, b & 1> {},
-                           std::integral_constant<int, ( iC * kBlocks + b ) % ORDER> {} );
-                } );
+        for ( int tt = 0; tt < nTiles; tt++ )
+            unrollFor<kBlocks>( [ & ]( auto bC ) {
+                constexpr int b = bC, last = b == kBlocks - 1;
+                if constexpr ( last )
+                    advance( tt );
+                phase( tt % 3, 32 * b, ( tt + last ) & 1, last ? 0 : 32 * b + 32, std::integral_constant<int, b & 1> {} );
             } );
     }
     __syncthreads(); // a following tile stores over what other waves may still read
@@ -478,6 +565,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     if constexpr ( PARTS > 1 )
     {
         const int wave = tid >> 6, part = wave % PARTS;
+        addHalves();
         constexpr int kRed = WAVES / PARTS * ( PARTS - 1 ) * UMAX * 64;
         constexpr bool inTile = sizeof( sZ ) >= kRed * sizeof( float2 );
         __shared__ float2 sRed[ inTile ? 1 : kRed ];
@@ -485,7 +573,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         if ( part > 0 )
 #pragma unroll
             for ( int u = 0; u < UMAX; u++ )
-                red[ ( ( part - 1 ) * UMAX + u ) * 64 ] = make_float2( fa[ 0 ][ u ], fb[ 0 ][ u ] );
+                red[ ( ( part - 1 ) * UMAX + u ) * 64 ] = make_float2( fa[ u ], fb[ u ] );
         __syncthreads();
         if ( part == 0 )
         {
@@ -495,29 +583,32 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
                 for ( int u = 0; u < UMAX; u++ )
                 {
                     const float2 v = red[ ( k * UMAX + u ) * 64 ];
-                    fa[ 0 ][ u ] += v.x;
-                    fb[ 0 ][ u ] += v.y;
+                    fa[ u ] += v.x;
+                    fb[ u ] += v.y;
                 }
-            finish( fa[ 0 ], fb[ 0 ] );
+            finish( fa, fb );
         }
         __syncthreads(); // a following tile stores over what was read
     }
     else
     {
-#pragma unroll
-        for ( int o = 1; o < ORDER; o++ )
+        if constexpr ( ORDER > 1 )
+        {
 #pragma unroll
             for ( int u = 0; u < UMAX; u++ )
             {
-                fa[ 0 ][ u ] += fa[ o ][ u ];
-                fb[ 0 ][ u ] += fb[ o ][ u ];
+                fa[ u ] = SUMLDS ? sums[ u * 64 * WAVES ] : sum[ SUMLDS ? 0 : u ];
+                fb[ u ] = __shfl_xor( fa[ u ], 32 );
             }
-        finish( fa[ 0 ], fb[ 0 ] );
+        }
+        else
+            addHalves();
+        finish( fa, fb );
     }
 }
 
 // One tile of 32 * WAVES / PARTS data samples of a detect.
-template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0, int PARTS = 1, int ORDER = 1>
+template <int NMAX, int UMAX, int PREC, int WAVES = 4, int ETILE = 0, int PARTS = 1>
 __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, int64_t M, const float* __restrict__ Z,
                                                 const float* __restrict__ Zn, const float* __restrict__ C, int64_t ldC,
                                                 const float* __restrict__ theta, int64_t G, int U, float wL, float wG, float g2,
@@ -527,17 +618,12 @@ __device__ __forceinline__ void detectTileMfma( const float* __restrict__ rx, in
     const int64_t m = tile * ( 32 * WAVES / PARTS ) + ( threadIdx.x >> 6 ) / PARTS * 32 + ( threadIdx.x & 31 ); // this lane's sample
     const bool valid = m < M;
     const float2* x = reinterpret_cast<const float2*>( rx ) + m;
+    constexpr int ORDER = PREC == PREC_F32 && PARTS == 1 ? partsOf( NMAX ) : 1;
     gaussianMfma<NMAX, UMAX, PREC, WAVES, ETILE, false, PARTS, ORDER>(
         Z, Zn, C, ldC, G, U, g2, N, [ & ]( int n ) { return valid && n < N ? x[ (int64_t)n * M ] : make_float2( 0.f, 0.f ); },
         []( int64_t ) { return 0; },
         [ & ]( float( &fa )[ UMAX ], float( &fb )[ UMAX ] ) {
             // f = wL theta . x + wG (Gaussian part), x read again
-#pragma unroll
-            for ( int u = 0; u < UMAX; u++ )
-            {
-                fa[ u ] += __shfl_xor( fa[ u ], 32 );
-                fb[ u ] += __shfl_xor( fb[ u ], 32 );
-            }
             if ( !valid || h != 0 )
                 return;
             float la[ UMAX ], lb[ UMAX ];

@@ -48,12 +48,6 @@ __device__ __forceinline__ void entryChunkMfma( const float* __restrict__ Z, con
             return d < 0 ? 0 : d > kEntryChunk ? (int)kEntryChunk : (int)d;
         },
         [ & ]( float( &fa )[ UMAX ], float( &fb )[ UMAX ] ) {
-#pragma unroll
-            for ( int u = 0; u < UMAX; u++ )
-            {
-                fa[ u ] += __shfl_xor( fa[ u ], 32 );
-                fb[ u ] += __shfl_xor( fb[ u ], 32 );
-            }
             if ( !valid || h != 0 )
                 return;
 #pragma unroll

@@ -502,29 +502,26 @@ bool serverLaunchDetect( apsm_server* S )
     D.frames = admitted;
     DescArena arena;
     std::vector<apsm::DetDesc> det;
-    std::map<std::array<int, 4>, std::vector<int>> dBuckets;
+    std::map<std::array<int, 3>, std::vector<int>> dBuckets;
     for ( ServeFrame* f : admitted )
     {
         apsm_handle* h = S->links[ f->f.link ].h;
         det.push_back( detectDescOf( h, f->dRxD, f->f.n_data, f->dEst ) );
         const int kernel = detectKernelOf( h->p.detect_precision );
-        const bool parts = apsm::detectByParts( kernel, f->f.n_data );
-        dBuckets[ { kernel, nmaxOf( h->N ), detectUmaxOf( kernel, h->U, parts ), parts } ].push_back( (int)det.size() - 1 );
+        dBuckets[ { kernel, nmaxOf( h->N ), detectUmaxOf( kernel, h->U ) } ].push_back( (int)det.size() - 1 );
         f->detectBatch = id;
     }
     const size_t detOff = arena.add( det );
     struct DetL
     {
         int kernel, nmax, umax, nItems;
-        bool parts;
         size_t itemOff;
     };
     std::vector<DetL> detL;
     for ( auto& kv : dBuckets )
     {
         const int kernel = kv.first[ 0 ];
-        const bool parts = kv.first[ 3 ];
-        const int tile = parts ? apsm::batchPartsSamples( kv.first[ 2 ] ) : kernel < 0 ? apsm::kDetThreads : apsm::mfmaShapeSamples( 0 );
+        const int tile = kernel < 0 ? apsm::kDetThreads : apsm::mfmaShapeSamples( 0 );
         // frames of the largest dictionaries first (see the batched detect)
         std::vector<int> order( kv.second );
         std::stable_sort( order.begin(), order.end(), [ & ]( int x, int y ) { return det[ x ].G > det[ y ].G; } );
@@ -532,7 +529,7 @@ bool serverLaunchDetect( apsm_server* S )
         for ( int i : order )
             for ( int64_t t = 0; t < ( det[ i ].M + tile - 1 ) / tile; t++ )
                 items.push_back( apsm::WorkItem { i, (int)t } );
-        detL.push_back( DetL { kernel, kv.first[ 1 ], kv.first[ 2 ], (int)items.size(), parts, arena.add( items ) } );
+        detL.push_back( DetL { kernel, kv.first[ 1 ], kv.first[ 2 ], (int)items.size(), arena.add( items ) } );
     }
     // the large copies (data and pilot samples) go on the upload stream; the small ones
     // (descriptors, transmitted pilots) on the detect stream, where the runtime's copy kernel
@@ -571,9 +568,7 @@ bool serverLaunchDetect( apsm_server* S )
     {
         const int grid = std::max( 1, std::min( d.nItems, S->cus * 4 ) );
         const apsm::WorkItem* it = (const apsm::WorkItem*)( base + d.itemOff );
-        if ( d.parts )
-            HIP_OR_THROW( apsm::launchBatchDetectParts( d.nmax, d.umax, st, dd, it, d.nItems, grid ) );
-        else if ( d.kernel < 0 )
+        if ( d.kernel < 0 )
             launchBatchDetectAny( st, d.nmax, d.umax, apsm::kDetThreads, dd, it, d.nItems, grid );
         else
             HIP_OR_THROW( apsm::launchBatchDetectMfma( d.kernel, d.nmax, d.umax, st, dd, it, d.nItems, grid ) );
