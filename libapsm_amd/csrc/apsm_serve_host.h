@@ -20,6 +20,8 @@
 // (serverUploadAhead).
 #pragma once
 
+#include "apsm_serve_ahead.h"
+
 #include <chrono>
 #include <deque>
 
@@ -427,27 +429,25 @@ void serveUpload( apsm_server* S, const ServeFrame* f )
 
 // Uploads waiting frames (busy link, or no batch slot) in arrival order, so that the copy engine,
 // which bounds a saturated server, does not idle until a link's train completes (64 frames of 32 links, 24
-// antennas, 211 MB: 7.0 -> 6.0 ms). Only while at most one group of copies is queued, so that a frame of an
-// idle link waits for two frames' copies at most (with the queue kept full a saturated replay of
-// 2048 links was 5 % slower), and only a batch's bytes and a quarter of the arena. Uploaded frames
-// precede all others in `waiting`, so a frame without room never stands before them.
+// antennas, 211 MB: 7.0 -> 6.0 ms). Only while at most one group of copies is queued, and two frames a step
+// (apsm_serve_ahead.h), so that a frame of an idle link waits for two frames' copies at most, from pinned
+// or pageable memory (with the queue kept full a saturated replay of 2048 links was 5 % slower), and only
+// a batch's bytes and a quarter of the arena. Uploaded frames precede all others in `waiting`, so a frame
+// without room never stands before them.
 void serverUploadAhead( apsm_server* S )
 {
-    const size_t most = std::min<size_t>( S->batchBytes, (size_t)S->cfg.frame_arena / 4 );
+    AheadStep step( std::min<size_t>( S->batchBytes, (size_t)S->cfg.frame_arena / 4 ) );
+    auto pending = [ S ]() {
+        const hipError_t e = S->upPrev ? hipEventQuery( S->upPrev ) : hipSuccess;
+        if ( e != hipErrorNotReady )
+            HIP_OR_THROW( e );
+        return e == hipErrorNotReady;
+    };
     for ( ServeFrame* f : S->waiting )
     {
         if ( f->upload >= 0 )
             continue;
-        if ( S->aheadBytes + f->arenaBytes > most )
-            break;
-        if ( S->upPrev )
-        {
-            const hipError_t e = hipEventQuery( S->upPrev );
-            if ( e == hipErrorNotReady )
-                break;
-            HIP_OR_THROW( e );
-        }
-        if ( !servePlace( S, f ) )
+        if ( !step.take( S->aheadBytes, f->arenaBytes, pending ) || !servePlace( S, f ) )
             break;
         S->aheadBytes += f->arenaBytes;
         if ( S->uploadEvFree.empty() )
