@@ -72,11 +72,11 @@ struct Seq2Args
 __device__ __forceinline__ void ldsBarrier() { asm volatile( "s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory" ); }
 
 // Asynchronous global -> LDS copy of one dword per lane (lane i writes ldsWaveBase + 4*i).
-// M0 carries the wave's LDS destination (one wait state between the M0 write and the load);
-// the sequencer kernel uses M0 for nothing else.
+// M0 carries the wave's LDS destination (one wait state between the M0 write and the load), and is
+// declared changed: the compiler uses it too, for indexed register writes among others.
 __device__ __forceinline__ void dmaDword( const float* src, uint32_t ldsWaveBase )
 {
-    asm volatile( "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"( ldsWaveBase ), "v"( src ) : "memory" );
+    asm volatile( "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"( ldsWaveBase ), "v"( src ) : "memory", "m0" );
 }
 
 // The same with 16 bytes per lane from a wave-uniform base plus a per-lane 32-bit byte offset
@@ -85,7 +85,7 @@ __device__ __forceinline__ void dmaDword( const float* src, uint32_t ldsWaveBase
 // the offset, so no 64-bit address arithmetic runs on the vector ALU
 __device__ __forceinline__ void dmaDwordx4( const float* base, uint32_t byteOff, uint32_t ldsWaveBase )
 {
-    asm volatile( "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"( ldsWaveBase ), "v"( byteOff ), "s"( base ) : "memory" );
+    asm volatile( "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"( ldsWaveBase ), "v"( byteOff ), "s"( base ) : "memory", "m0" );
 }
 
 // threadIdx.x behind an empty asm: indices derived from it inside the step loop are recomputed
