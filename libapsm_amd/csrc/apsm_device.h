@@ -813,8 +813,9 @@ __device__ __forceinline__ uint32_t vhBin( uint32_t bits, int pass, uint32_t pre
     return bits & 0xFFu;
 }
 
-// |x + iy| where the squares neither overflow nor vanish (1 ulp, as hypotf, at less than half its
-// instructions; a sum of N such values between 1e-10 and 1e15 loses at most 64 * 1e-19 to
+// |x + iy| where the squares neither overflow nor vanish, at less than half of hypotf's instructions and with
+// its error (over 4 million pairs both are off by at most 1.48 ulp, 1.41e-7, and a trained variance has the
+// same bits with either; a sum of N such values between 1e-10 and 1e15 loses at most 64 * 1e-19 to
 // vanished squares).
 __device__ __forceinline__ float vhAbs( float x, float y ) { return __builtin_amdgcn_sqrtf( fmaf( x, x, y * y ) ); }
 
