@@ -396,8 +396,10 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     constexpr int kProducts = ( NS == 3 ? 12 : 2 ) * T;
     // The next block's products run under this one's exponentials, into a second set of accumulators
     // (one set, and one after the other, where two do not fit the registers, and for the entering
-    // pilots' chunks of one or two blocks).
-    constexpr bool PIPE = !SUBTRACT && !MASK;
+    // pilots' chunks of one or two blocks). At 32 antennas that is so from 13 users on: with two sets
+    // 145 registers spilled at 16 users, and 2000 centres took 1474 us for 120k samples, 762 with one (1350
+    // before the three-part products).
+    constexpr bool PIPE = !SUBTRACT && !MASK && !( NS == 3 && NMAX >= 32 && UMAX > 12 );
     mf32x16 accP[ PIPE ? 2 : 1 ], accS[ PIPE ? 2 : 1 ], accM;
     V az[ 2 ][ NS ];
     auto readGroup = [ & ]( int buf, int cb, auto gC ) {
