@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <array>
 #include <functional>
+#include <cfloat>
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -669,7 +670,7 @@ int64_t planBlock( const apsm_handle* h, const StreamBuf& b, int64_t usedOld, in
     s2.ldYC = ld;
     s2.wL = wL;
     s2.wG = wG;
-    s2.eB = h->p.eB;
+    s2.eB = std::min( h->p.eB, FLT_MAX ); // (the window sequencer adds eB and -eB)
     const int64_t aR = a0 - rowBase; // local real row of the first active row
     k.s.Z = b.Z.ptr + ( aR / 2 ) * L;
     k.s.Zn = b.Zn.ptr + aR / 2;

@@ -391,8 +391,9 @@ __device__ __forceinline__ void winBody( const float* __restrict__ Z, const floa
             // (one rounding at f's size: the shares are added up among themselves first)
             f += x + ( ( isP ? hs : 0.f ) - ( a.hasEv ? evv : 0.f ) );
             const float res = y - f;
-            // (compared, so that a residual that is not a number, an unknown target's, projects nothing)
-            const float bb = __builtin_fabsf( res ) > a.eB ? res - __builtin_amdgcn_fmed3f( res, -a.eB, a.eB ) : 0.f;
+            // (for a residual that is not a number, an unknown target's, maximum and minimum give the other
+            // operand: it projects nothing)
+            const float bb = fmaxf( res, a.eB ) + fminf( res, -a.eB );
             const float beta = bb * ( iw * inv );
             c += beta;
             // (the two upper rows of a wave write what the two lower ones write)
