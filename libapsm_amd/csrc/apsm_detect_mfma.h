@@ -259,6 +259,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     constexpr int kTileBlocks = kTile / 32;
     static_assert( kTileBlocks <= 2 || kTileBlocks == 4, "blockOf" );
     int bLoad = 0, runLoad = 0; // next block to load, its run
+    const float* zLoad = Z; // and its first row
     auto nextBlock = [ & ]() { // of the runs
         const int b = bLoad;
         bLoad += ORDER;
@@ -317,28 +318,35 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     };
     auto loadBlocks = [ & ]() { // a tile of the next blocks of the runs
         int blk[ kTileBlocks ];
-        unrollFor<kTileBlocks>( [ & ]( auto iC ) { blk[ iC ] = nextBlock(); } );
-        // (of values: selects of elements would keep the array in memory)
-        const int b0 = blk[ 0 ], b1 = blk[ kTileBlocks > 1 ? 1 : 0 ], b2 = blk[ kTileBlocks > 2 ? 2 : 0 ], b3 = blk[ kTileBlocks - 1 ];
-        auto blockOf = [ & ]( int i ) { // block i of the tile
-            const int lo = i < 1 ? b0 : b1, hi = i < 3 ? b2 : b3;
+        const float* row[ kTileBlocks ]; // their first rows
+        unrollFor<kTileBlocks>( [ & ]( auto iC ) {
+            row[ iC ] = zLoad;
+            const int run = runLoad;
+            blk[ iC ] = nextBlock();
+            zLoad = runLoad == run ? zLoad + ORDER * 32 * L : Z + (int64_t)bLoad * 32 * L;
+        } );
+        // element i (of values: selects of elements would keep the array in memory)
+        auto pick = [ & ]( const auto& v, int i ) {
+            const auto v0 = v[ 0 ], v1 = v[ kTileBlocks > 1 ? 1 : 0 ], v2 = v[ kTileBlocks > 2 ? 2 : 0 ], v3 = v[ kTileBlocks - 1 ];
+            const auto lo = i < 1 ? v0 : v1, hi = i < 3 ? v2 : v3;
             return kTileBlocks < 4 || i < 2 ? lo : hi;
         };
+        const int Gi = (int)G;
         constexpr int kBlockQuads = 8 * K16; // a wave's quads lie in one block
 #pragma unroll
         for ( int r = 0; r < kQuads; r++ )
         {
             const int bi = __builtin_amdgcn_readfirstlane( ( r * kThreads + tid ) / kBlockQuads ), i = r * kThreads + tid - bi * kBlockQuads;
-            const int e = i / ( K16 / 4 ), b = __builtin_amdgcn_readfirstlane( blockOf( bi ) );
-            const int64_t j0 = (int64_t)b * 32;
-            const int nt = kAllQuads % kThreads != 0 && bi >= kTileBlocks ? 0 : G - j0 < 32 ? (int)( G - j0 ) : 32;
+            const int e = i / ( K16 / 4 );
+            const int nt = kAllQuads % kThreads != 0 && bi >= kTileBlocks ? 0 : Gi - 32 * pick( blk, bi ); // (32 and more: a whole block)
+            const float* z0 = pick( row, bi );
             if ( whole )
-                zreg[ r ] = e < nt ? reinterpret_cast<const float4*>( Z + j0 * L )[ i ] : make_float4( 0.f, 0.f, 0.f, 0.f );
+                zreg[ r ] = e < nt ? reinterpret_cast<const float4*>( z0 )[ i ] : make_float4( 0.f, 0.f, 0.f, 0.f );
             else
             {
                 const int k = 4 * ( i % ( K16 / 4 ) );
                 const int n = k < NMAX ? k : k - NMAX;
-                const float* z = Z + ( j0 + e ) * L + ( k < NMAX ? n : N + n );
+                const float* z = z0 + e * L + ( k < NMAX ? n : N + n );
                 const int have = e < nt && k < K ? N - n : 0;
                 zreg[ r ].x = have > 0 ? z[ 0 ] : 0.f;
                 zreg[ r ].y = have > 1 ? z[ 1 ] : 0.f;
@@ -347,14 +355,15 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
             }
         }
         static_assert( kThreads % kTile == 0, "a thread stages one entry's norm and coefficients" );
-        const int64_t j = (int64_t)blockOf( tid % kTile / 32 ) * 32 + tid % 32;
-        zn = tid < kTile && j < G ? -g2 * Zn[ j ] : 0.f;
+        const int j = pick( blk, tid % kTile / 32 ) * 32 + tid % 32;
+        const bool in = j < Gi;
+        zn = tid < kTile && in ? -g2 * Zn[ j ] : 0.f;
 #pragma unroll
         for ( int r = 0; r < kCLoads; r++ )
         {
             const int u = r * ( kThreads / kTile ) + tid / kTile;
             // (C and ldC are even numbers of floats from an allocation's start)
-            creg[ r ] = u < UMAX && u < U && j < G ? *reinterpret_cast<const float2*>( C + u * ldC + 2 * j ) : make_float2( 0.f, 0.f );
+            creg[ r ] = u < UMAX && u < U && in ? reinterpret_cast<const float2*>( C + u * ldC )[ j ] : make_float2( 0.f, 0.f );
         }
     };
     auto loadTile = [ & ]() {
