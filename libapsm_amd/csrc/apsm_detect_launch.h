@@ -84,9 +84,9 @@ struct EntryMfmaDesc
 // to c0), kappa = wL x.z + wG K in the three real forms A = kappa(a_i,a_j) = kappa(b_i,b_j),
 // B = kappa(a_i,b_j), C = kappa(b_i,a_j); 32 x 32 sample blocks of the lower triangle on the
 // matrix cores, four per workgroup.
-// With Wc > 0 the buffer has the window sequencer's layout instead (apsm_train_win.h): Wc the
-// window's complex samples, newRel0 the first entering sample (relative to c0), cMod the slot of
-// sample 0, tp its t-slots per lane.
+// With Wc > 0 (sampleStep 2) the buffer has the window sequencer's layout instead (apsm_win_layout.h), from
+// 16 x 16 blocks: Wc the window's complex samples, newRel0 the first entering sample (relative to c0),
+// cMod the slot of sample 0, tp its t-slots per lane.
 struct GramArgs
 {
     int N, L;
@@ -162,9 +162,17 @@ struct WorkItem
 // (apsm_detect_mfma_parts.hip), a longer one, and those of a batch or a server, which fill the chip together,
 // takes them one after another in a wave: the same bits, however a recording is cut into calls.
 // One workgroup per compute unit takes 64 samples by parts, so up to 256 * 64 samples the parts of a call run
-// at once (8 antennas, 685 centres, 4000 samples 14.5 us against 22.6, 16384 samples 16.0 against 23.5; 4096
-// centres 51 / 103 and 57 / 108); beyond, whole dictionaries per wave are as fast or faster (24000
-// samples: 26.7 against 23.7; 105 / 110).
+// at once; beyond, a second round of workgroups makes it slower (8 antennas, 685 centres, 24000 samples 26.7
+// against 23.7 us in the kernel). A call of 16384 samples by parts and of 16385 in one wave, microseconds:
+//   antennas  users   685 centres   4096 centres
+//      8        1       21 / 31        62 / 120
+//      8       12       39 / 69       150 / 332
+//     32        1       34 / 45       117 / 199
+//     32       10       94 / 87       422 / 392   (10 users run as 12 by parts)
+//     32       12       95 / 117      427 / 559
+//     64        1       53 / 80       223 / 402
+//     64       12       84 / 162      369 / 837
+// and 1000 samples take by parts what 4000 take.
 constexpr int64_t kPartsMaxSamples = 16384;
 constexpr int kPartsSamples = 64; // per workgroup
 __host__ __device__ constexpr int partsEntries( int nmax ) { return nmax > 32 ? 64 : 128; } // per LDS tile

@@ -26,10 +26,11 @@
 // the clock falls from 2.1 GHz to 1.6 to 1.75. Detect calls before (FP32 products on
 // v_mfma_f32_32x32x2_f32, one block's products and exponentials after each other) and now:
 //   8 antennas, 685 centres, 3840 samples              60 -> 33 us
-//   16 antennas, 10 users, 4096 centres, 500k samples  5.69 -> 3.39 ms
-//   32 antennas, 3690 centres, 49999 samples           678 -> 280 us
-//   64 antennas, 12 users, 16384 centres, 400k samples, bf16  16.1 -> 12.9 ms
-// or per block of 32 x 32 and SIMD, in cycles as if at 2.4 GHz: 1460 (8 antennas), 2070 (16), 3340 (32), 6880 (64).
+//   16 antennas, 10 users, 4096 centres, 500k samples  5.69 -> 3.38 ms
+//   32 antennas, 3690 centres, 49999 samples           678 -> 279 us
+//   64 antennas, 12 users, 16384 centres, 400k samples, bf16  16.1 -> 13.0 ms
+// or per block of 32 x 32 and SIMD, in cycles as if at 2.4 GHz: 1460 (8 antennas), 2070 (16), 3340 (32), 6880 (64),
+// measured with the blocks in plain order; taken by parts, 8 and 16 antennas cost 1 to 4 % more (ORDER).
 // Measured and not kept: two column blocks per wave sharing the coefficient reads (10 % faster at 4 users,
 // slower elsewhere, 64 antennas spilled); 8 waves per workgroup (within 2 %); staging loads without
 // the bounds branches (20 % slower); all products before all exponentials (as fast up to 16

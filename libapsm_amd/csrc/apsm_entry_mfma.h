@@ -1,5 +1,5 @@
 // Frozen-dictionary share of the entering pilots of one train block, with the cross terms on
-// the matrix cores (FP32 inputs and accumulation).
+// the matrix cores (FP32 inputs as three bf16 parts each, FP32 accumulation: the detect's core).
 //
 // For the entering complex samples i < nNewC of a block (rows newC0 + i of the stream buffer)
 // and every user u: g_u(i) = sum over frozen dictionary entries j in [j0(i), j1) of

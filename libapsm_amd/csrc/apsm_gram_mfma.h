@@ -1,8 +1,10 @@
 // Gram among the active samples of a train block on the matrix cores (FP32 inputs and
-// accumulation). One wave computes a 32 x 32 block (rows i of block bi as the B operand, held
-// in registers; rows j of block bj <= bi as the A operand, loaded from the stream buffer) of the
-// two cross terms p = a_i.a_j and s = a_i.b_j with v_mfma_f32_32x32x2f32, and writes the lower
-// triangle's kappa values; a workgroup takes four blocks.
+// accumulation), one block of the lower triangle per wave, four per workgroup.
+//
+// For two entering samples per step (gramBlockMfma): 32 x 32 blocks (rows i of block bi as the B
+// operand, held in registers; rows j of block bj <= bi as the A operand, loaded from the stream buffer) of
+// the two cross terms p = a_i.a_j and s = a_i.b_j with v_mfma_f32_32x32x2f32, written row by row. For the
+// window sequencer (gramWinMfma): 16 x 16 blocks with v_mfma_f32_16x16x4f32, written in its layout.
 #pragma once
 
 #include "apsm_detect_mfma.h"

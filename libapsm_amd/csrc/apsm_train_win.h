@@ -25,7 +25,7 @@
 // Bound: the chain LDS write -> barrier -> LDS read -> product -> lane swaps -> projection (about 850
 // cycles at the small windows), and vector-ALU issue of the product where several product waves share a
 // SIMD (windowSize 160: 160 multiply-adds x 3 waves x 2.2 to 3.1 cycles, of 2500 cycles a step).
-// Measured, microseconds per step at windowSize 20 / 40 / 80 / 112 / 160: 0.37 / 0.41 / 0.51 / 0.64 / 1.06;
+// Measured, microseconds per step at windowSize 20 / 40 / 80 / 112 / 160: 0.38 / 0.42 / 0.52 / 0.64 / 1.06;
 // with two barriers per step and the projection in waves of its own (as apsm_train_seq2, which still
 // runs sampleStep 4) 1.30 / 1.40 / 1.44 / 1.6 / 1.83.
 #pragma once
