@@ -30,7 +30,7 @@
 //   32 antennas, 3690 centres, 49999 samples           678 -> 279 us
 //   64 antennas, 12 users, 16384 centres, 400k samples, bf16  16.1 -> 13.0 ms
 // or per block of 32 x 32 and SIMD, in cycles as if at 2.4 GHz: 1460 (8 antennas), 2070 (16), 3340 (32), 6880 (64),
-// measured with the blocks in plain order; taken by parts, 8 and 16 antennas cost 1 to 4 % more (ORDER).
+// measured with one sum per user; kept by parts (ORDER) within 4 % of that.
 // Measured and not kept: two column blocks per wave sharing the coefficient reads (10 % faster at 4 users,
 // slower elsewhere, 64 antennas spilled); 8 waves per workgroup (within 2 %); staging loads without
 // the bounds branches (20 % slower); all products before all exponentials (as fast up to 16
@@ -107,9 +107,9 @@ __device__ __forceinline__ void unrollFor( F f )
 // WAVES: waves per workgroup; ETILE: dictionary entries per LDS tile (0: mfmaTileOf). PARTS > 1: the
 // entries of a tile (32 PARTS) are shared out over PARTS waves of the same samples, wave w taking block
 // w % PARTS, and finish is called for the first of them with the parts added in order. ORDER > 1: a wave
-// takes all entries in the order 0, ORDER, 2 ORDER, ..., 1, ORDER + 1, ... of the 32-entry blocks and adds
-// each of the ORDER runs up by itself, which gives the bits of PARTS = ORDER. From 6 users on the sums of
-// the finished runs wait in LDS, for the registers' sake.
+// takes all entries and adds the blocks b % ORDER up by themselves, which gives the bits of PARTS = ORDER:
+// for few users side by side, otherwise in the order 0, ORDER, 2 ORDER, ..., 1, ORDER + 1, ... of the blocks,
+// one run after another (from 6 users on the finished runs' sums wait in LDS, for the registers' sake).
 template <int NMAX, int UMAX, int PREC, int WAVES, int ETILE, bool MASK, int PARTS, int ORDER, class LOAD, class FIRST, class FINISH>
 __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const float* __restrict__ Zn, const float* __restrict__ C,
                                               int64_t ldC, int64_t G, int U, float g2, int N, LOAD load, FIRST first, FINISH finish )
@@ -131,7 +131,13 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     __shared__ __attribute__( ( aligned( 16 ) ) ) uint16_t sZ[ 2 ][ NS ][ kTile * RowH ];
     __shared__ __attribute__( ( aligned( 16 ) ) ) float sZn[ 3 ][ kTile ];
     __shared__ __attribute__( ( aligned( 16 ) ) ) float2 sC[ 3 ][ kTile * UMAX ]; // [entry][user]
-    constexpr bool SUMLDS = ORDER > 1 && UMAX > 4;
+    // Few users: all ORDER sums in registers and the blocks in plain order, block b in sum b % ORDER; else one run after
+    // another. By runs a tile's rows are not consecutive and every block may end one: up to 4 % (512 detectors
+    // as a batch, one user each: detect 47.6 ms by runs, 42.4 side by side). At 32 antennas and two users the
+    // sums spill, and from 6 users on they do not fit; at 64 antennas runs are as fast.
+    constexpr bool KEEP = ORDER > 1 && NMAX <= 32 && ( UMAX == 1 || ( UMAX <= 4 && NMAX <= 16 ) ), RUNS = ORDER > 1 && !KEEP;
+    constexpr int SUMS = KEEP ? ORDER : 1;
+    constexpr bool SUMLDS = RUNS && UMAX > 4;
     __shared__ float sSum[ SUMLDS ? UMAX * 64 * WAVES : 1 ]; // [user][lane]: sums of the finished runs
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -231,21 +237,25 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     float k2 = 2.f * g2, k2n = -2.f * g2;
     asm( "" : "+v"( k2 ), "+v"( k2n ) );
 
-    float fa[ UMAX ], fb[ UMAX ];
+    float fa[ SUMS ][ UMAX ], fb[ SUMS ][ UMAX ];
     auto addHalves = [ & ]() {
 #pragma unroll
-        for ( int u = 0; u < UMAX; u++ )
-        {
-            fa[ u ] += __shfl_xor( fa[ u ], 32 );
-            fb[ u ] += __shfl_xor( fb[ u ], 32 );
-        }
+        for ( int o = 0; o < SUMS; o++ )
+#pragma unroll
+            for ( int u = 0; u < UMAX; u++ )
+            {
+                fa[ o ][ u ] += __shfl_xor( fa[ o ][ u ], 32 );
+                fb[ o ][ u ] += __shfl_xor( fb[ o ][ u ], 32 );
+            }
     };
     float sum[ SUMLDS ? 1 : UMAX ]; // sums of the finished runs, fa's in lane half 0 and fb's in 1
     float* const sums = sSum + ( SUMLDS ? tid : 0 );
 #pragma unroll
     for ( int u = 0; u < UMAX; u++ )
     {
-        fa[ u ] = fb[ u ] = 0.f;
+#pragma unroll
+        for ( int o = 0; o < SUMS; o++ )
+            fa[ o ][ u ] = fb[ o ][ u ] = 0.f;
         if ( SUMLDS )
             sums[ u * 64 * WAVES ] = 0.f;
         else
@@ -276,8 +286,8 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     float2 creg[ kCLoads ];
     const bool whole = N == NMAX && K == K16 && ( reinterpret_cast<uintptr_t>( Z ) & 15 ) == 0;
     auto loadRows = [ & ]() { // a tile of consecutive rows
-        const int64_t j0 = (int64_t)( ORDER > 1 ? nextBlock() : bLoad ) * 32;
-        if ( ORDER == 1 )
+        const int64_t j0 = (int64_t)( RUNS ? nextBlock() : bLoad ) * 32;
+        if ( !RUNS )
             bLoad += kTileBlocks;
         const int nt = ( G - j0 ) < kTile ? (int)( G - j0 ) : kTile;
         if ( whole )
@@ -368,7 +378,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         }
     };
     auto loadTile = [ & ]() {
-        if constexpr ( ORDER > 1 && ( kTileBlocks > 1 || UMAX > 8 || ( NMAX >= 64 && UMAX > 2 ) ) ) // (scalar addresses: fewer spills)
+        if constexpr ( RUNS && ( kTileBlocks > 1 || UMAX > 8 || ( NMAX >= 64 && UMAX > 2 ) ) ) // (scalar addresses: fewer spills)
             loadBlocks();
         else
             loadRows();
@@ -443,10 +453,10 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
     // Distances, exponentials and every user's contraction of the block in accumulators S (entries cb of
     // coefficient slot `slot`), between them the products of the next block (entries cbn of buffer
     // bufn) into the other set. The fences keep the two streams interleaved entry by entry.
-    constexpr int PF = UMAX <= 2 ? 4 : 1; // entries whose coefficients are read ahead together
+    constexpr int PF = UMAX > 2 ? 1 : UMAX == 2 && NMAX >= 32 ? 2 : 4; // entries whose coefficients are read ahead together
     int run = 0, runLeft = ( nBlocks + ORDER - 1 ) / ORDER; // run of the next phase, blocks left in it
-    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, int rel = 0 ) {
-        constexpr int d = dC;
+    auto phase = [ & ]( int slot, int cb, int bufn, int cbn, auto dC, auto oC, int rel = 0 ) {
+        constexpr int d = dC, ord = oC; // accumulators, sum
         float2 co[ 2 ][ PF * UMAX ];
         float4 zq[ 2 ];
         auto entryOf = [ & ]( int i ) { return cb + 8 * ( i / 4 ) + 4 * h + i % 4; }; // the lane's entry i within the tile
@@ -483,21 +493,21 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
             for ( int u = 0; u < UMAX; u++ )
             {
                 const float2 c = co[ i / PF & 1 ][ i % PF * UMAX + u ];
-                fa[ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ u ] ) );
-                fb[ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ u ] ) );
-                asm volatile( "" : "+v"( fa[ u ] ), "+v"( fb[ u ] )::"memory" );
+                fa[ ord ][ u ] = fmaf( c.x, E0, fmaf( c.y, E1, fa[ ord ][ u ] ) );
+                fb[ ord ][ u ] = fmaf( c.x, E2, fmaf( c.y, E0, fb[ ord ][ u ] ) );
+                asm volatile( "" : "+v"( fa[ ord ][ u ] ), "+v"( fb[ ord ][ u ] )::"memory" );
             }
             __builtin_amdgcn_sched_barrier( 0 );
         } );
-        if constexpr ( ORDER > 1 )
+        if constexpr ( RUNS )
             if ( --runLeft == 0 ) // the run ends with this block
             {
 #pragma unroll
                 for ( int u = 0; u < UMAX; u++ )
                 {
-                    const auto s = __builtin_amdgcn_permlane32_swap( __float_as_uint( fa[ u ] ), __float_as_uint( fb[ u ] ), false, false );
+                    const auto s = __builtin_amdgcn_permlane32_swap( __float_as_uint( fa[ 0 ][ u ] ), __float_as_uint( fb[ 0 ][ u ] ), false, false );
                     ( SUMLDS ? sums[ u * 64 * WAVES ] : sum[ SUMLDS ? 0 : u ] ) += __uint_as_float( s[ 0 ] ) + __uint_as_float( s[ 1 ] );
-                    fa[ u ] = fb[ u ] = 0.f;
+                    fa[ 0 ][ u ] = fb[ 0 ][ u ] = 0.f;
                 }
                 run++;
                 runLeft = ( nBlocks - run + ORDER - 1 ) / ORDER;
@@ -533,6 +543,8 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         __syncthreads();
     };
     // (the products past the last block read what the buffers hold, and are not used)
+    static_assert( SUMS == 1 || PIPE, "sums kept apart in the pipelined loops" );
+    static_assert( SUMS == 1 || kBlocks == 1 || SUMS % kBlocks == 0, "whole turns of the sums" );
     if constexpr ( !PIPE )
     {
 #pragma unroll 1
@@ -544,32 +556,40 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
                 if ( (int64_t)tt * kTile + cb >= G )
                     break;
                 products( tt & 1, cb );
-                phase( tt % 3, cb, 0, 0, D0 {}, MASK ? first( (int64_t)tt * kTile ) : 0 );
+                phase( tt % 3, cb, 0, 0, D0 {}, D0 {}, MASK ? first( (int64_t)tt * kTile ) : 0 );
             }
             advance( tt );
         }
     }
     else if constexpr ( kBlocks == 1 )
     {
+        constexpr int STEP = SUMS > 2 ? SUMS : 2;
 #pragma unroll 1
-        for ( int t0 = 0; t0 < nTiles; t0 += 2 )
-            unrollFor<2>( [ & ]( auto iC ) {
+        for ( int t0 = 0; t0 < nTiles; t0 += STEP )
+            unrollFor<STEP>( [ & ]( auto iC ) {
                 const int tt = t0 + iC;
                 if ( tt >= nTiles )
                     return;
                 advance( tt );
-                phase( tt % 3, cw, ( tt + 1 ) & 1, cw, std::integral_constant<int, iC> {} );
+                phase( tt % 3, cw, ( tt + 1 ) & 1, cw, std::integral_constant<int, iC & 1> {}, std::integral_constant<int, iC % SUMS> {} );
             } );
     }
     else
     {
+        constexpr int STEP = SUMS > kBlocks ? SUMS / kBlocks : 1;
 #pragma unroll 1
-        for ( int tt = 0; tt < nTiles; tt++ )
-            unrollFor<kBlocks>( [ & ]( auto bC ) {
-                constexpr int b = bC, last = b == kBlocks - 1;
-                if constexpr ( last )
-                    advance( tt );
-                phase( tt % 3, 32 * b, ( tt + last ) & 1, last ? 0 : 32 * b + 32, std::integral_constant<int, b & 1> {} );
+        for ( int t0 = 0; t0 < nTiles; t0 += STEP )
+            unrollFor<STEP>( [ & ]( auto iC ) {
+                const int tt = t0 + iC;
+                if ( tt >= nTiles )
+                    return;
+                unrollFor<kBlocks>( [ & ]( auto bC ) {
+                    constexpr int b = bC, last = b == kBlocks - 1;
+                    if constexpr ( last )
+                        advance( tt );
+                    phase( tt % 3, 32 * b, ( tt + last ) & 1, last ? 0 : 32 * b + 32, std::integral_constant<int, b & 1> {},
+                           std::integral_constant<int, ( iC * kBlocks + b ) % SUMS> {} );
+                } );
             } );
     }
     __syncthreads(); // a following tile stores over what other waves may still read
@@ -585,7 +605,7 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
         if ( part > 0 )
 #pragma unroll
             for ( int u = 0; u < UMAX; u++ )
-                red[ ( ( part - 1 ) * UMAX + u ) * 64 ] = make_float2( fa[ u ], fb[ u ] );
+                red[ ( ( part - 1 ) * UMAX + u ) * 64 ] = make_float2( fa[ 0 ][ u ], fb[ 0 ][ u ] );
         __syncthreads();
         if ( part == 0 )
         {
@@ -595,27 +615,37 @@ __device__ __forceinline__ void gaussianMfma( const float* __restrict__ Z, const
                 for ( int u = 0; u < UMAX; u++ )
                 {
                     const float2 v = red[ ( k * UMAX + u ) * 64 ];
-                    fa[ u ] += v.x;
-                    fb[ u ] += v.y;
+                    fa[ 0 ][ u ] += v.x;
+                    fb[ 0 ][ u ] += v.y;
                 }
-            finish( fa, fb );
+            finish( fa[ 0 ], fb[ 0 ] );
         }
         __syncthreads(); // a following tile stores over what was read
     }
     else
     {
-        if constexpr ( ORDER > 1 )
+        if constexpr ( RUNS )
         {
 #pragma unroll
             for ( int u = 0; u < UMAX; u++ )
             {
-                fa[ u ] = SUMLDS ? sums[ u * 64 * WAVES ] : sum[ SUMLDS ? 0 : u ];
-                fb[ u ] = __shfl_xor( fa[ u ], 32 );
+                fa[ 0 ][ u ] = SUMLDS ? sums[ u * 64 * WAVES ] : sum[ SUMLDS ? 0 : u ];
+                fb[ 0 ][ u ] = __shfl_xor( fa[ 0 ][ u ], 32 );
             }
         }
         else
+        {
             addHalves();
-        finish( fa, fb );
+#pragma unroll
+            for ( int o = 1; o < SUMS; o++ )
+#pragma unroll
+                for ( int u = 0; u < UMAX; u++ )
+                {
+                    fa[ 0 ][ u ] += fa[ o ][ u ];
+                    fb[ 0 ][ u ] += fb[ o ][ u ];
+                }
+        }
+        finish( fa[ 0 ], fb[ 0 ] );
     }
 }
 
